@@ -284,10 +284,13 @@ template <>
 struct LdsAcc<float> {
   using T = unsigned long long;
   __device__ static __forceinline__ T enc(float v) {
-    double d = double(v) * 268435456.0;  // 2^28
-    d = fmin(fmax(d, -1125899906842624.0), 1125899906842624.0);  // +-2^50
-    d = d + 6755399441055744.0;                                   // 1.5 * 2^52
+    v = __builtin_amdgcn_fmed3f(v, -4194304.0f, 4194304.0f);  // +-2^22
+    const double d = __builtin_fma(double(v), 268435456.0, 6755399441055744.0);  // 2^28, 1.5 * 2^52
     return (T)(__double_as_longlong(d) - 0x4338000000000000LL);
+  }
+  // *p -= v
+  __device__ static __forceinline__ void sub(T* p, T v) {
+    __hip_atomic_fetch_sub(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   }
   __device__ static __forceinline__ float dec(T x) {
     return float(double((long long)x) * (1.0 / 268435456.0));
@@ -298,6 +301,7 @@ template <>
 struct LdsAcc<double> {
   using T = double;
   __device__ static __forceinline__ T enc(double v) { return v; }
+  __device__ static __forceinline__ void sub(T* p, T v) { atomicAdd(p, -v); }
   __device__ static __forceinline__ double dec(T x) { return x; }
 };
 

@@ -177,9 +177,9 @@ __device__ __forceinline__ void eval_elec(ElecLDS<Real, MODE>& L, int consume,
           atomicAdd(&L.grad[0][s1], ex);
           atomicAdd(&L.grad[1][s1], ey);
           atomicAdd(&L.grad[2][s1], ez);
-          atomicAdd(&L.grad[0][s2], typename Acc::T(0) - ex);
-          atomicAdd(&L.grad[1][s2], typename Acc::T(0) - ey);
-          atomicAdd(&L.grad[2][s2], typename Acc::T(0) - ez);
+          Acc::sub(&L.grad[0][s2], ex);
+          Acc::sub(&L.grad[1][s2], ey);
+          Acc::sub(&L.grad[2][s2], ez);
         }
       }
     }

@@ -233,9 +233,9 @@ __device__ __forceinline__ void elec_chunk_eval(ElecRotLDS2<Real, BWD>& L, int c
         atomicAdd(&L.acc1[0][j], ex);
         atomicAdd(&L.acc1[1][j], ey);
         atomicAdd(&L.acc1[2][j], ez);
-        atomicAdd(&L.acc2[0][l2], T(0) - ex);
-        atomicAdd(&L.acc2[1][l2], T(0) - ey);
-        atomicAdd(&L.acc2[2][l2], T(0) - ez);
+        Acc::sub(&L.acc2[0][l2], ex);
+        Acc::sub(&L.acc2[1][l2], ey);
+        Acc::sub(&L.acc2[2][l2], ez);
       }
     }
   }

@@ -2,14 +2,17 @@
 //
 // Same functions as the reference (tmol/score/ljlk/potentials/lj.hh:21-177,
 // lk_isotropic.hh:22-360, common.hh:13-44, tmol/score/common/
-// cubic_hermite_polynomial.hh), arranged so that each region of a piecewise
-// potential evaluates the underlying closed form once at a clamped abscissa
-// instead of branching per region:
+// cubic_hermite_polynomial.hh), arranged so that the regions of a piecewise
+// potential share one evaluation of the underlying closed form at a clamped
+// abscissa x, and the pieces that extend it (linear, Hermite to zero) are one
+// expression in d - x:
 //
 //   LJ:  x = clamp(d, d_lin, cpoly_dmin); one 12-6 evaluation V(x), V'(x);
-//        linear extension below d_lin, Hermite-to-zero above cpoly_dmin.
+//        no branches.
 //   LK:  one f_desolv evaluation at clamp(d, close_dmax, far_dmin) per
-//        direction, a second one at d_min only where d < close_dmax.
+//        direction, a second one at d_min only where d < close_dmax; both
+//        directions have the same knots, so their values are summed before
+//        the (linear) interpolation.
 //
 // Float builds use the hardware rcp / sqrt / exp (1-2 ulp); the double
 // instantiation (the oracle run) uses correctly rounded division, sqrt and
@@ -101,7 +104,8 @@ __device__ __forceinline__ Real cp_weight(int sep) {
 template <typename Real>
 __device__ __forceinline__ Real lj_sigma(int fi, int fj, Real ri, Real rj,
                                          const GlobalParams<Real>& g) {
-  const int both = ((fi >> 3) & 1 ? fj : 0) | ((fj >> 3) & 1 ? fi : 0);
+  // bit 3 of each sign-extended to a mask
+  const int both = (__builtin_amdgcn_sbfe(fi, 3, 1) & fj) | (__builtin_amdgcn_sbfe(fj, 3, 1) & fi);
   const bool da = both & F_DONOR;
   const bool ha = both & F_POLARH;
   const bool oh = (fi | fj) & F_OH_DONOR;
@@ -113,46 +117,38 @@ __device__ __forceinline__ Real lj_sigma(int fi, int fj, Real ri, Real rj,
 
 // LJ for one pair: returns weighted (atr, rep) and d(atr+rep)/dd.
 // Only one of atr/rep carries the derivative: rep inside sigma, atr outside.
+// With u = d - x: u < 0 on the linear piece (V + V' u), 0 on the 12-6 piece,
+// and on the Hermite piece to (0, 0) at max_dis, t = u / w, the value is
+// (1 - t)^2 (V + V' u + 2 t V); t = 0 elsewhere, so one expression covers all
+// three.
 template <typename Real, bool DERIV>
 __device__ __forceinline__ void lj_pair(Real dist, Real sigma, Real eps,
                                         Real weight,
                                         const GlobalParams<Real>& g,
                                         Real& atr, Real& rep, Real& dlj) {
-  Real d_lin = sigma * g.dlin_factor;
+  const Real d_lin = sigma * g.dlin_factor;
   Real cpoly_dmin = sigma > g.spline_start ? sigma : g.spline_start;
   cpoly_dmin = cpoly_dmin > g.cpoly_cap ? g.cpoly_cap : cpoly_dmin;
   // evaluation point of the 12-6 form
-  Real x = dist < d_lin ? d_lin : (dist < cpoly_dmin ? dist : cpoly_dmin);
-  Real inv_x = fast_rcp(x);
-  Real sd = sigma * inv_x;
-  Real sd2 = sd * sd;
-  Real sd6 = sd2 * sd2 * sd2;
-  Real sd12 = sd6 * sd6;
-  Real V = eps * (sd12 - Real(2) * sd6);
-  Real dV = eps * Real(12) * (sd6 - sd12) * inv_x;
-  Real lj, dl;
-  if (dist < d_lin) {
-    lj = V + dV * (dist - d_lin);
-    dl = dV;
-  } else if (dist < cpoly_dmin) {
-    lj = V;
-    dl = dV;
-  } else {
-    // Hermite to (0, 0) at max_dis (interpolate_to_zero_V_dV)
-    Real w = g.max_dis - cpoly_dmin;
-    Real inv_w = fast_rcp(w);
-    Real t = (dist - cpoly_dmin) * inv_w;
-    Real dp0 = dV * w;
-    lj = V + t * (dp0 + t * (Real(-2) * dp0 - Real(3) * V + t * (dp0 + Real(2) * V)));
-    dl = (dp0 + t * (Real(-4) * dp0 - Real(6) * V + t * (Real(3) * dp0 + Real(6) * V))) * inv_w;
-    bool out = dist >= g.max_dis;
-    lj = out ? Real(0) : lj;
-    dl = out ? Real(0) : dl;
-  }
-  bool inside = dist < sigma;
+  const Real x = dist < d_lin ? d_lin : (dist < cpoly_dmin ? dist : cpoly_dmin);
+  const Real inv_x = fast_rcp(x);
+  const Real sd = sigma * inv_x;
+  const Real sd2 = sd * sd;
+  const Real sd6 = sd2 * sd2 * sd2;
+  const Real es = eps * sd6;
+  const Real V = es * (sd6 - Real(2));
+  const Real dV = es * Real(12) * (Real(1) - sd6) * inv_x;
+  const Real u = dist - x;
+  const Real iw = u > Real(0) ? fast_rcp(g.max_dis - cpoly_dmin) : Real(0);
+  const Real t = u * iw;
+  Real q = Real(1) - t;
+  q = q > Real(0) ? q : Real(0);  // zero at and beyond max_dis
+  const Real b = V + dV * u + Real(2) * t * V;
+  const Real lj = q * q * b;
+  const bool inside = dist < sigma;
   atr = weight * (inside ? -eps : lj);
   rep = weight * (inside ? lj + eps : Real(0));
-  dlj = DERIV ? weight * dl : Real(0);
+  dlj = DERIV ? weight * (q * (q * (dV + Real(2) * iw * V) - Real(2) * iw * b)) : Real(0);
 }
 
 // LK knots on the 1/20 A^2 etable grid (lk_isotropic.hh:116-125)
@@ -171,62 +167,63 @@ __device__ __forceinline__ void lk_knots(Real sigma, bool is_cc, Real& d_min,
   close_dmax = fast_sqrt(hi * Real(0.05));
 }
 
-// f_desolv and its derivative with c = -vol_j * dg_i / (2 pi^1.5 lambda_i)
-// precomputed per atom as -vol_j * K_i, K_i = dg_i / (2 pi^1.5 lambda_i)
+// one direction of LK: c = -vol_j * K_i with K_i = dg_i / (2 pi^1.5 lambda_i),
+// r_i and 1 / lambda_i^2
 template <typename Real>
-__device__ __forceinline__ void fdesolv(Real x, Real c, Real r_i,
-                                        Real inv_lam2_i, Real& f, Real& df) {
-  Real inv_x = fast_rcp(x);
-  Real dr = x - r_i;
-  Real e = fast_exp(-dr * dr * inv_lam2_i);
-  f = c * inv_x * inv_x * e;
-  df = f * (Real(-2) * inv_x - Real(2) * dr * inv_lam2_i);
+struct LkSide {
+  Real c, r, inv_lam2;
+};
+
+// sum over the directions of f_desolv and its derivative at x
+template <typename Real, int SIDES>
+__device__ __forceinline__ void fdesolv(Real x, const LkSide<Real> (&side)[SIDES], Real& f,
+                                        Real& df) {
+  const Real inv_x = fast_rcp(x);
+  const Real inv_x2 = inv_x * inv_x;
+  f = df = Real(0);
+#pragma unroll
+  for (int k = 0; k < SIDES; ++k) {
+    const Real dr = x - side[k].r;
+    const Real sl = dr * side[k].inv_lam2;
+    const Real e = side[k].c * inv_x2 * fast_exp(-dr * sl);
+    f += e;
+    df += e * (Real(-2) * (inv_x + sl));
+  }
 }
 
-// one direction of isotropic LK (lk_isotropic.hh:167-235), unweighted
-template <typename Real, bool DERIV>
-__device__ __forceinline__ void lk_dir(Real dist, Real d_min, Real cdmin,
-                                       Real cdmax, Real c, Real r_i,
-                                       Real inv_lam2_i,
-                                       const GlobalParams<Real>& g, Real& V,
-                                       Real& dV) {
-  Real x = dist < cdmax ? cdmax : (dist < g.spline_start ? dist : g.spline_start);
+// isotropic LK (lk_isotropic.hh:167-235), unweighted, summed over the given
+// directions (their knots are the same): f at clamp(d, cdmax, far_dmin), the
+// Hermite piece to zero as in lj_pair, and below cdmax the Hermite piece from
+// (cdmin, f(d_min), slope 0), constant below cdmin.
+template <typename Real, bool DERIV, int SIDES>
+__device__ __forceinline__ void lk_sides(Real dist, Real d_min, Real cdmin, Real cdmax,
+                                         const LkSide<Real> (&side)[SIDES],
+                                         const GlobalParams<Real>& g, Real& V, Real& dV) {
+  const bool close = dist < cdmax;
+  const Real x = close ? cdmax : (dist < g.spline_start ? dist : g.spline_start);
   Real f, df;
-  fdesolv(x, c, r_i, inv_lam2_i, f, df);
-  if (dist >= cdmax) {
-    if (dist < g.spline_start) {
-      V = f;
-      dV = df;
-    } else {
-      // Hermite to zero over [max_dis - 1.5, max_dis]
-      Real w = g.max_dis - g.spline_start;
-      Real inv_w = fast_rcp(w);
-      Real t = (dist - g.spline_start) * inv_w;
-      Real dp0 = df * w;
-      V = f + t * (dp0 + t * (Real(-2) * dp0 - Real(3) * f + t * (dp0 + Real(2) * f)));
-      dV = (dp0 + t * (Real(-4) * dp0 - Real(6) * f + t * (Real(3) * dp0 + Real(6) * f))) * inv_w;
-      bool out = dist >= g.max_dis;
-      V = out ? Real(0) : V;
-      dV = out ? Real(0) : dV;
-    }
-  } else {
+  fdesolv<Real, SIDES>(x, side, f, df);
+  const Real u = dist - x;
+  const Real iw = u > Real(0) ? fast_rcp(g.max_dis - g.spline_start) : Real(0);
+  const Real t = u * iw;
+  Real q = Real(1) - t;
+  q = q > Real(0) ? q : Real(0);
+  const Real b = f + df * u + Real(2) * t * f;
+  V = q * q * b;
+  dV = DERIV ? q * (q * (df + Real(2) * iw * f) - Real(2) * iw * b) : Real(0);
+  if (close) {
     Real f0, df0;
-    fdesolv(d_min, c, r_i, inv_lam2_i, f0, df0);
-    if (dist < cdmin) {
-      V = f0;
-      dV = Real(0);
-    } else {
-      // Hermite from (cdmin, f(d_min), 0) to (cdmax, f, df)
-      Real w = cdmax - cdmin;
-      Real inv_w = fast_rcp(w);
-      Real t = (dist - cdmin) * inv_w;
-      Real dp1 = df * w;
-      Real p0 = f0, p1 = f;
-      V = p0 + t * (t * (-dp1 - Real(3) * p0 + Real(3) * p1 + t * (dp1 + Real(2) * p0 - Real(2) * p1)));
-      dV = (t * (Real(-2) * dp1 - Real(6) * p0 + Real(6) * p1 + t * (Real(3) * dp1 + Real(6) * p0 - Real(6) * p1))) * inv_w;
-    }
+    fdesolv<Real, SIDES>(d_min, side, f0, df0);
+    const Real w = cdmax - cdmin;
+    const Real inv_w = fast_rcp(w);
+    Real tc = (dist - cdmin) * inv_w;
+    tc = tc > Real(0) ? tc : Real(0);
+    const Real dp1 = df * w;
+    const Real c2 = Real(3) * (f - f0) - dp1;
+    const Real c3 = dp1 - Real(2) * (f - f0);
+    V = f0 + tc * tc * (c2 + tc * c3);
+    dV = DERIV ? tc * (Real(2) * c2 + Real(3) * tc * c3) * inv_w : Real(0);
   }
-  if (!DERIV) dV = Real(0);
 }
 
 // ---- elec (tmol/score/elec/potentials/potentials.hh)

@@ -417,14 +417,15 @@ __device__ __forceinline__ Real rot_pair(const RotLDS<Real>& L, int j, const Ato
     const bool cc = (f1 & F_CARBON_LK) && (R2.flags & F_CARBON_LK);
     Real d_min, cdmin, cdmax;
     lk_knots(sigma, cc, d_min, cdmin, cdmax);
-    Real va, dva, vb, dvb;
-    lk_dir<Real, BWD>(dist, d_min, cdmin, cdmax, -R2.vol * q1.y, p1.w, q1.z, gp, va, dva);
-    lk_dir<Real, BWD>(dist, d_min, cdmin, cdmax, -q1.w * R2.r0.z, R2.r0.x, R2.r0.w, gp, vb, dvb);
+    const LkSide<Real> side[2] = {{-R2.vol * q1.y, p1.w, q1.z},
+                                  {-q1.w * R2.r0.z, R2.r0.x, R2.r0.w}};
+    Real v, dv;
+    lk_sides<Real, BWD>(dist, d_min, cdmin, cdmax, side, gp, v, dv);
     if (heavy) {
       if (!BWD)
-        el += wcp * (va + vb);
+        el += wcp * v;
       else if (dist > Real(0))
-        gs += w2 * (wcp * (dva + dvb)) * inv_d;
+        gs += w2 * (wcp * dv) * inv_d;
     }
   }
   return gs;
@@ -810,10 +811,10 @@ __device__ __forceinline__ void rot_fifo_lk(RotLDS2<Real>& L, int consume,
     const bool cc = (f1 & F_CARBON_LK) && (f2 & F_CARBON_LK);
     Real d_min, cdmin, cdmax;
     lk_knots(sigma, cc, d_min, cdmin, cdmax);
-    Real va, dva, vb, dvb;
-    lk_dir<Real, false>(dist, d_min, cdmin, cdmax, -q2.w * q1.y, p1.w, q1.z, gp, va, dva);
-    lk_dir<Real, false>(dist, d_min, cdmin, cdmax, -q1.w * q2.y, p2.w, q2.z, gp, vb, dvb);
-    atomicAdd(&L.lacc[2][l2], Acc::enc(wcp * (va + vb)));
+    const LkSide<Real> side[2] = {{-q2.w * q1.y, p1.w, q1.z}, {-q1.w * q2.y, p2.w, q2.z}};
+    Real v, dv;
+    lk_sides<Real, false>(dist, d_min, cdmin, cdmax, side, gp, v, dv);
+    atomicAdd(&L.lacc[2][l2], Acc::enc(wcp * v));
   }
 }
 

@@ -31,9 +31,9 @@ __device__ __forceinline__ void grad_pair(GenLDS<Real>& L, int term, int i1, int
   atomicAdd(&L.grad[term][0][i1], ex);
   atomicAdd(&L.grad[term][1][i1], ey);
   atomicAdd(&L.grad[term][2][i1], ez);
-  atomicAdd(&L.grad[term][0][i2], T(0) - ex);
-  atomicAdd(&L.grad[term][1][i2], T(0) - ey);
-  atomicAdd(&L.grad[term][2][i2], T(0) - ez);
+  Acc::sub(&L.grad[term][0][i2], ex);
+  Acc::sub(&L.grad[term][1][i2], ey);
+  Acc::sub(&L.grad[term][2][i2], ez);
 }
 
 template <typename Real, int MODE>
@@ -263,15 +263,14 @@ __global__ __launch_bounds__(256) void score_general_kernel(ScoreArgs<Real> A) {
                   bool cc = (f1 & F_CARBON_LK) && (f2 & F_CARBON_LK);
                   Real d_min, cdmin, cdmax;
                   lk_knots(sigma, cc, d_min, cdmin, cdmax);
-                  Real v1, dv1, v2, dv2;
-                  lk_dir<Real, DERIV>(dist, d_min, cdmin, cdmax, -L.vol[i2] * L.K[i1], L.rad[i1],
-                                      L.il2[i1], gp, v1, dv1);
-                  lk_dir<Real, DERIV>(dist, d_min, cdmin, cdmax, -L.vol[i1] * L.K[i2], L.rad[i2],
-                                      L.il2[i2], gp, v2, dv2);
+                  const LkSide<Real> side[2] = {{-L.vol[i2] * L.K[i1], L.rad[i1], L.il2[i1]},
+                                                {-L.vol[i1] * L.K[i2], L.rad[i2], L.il2[i2]}};
+                  Real v, dv;
+                  lk_sides<Real, DERIV>(dist, d_min, cdmin, cdmax, side, gp, v, dv);
                   Real wcp = cp_weight<Real>(sep);
-                  e_lk.add(wcp * (v1 + v2));
+                  e_lk.add(wcp * v);
                   if (DERIV && dist > Real(0)) {
-                    Real dlk = wcp * (dv1 + dv2);
+                    Real dlk = wcp * dv;
                     if (dlk != Real(0)) {
                       Real gs = dlk * fast_rcp(dist);
                       if (WGRAD) gs *= w[2];

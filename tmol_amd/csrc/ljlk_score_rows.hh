@@ -181,9 +181,9 @@ __device__ __forceinline__ void grad_scatter(LDS& L, int term, int s1, int s2,
   atomicAdd(&L.grad[c][term][0][s1], ex);
   atomicAdd(&L.grad[c][term][1][s1], ey);
   atomicAdd(&L.grad[c][term][2][s1], ez);
-  atomicAdd(&L.grad[c][term][0][s2], T(0) - ex);
-  atomicAdd(&L.grad[c][term][1][s2], T(0) - ey);
-  atomicAdd(&L.grad[c][term][2][s2], T(0) - ez);
+  Acc::sub(&L.grad[c][term][0][s2], ex);
+  Acc::sub(&L.grad[c][term][1][s2], ey);
+  Acc::sub(&L.grad[c][term][2][s2], ez);
 }
 
 // Evaluate LJ entries [0, consume) of the FIFO, one per lane.
@@ -255,10 +255,10 @@ __device__ __forceinline__ void eval_lk(LDS& L, int consume,
       const bool cc = (f1 & F_CARBON_LK) && (f2 & F_CARBON_LK);
       Real d_min, cdmin, cdmax;
       lk_knots(sigma, cc, d_min, cdmin, cdmax);
-      Real va, dva, vb, dvb;
-      lk_dir<Real, C::DERIV>(dist, d_min, cdmin, cdmax, -q2.w * q1.y, p1.w, q1.z, gp, va, dva);
-      lk_dir<Real, C::DERIV>(dist, d_min, cdmin, cdmax, -q1.w * q2.y, p2.w, q2.z, gp, vb, dvb);
-      const Real lk = wcp * (va + vb);
+      const LkSide<Real> side[2] = {{-q2.w * q1.y, p1.w, q1.z}, {-q1.w * q2.y, p2.w, q2.z}};
+      Real v, dv;
+      lk_sides<Real, C::DERIV>(dist, d_min, cdmin, cdmax, side, gp, v, dv);
+      const Real lk = wcp * v;
       if (!C::NOE) {
         if (C::BP)
           atomicAdd(&L.ebp[entry_owner(s2)][2], LdsAcc<Real>::enc(lk));
@@ -266,7 +266,7 @@ __device__ __forceinline__ void eval_lk(LDS& L, int consume,
           e_lk.add(lk);
       }
       if (C::DERIV && dist > Real(0)) {
-        const Real dlk = wcp * (dva + dvb);
+        const Real dlk = wcp * dv;
         if (dlk != Real(0)) {
           Real gs = dlk * inv_d;
           if (C::WGRAD) gs *= C::BP ? L.wt[entry_owner(s2)][2] : wrow[2];

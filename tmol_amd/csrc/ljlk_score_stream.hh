@@ -70,7 +70,6 @@ struct StreamLDS {
   Real wt[1][3];
   alignas(4 * sizeof(Real)) Real pos[SSLOTS][4];  // x, y, z, lj_radius
   alignas(4 * sizeof(Real)) Real prm[SSLOTS][4];  // sqrt(lj_wdepth), K, 1/lambda^2, lk_volume
-  alignas(4 * sizeof(Real)) Real tst[SCH][4];  // test chunk atoms: x, y, z
   uint32_t tq[SCH];      // test chunk atoms: connection bytes q | Q_HEAVY | Q_LIG
   uint8_t flg[SSLOTS];
   uint16_t lj[SLIST];
@@ -139,9 +138,9 @@ __device__ __forceinline__ void grad_scatter(StreamLDS<Real, MODE>& L, int term,
   atomicAdd(b1, ex);
   atomicAdd(b1 + TILE, ey);
   atomicAdd(b1 + 2 * TILE, ez);
-  atomicAdd(b2, T(0) - ex);
-  atomicAdd(b2 + k2, T(0) - ey);
-  atomicAdd(b2 + 2 * k2, T(0) - ez);
+  Acc::sub(b2, ex);
+  Acc::sub(b2 + k2, ey);
+  Acc::sub(b2 + 2 * k2, ez);
 }
 
 // flush the gradients of ring chunk r (n atoms, slots TILE + SCH r ...) to
@@ -319,7 +318,7 @@ __global__ __launch_bounds__(256, (stream_waves_per_simd<MODE, OCC>())) void sco
     auto test_chunk = [&]() {
       const int r = cur;
       const int n = fill;
-      const V tr = *(const V*)L.tst[u];
+      const V tr = *(const V*)L.pos[TILE + SCH * r + u];
       const uint32_t qb = L.tq[u];
       const bool heavy2 = (qb & Q_HEAVY) != 0;
       const bool lig2 = (qb & Q_LIG) != 0;
@@ -461,7 +460,6 @@ __global__ __launch_bounds__(256, (stream_waves_per_simd<MODE, OCC>())) void sco
             pq.x = R.r0.y; pq.y = R.r0.z; pq.z = R.r0.w; pq.w = R.vol;
             *(V*)L.pos[slot] = pp;
             *(V*)L.prm[slot] = pq;
-            *(V*)L.tst[pos] = pp;
             L.tq[pos] = qv;
             L.flg[slot] = (uint8_t)R.flags;
             L.atom[SCH * cur + pos] = o2 + a;

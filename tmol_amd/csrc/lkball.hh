@@ -443,7 +443,8 @@ __device__ __forceinline__ int lkb_eval(const LkbAtom<Real>& I, const LkbAtom<Re
   Real d_min, cdmin, cdmax;
   lk_knots(sigma, bool((I.flg & F_CARBON_LK) && (J.flg & F_CARBON_LK)), d_min, cdmin, cdmax);
   Real iso, diso;
-  lk_dir<Real, DERIV>(dist, d_min, cdmin, cdmax, -J.vol * I.K, I.r, I.il2, g, iso, diso);
+  const LkSide<Real> side[1] = {{-J.vol * I.K, I.r, I.il2}};
+  lk_sides<Real, DERIV>(dist, d_min, cdmin, cdmax, side, g, iso, diso);
   iso *= wcp;
   diso *= wcp;
   // lk_fraction (lk_ball.hh:42-124)
