@@ -288,6 +288,12 @@ struct LdsAcc<float> {
     const double d = __builtin_fma(double(v), 268435456.0, 6755399441055744.0);  // 2^28, 1.5 * 2^52
     return (T)(__double_as_longlong(d) - 0x4338000000000000LL);
   }
+  // enc() of a value already times SCALE (a power of two: the same result)
+  static constexpr float SCALE = 268435456.0f;
+  __device__ static __forceinline__ T enc_scaled(float v) {
+    v = __builtin_amdgcn_fmed3f(v, -1125899906842624.0f, 1125899906842624.0f);  // +-2^50
+    return (T)(__double_as_longlong(double(v) + 6755399441055744.0) - 0x4338000000000000LL);
+  }
   // *p -= v
   __device__ static __forceinline__ void sub(T* p, T v) {
     __hip_atomic_fetch_sub(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -301,6 +307,8 @@ template <>
 struct LdsAcc<double> {
   using T = double;
   __device__ static __forceinline__ T enc(double v) { return v; }
+  static constexpr double SCALE = 1.0;
+  __device__ static __forceinline__ T enc_scaled(double v) { return v; }
   __device__ static __forceinline__ void sub(T* p, T v) { atomicAdd(p, -v); }
   __device__ static __forceinline__ double dec(T x) { return x; }
 };
@@ -350,7 +358,8 @@ struct ScoreArgs {
   const Real* global_params;
   const uint32_t* counters;
   uint32_t* row_cursor;        // [8 * QSTRIDE] RowQueue cursors (workspace)
-  int row_grab;                // rows per queue grab (0: QROWS)
+  int row_grab;                // queue units per grab (0: QROWS)
+  int part_shift;              // a row is 2^part_shift queue units (parts of its items)
   const Real* weights;         // [3, P] or [3, P, B, B]
   double* energies64;          // [3, P] whole pose
   Real* energies_bp;           // [3, P, B, B] block pair

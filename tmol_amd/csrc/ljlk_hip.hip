@@ -225,7 +225,7 @@ static void launch_stream(const ScoreArgs<Real>& a, int occ, int n_wg, hipStream
     if (n_wg <= 0) n_wg = resident_workgroups(k);
     hipLaunchKernelGGL(k, dim3(n_wg), dim3(256), 0, stream, a);
   };
-  if constexpr (std::is_same<Real, float>::value) {
+  if constexpr (std::is_same<Real, float>::value && !(MODE & M_ELEC)) {
     switch (occ) {
       case 3: go(score_stream_kernel<Real, MODE, 3>); return;
       case 5: go(score_stream_kernel<Real, MODE, 5>); return;
@@ -285,13 +285,14 @@ static int run_score(const tmol_ljlk_stack* st, const tmol_ljlk_block_types* btp
   if ((flags & TMOL_LJLK_WGRAD) && !acc && !det) fill<Real>((Real*)grad, NA3, stream);
   const int n_wg = n_wave_groups;
   int mode = flags & (TMOL_LJLK_DVDX | TMOL_LJLK_WGRAD | TMOL_LJLK_BLOCK_PAIR | TMOL_LJLK_NO_ENERGY);
-  if (ek) mode |= M_ELEC;
   // launch variants (autotuner): waves per SIMD and rows per queue grab
   const int occ = (flags >> 16) & 15;
   a.row_grab = (flags >> 20) & 15;
-  // whole-pose energies and the weighted gradient stream each row's atoms
-  const bool stream_k = !general && !ek && !(flags & TMOL_LJLK_ROW_KERNEL) &&
-                        (mode == 0 || mode == M_WGRAD || mode == (M_WGRAD | M_NOE));
+  // whole-pose energies and the weighted gradient stream each row's atoms,
+  // with elec as a fourth term only there (elec's blocks hold at most 32 atoms)
+  const bool whole = mode == 0 || mode == M_WGRAD || mode == (M_WGRAD | M_NOE);
+  if (ek && (general || !whole)) return TMOL_LJLK_ENOTSUP;
+  const bool stream_k = ek || (!general && !(flags & TMOL_LJLK_ROW_KERNEL) && whole);
   if (det) {
     if constexpr (std::is_same<Real, float>::value) {
       if (stream_k) {
@@ -320,13 +321,16 @@ static int run_score(const tmol_ljlk_stack* st, const tmol_ljlk_block_types* btp
     return TMOL_LJLK_ENOTSUP;
   }
   if (stream_k) {
-    switch (mode) {
+    switch (mode | (ek ? M_ELEC : 0)) {
       case 0: launch_stream<Real, 0>(a, occ, n_wg, stream); break;
       case M_WGRAD: launch_stream<Real, M_WGRAD>(a, occ, n_wg, stream); break;
-      default: launch_stream<Real, M_WGRAD | M_NOE>(a, occ, n_wg, stream); break;
+      case M_WGRAD | M_NOE: launch_stream<Real, M_WGRAD | M_NOE>(a, occ, n_wg, stream); break;
+      case M_ELEC: launch_stream<Real, M_ELEC>(a, 0, n_wg, stream); break;
+      case M_ELEC | M_WGRAD: launch_stream<Real, M_ELEC | M_WGRAD>(a, 0, n_wg, stream); break;
+      default: launch_stream<Real, M_ELEC | M_WGRAD | M_NOE>(a, 0, n_wg, stream); break;
     }
     mode = -1;  // launched
-  } else if (occ && !general && !ek && (mode == 0 || mode == M_WGRAD)) {
+  } else if (occ && !general && (mode == 0 || mode == M_WGRAD)) {
     if (mode == 0)
       launch_rows_occ<Real, 0>(a, occ, n_wg, stream);
     else
@@ -335,11 +339,6 @@ static int run_score(const tmol_ljlk_stack* st, const tmol_ljlk_block_types* btp
   }
   switch (mode) {
     case -1: break;
-    case M_ELEC: launch_rows<Real, M_ELEC>(a, n_wave_groups, stream); break;
-    case M_ELEC | M_WGRAD: launch_rows<Real, M_ELEC | M_WGRAD>(a, n_wave_groups, stream); break;
-    case M_ELEC | M_WGRAD | M_NOE:
-      launch_rows<Real, M_ELEC | M_WGRAD | M_NOE>(a, n_wave_groups, stream);
-      break;
     case 0: launch_score<Real, 0>(a, general, n_wg, stream); break;
     case M_DVDX: launch_score<Real, M_DVDX>(a, general, n_wg, stream); break;
     case M_WGRAD: launch_score<Real, M_WGRAD>(a, general, n_wg, stream); break;

@@ -18,11 +18,15 @@
 //                distance and, only in chunks holding atoms within 4 bonds
 //                of g1, the count-pair separation from precombined path
 //                bytes.  In-range pairs of non-zero weight are
-//                ballot-compacted into the LJ (and LK) FIFOs
-//   phase B      64 FIFO entries at a time, one per lane (the evaluators of
-//                the row kernel); gradients accumulate in LDS as 64-bit fixed
-//                point and a ring chunk is flushed to global memory when its
-//                slots are reused, g1 at row end
+//                ballot-compacted into the pair FIFO
+//   phase B      64 FIFO entries at a time, one per lane: LJ, and elec in the
+//                fused mode (its 5.5 A reach lies inside LJ's 6 A, so a pair's
+//                distance, LDS reads and gradient sums are shared); the
+//                heavy-heavy entries among them, about a quarter, are
+//                compacted again into the LK FIFO, evaluated 64 at a time.
+//                Gradients accumulate in LDS as 64-bit fixed point and a ring
+//                chunk is flushed to global memory when its slots are reused,
+//                g1 at row end
 //
 // Per block pair the row kernel pays staging, a cull of both blocks and
 // bookkeeping; here that work is per 64 atoms of the stream, and the pair
@@ -31,6 +35,13 @@
 // q[c1] = min_c2 cs[c1][c2] + pd2[c2] combined once per g2 atom (absent
 // connections carry path distance 6, so their sums never reach below 5), the
 // count-pair rule of impl.hh:47-67 / count_pair.hh:162-207.
+//
+// A wave takes a part of a row: A.part_shift > 0 splits every row's items into
+// 2^part_shift parts, so that a batch with fewer rows than resident waves
+// still fills the chip (see row_part_shift).
+//
+// Bound: VALU issue.  LDS (40 KB a workgroup: four of them fill a CU's 160 KB)
+// and 128 VGPRs both hold the gradient modes at 4 waves per SIMD.
 #pragma once
 
 #include "ljlk_score_rows.hh"
@@ -42,42 +53,52 @@ constexpr int SRING = 3 * SCH;         // ring slots
 constexpr int SSLOTS = TILE + SRING;   // g1 slots 0..31, ring 32..127
 constexpr int SLIST = 128;             // FIFO capacity (drained at 64)
 constexpr uint32_t Q_NONE = 0x64646464u;  // q bytes of blocks more than 4 bonds apart (100)
-constexpr uint32_t Q_HEAVY = 0x80000000u; // bit 7 of byte 3: heavy atom
 constexpr uint32_t Q_LIG = 0x00800000u;   // bit 7 of byte 2: ligand-fragment block
 
-// Copies of the LDS gradient accumulators, chosen by lane: LDS atomics on one
-// address serialize, and consecutive FIFO entries share their g1 atom (and,
-// less often, their ring atom).  g1 slots: G1COPIES copies (lane % G1COPIES);
-// ring slots: RINGCOPIES copies ((lane / 2) % RINGCOPIES).  Flushes add the
-// copies.
-#ifndef TMOL_STREAM_G1COPIES
-#define TMOL_STREAM_G1COPIES 2
-#endif
-#ifndef TMOL_STREAM_RINGCOPIES
-#define TMOL_STREAM_RINGCOPIES 1
-#endif
-constexpr int G1COPIES = TMOL_STREAM_G1COPIES;
-constexpr int RINGCOPIES = TMOL_STREAM_RINGCOPIES;
+// Gradient accumulators: one entry per slot, and a second copy of g1's for odd
+// lanes: LDS atomics on one address serialize, and consecutive FIFO entries
+// share their g1 atom.  Ring slots stay single (a second copy of them costs a
+// workgroup per CU).  All in one row per component, so an entry's three
+// atomics differ by constant offsets.
+constexpr int GROW = SSLOTS + TILE;
+
+// FIFO entry: g1 slot (5 bits) | second slot (7 bits) | LJ / LK weight code
+// << 12 | elec weight code << 14; code 0: weight 1, 1: 0.2, 2: no contribution
+constexpr int CODE_LJ = 12, CODE_EL = 14;
+constexpr int CODE_NONE = 2;
 
 template <typename Real, int MODE>
 struct StreamLDS {
   using C = RowCtx<Real, MODE>;
   using T = typename LdsAcc<Real>::T;
   static constexpr int NGP = C::NG > 0 ? C::NG : 1;
-  T gring[RINGCOPIES][NGP][3][C::DERIV ? SRING : 1];  // ring slots TILE.. (index - TILE)
-  T g1acc[G1COPIES][NGP][3][C::DERIV ? TILE : 1];     // g1 slots 0..31
-  T ebp[1][3];  // block-pair modes run the row kernel; kept for the evaluators
-  Real wt[1][3];
+  T grad[NGP][3][C::DERIV ? GROW : 1];
   alignas(4 * sizeof(Real)) Real pos[SSLOTS][4];  // x, y, z, lj_radius
-  alignas(4 * sizeof(Real)) Real prm[SSLOTS][4];  // sqrt(lj_wdepth), K, 1/lambda^2, lk_volume
-  uint32_t tq[SCH];      // test chunk atoms: connection bytes q | Q_HEAVY | Q_LIG
-  uint8_t flg[SSLOTS];
-  uint16_t lj[SLIST];
-  uint16_t lk[SLIST];
+  alignas(4 * sizeof(Real)) Real prm[SSLOTS][4];  // K, 1/lambda^2, lk_volume, charge
+  alignas(2 * sizeof(Real)) Real lj2[SSLOTS][2];  // sqrt(lj_wdepth), flags (pack_flags)
+  uint16_t lj[SLIST];    // pair FIFO; its upper half holds the test chunk's tq
+  uint16_t lk[SLIST];    // LK FIFO; its upper half holds the raw chunk's marks
   int32_t atom[SRING];   // global atom of each ring slot
   uint32_t pd1[TILE];    // g1 atoms' connection path distances, byte per connection
-  uint8_t mark[WAVE];    // raw chunk: a block's first atom sits at this lane
+  uint32_t epd1[C::ELEC ? TILE : 1];  // elec's
+  uint32_t teq[C::ELEC ? SCH : 1];    // test chunk atoms: elec's connection bytes
+  // both FIFOs hold fewer than 64 entries outside phase B and the test loop
+  // (which reads tq before it appends)
+  __device__ __forceinline__ uint32_t* tq() { return (uint32_t*)(lj + WAVE); }
+  __device__ __forceinline__ uint8_t* mark() { return (uint8_t*)(lk + WAVE); }
 };
+static_assert(SCH * 4 <= 2 * (SLIST - WAVE) && WAVE <= 2 * (SLIST - WAVE), "aliased FIFO halves");
+
+__device__ __forceinline__ float pack_flags(int f, float) { return __int_as_float(f); }
+__device__ __forceinline__ double pack_flags(int f, double) { return double(f); }
+__device__ __forceinline__ int unpack_flags(float v) { return __float_as_int(v); }
+__device__ __forceinline__ int unpack_flags(double v) { return int(v); }
+
+// count-pair weight of a 2-bit code
+template <typename Real>
+__device__ __forceinline__ Real code_weight(int code) {
+  return code == 0 ? Real(1) : (code == 1 ? Real(0.2) : Real(0));
+}
 
 // smallest of the four 7-bit byte fields of v, capped at 5 (the count-pair
 // separation from packed sums)
@@ -121,26 +142,42 @@ __device__ __forceinline__ void conn_rows(const StackView& s, int g1, int g2, in
   for (int c1 = 0; c1 < nc1; ++c1) cs[c1] = (uint32_t)e[4 + c1];
 }
 
-// gradient of an entry's pair: + to the g1 atom's slot s1, - to slot s2
-// (a ring slot, or a g1 slot for intra-block pairs), into the lane's copies
+// gradient gs (x1 - x2) of an entry's pair: + to the g1 atom's slot s1 (odd
+// lanes: its second copy), - to slot s2 (a ring slot, or a g1 slot for
+// intra-block pairs)
 template <typename Real, int MODE>
-__device__ __forceinline__ void grad_scatter(StreamLDS<Real, MODE>& L, int term, int s1, int s2,
-                                             Real gx, Real gy, Real gz, int lane) {
+__device__ __forceinline__ void stream_scatter(StreamLDS<Real, MODE>& L, int term, int s1, int s2,
+                                               Real gs, Real dx, Real dy, Real dz, int odd) {
   using Acc = LdsAcc<Real>;
   using T = typename Acc::T;
-  const int c1 = lane & (G1COPIES - 1);
-  const T ex = Acc::enc(gx), ey = Acc::enc(gy), ez = Acc::enc(gz);
-  T* b1 = &L.g1acc[c1][term][0][s1];
-  const bool g2_in_g1 = s2 < TILE;
-  T* b2 = g2_in_g1 ? &L.g1acc[c1][term][0][s2]
-                   : &L.gring[(lane >> 1) & (RINGCOPIES - 1)][term][0][s2 - TILE];
-  const int k2 = g2_in_g1 ? TILE : SRING;
+  const Real g = gs * Acc::SCALE;
+  const T ex = Acc::enc_scaled(g * dx), ey = Acc::enc_scaled(g * dy), ez = Acc::enc_scaled(g * dz);
+  T* b1 = &L.grad[term][0][s1 + odd];
+  T* b2 = &L.grad[term][0][s2];
   atomicAdd(b1, ex);
-  atomicAdd(b1 + TILE, ey);
-  atomicAdd(b1 + 2 * TILE, ez);
+  atomicAdd(b1 + GROW, ey);
+  atomicAdd(b1 + 2 * GROW, ez);
   Acc::sub(b2, ex);
-  Acc::sub(b2 + k2, ey);
-  Acc::sub(b2 + 2 * k2, ez);
+  Acc::sub(b2 + GROW, ey);
+  Acc::sub(b2 + 2 * GROW, ez);
+}
+
+// one atom's accumulated gradient component to global memory
+template <typename Real, int MODE>
+__device__ __forceinline__ void flush_value(const ScoreArgs<Real>& A, int t, int64_t i,
+                                            typename LdsAcc<Real>::T acc) {
+  using C = RowCtx<Real, MODE>;
+  if (C::DET) {
+    if (acc != 0) atomicAdd(&A.fixed[int64_t(t) * A.n_atoms * 3 + i], acc);
+    return;
+  }
+  const Real v = LdsAcc<Real>::dec(acc);
+  if (v != Real(0)) {
+    if (C::DVDX)
+      unsafeAtomicAdd(&A.dvdx[int64_t(t) * A.n_atoms * 3 + i], v);
+    else
+      unsafeAtomicAdd(&A.grad[i], v);
+  }
 }
 
 // flush the gradients of ring chunk r (n atoms, slots TILE + SCH r ...) to
@@ -152,32 +189,18 @@ __device__ __forceinline__ void flush_chunk(StreamLDS<Real, MODE>& L, const Scor
   if (!C::DERIV) return;
   for (int i = lane; i < 3 * n; i += WAVE) {
     const int a = i / 3, k = i - 3 * a;
-    const int slot = SCH * r + a;
     const int64_t atom = L.atom[SCH * r + a];
 #pragma unroll
     for (int t = 0; t < C::NG; ++t) {
-      typename LdsAcc<Real>::T acc = 0;
-#pragma unroll
-      for (int c = 0; c < RINGCOPIES; ++c) {
-        acc += L.gring[c][t][k][slot];
-        L.gring[c][t][k][slot] = 0;
-      }
-      if (C::DET) {
-        if (acc != 0) atomicAdd(&A.fixed[(int64_t(t) * A.n_atoms + atom) * 3 + k], acc);
-        continue;
-      }
-      const Real v = LdsAcc<Real>::dec(acc);
-      if (v != Real(0)) {
-        if (C::DVDX)
-          unsafeAtomicAdd(&A.dvdx[(int64_t(t) * A.n_atoms + atom) * 3 + k], v);
-        else
-          unsafeAtomicAdd(&A.grad[atom * 3 + k], v);
-      }
+      auto* g = &L.grad[t][k][TILE + SCH * r + a];
+      const auto acc = *g;
+      *g = 0;
+      flush_value<Real, MODE>(A, t, atom * 3 + k, acc);
     }
   }
 }
 
-// g1's atoms [0, n) (slots 0..n-1, contiguous atoms from atom0)
+// g1's atoms [0, n) (slots 0..n-1 and their copies, contiguous atoms from atom0)
 template <typename Real, int MODE>
 __device__ __forceinline__ void flush_g1(StreamLDS<Real, MODE>& L, const ScoreArgs<Real>& A, int n,
                                          int64_t atom0, int lane) {
@@ -187,25 +210,97 @@ __device__ __forceinline__ void flush_g1(StreamLDS<Real, MODE>& L, const ScoreAr
     const int a = i / 3, k = i - 3 * a;
 #pragma unroll
     for (int t = 0; t < C::NG; ++t) {
-      typename LdsAcc<Real>::T acc = 0;
-#pragma unroll
-      for (int c = 0; c < G1COPIES; ++c) {
-        acc += L.g1acc[c][t][k][a];
-        L.g1acc[c][t][k][a] = 0;
-      }
-      if (C::DET) {
-        if (acc != 0) atomicAdd(&A.fixed[(int64_t(t) * A.n_atoms + atom0) * 3 + i], acc);
-        continue;
-      }
-      const Real v = LdsAcc<Real>::dec(acc);
-      if (v != Real(0)) {
-        if (C::DVDX)
-          unsafeAtomicAdd(&A.dvdx[(int64_t(t) * A.n_atoms + atom0) * 3 + i], v);
-        else
-          unsafeAtomicAdd(&A.grad[atom0 * 3 + i], v);
-      }
+      auto* g = &L.grad[t][k][a];
+      const auto acc = g[0] + g[SSLOTS];
+      g[0] = g[SSLOTS] = 0;
+      flush_value<Real, MODE>(A, t, atom0 * 3 + i, acc);
     }
   }
+}
+
+// running energies of one lane's entries
+struct StreamEnergies {
+  LaneSum atr, rep, lk, el;
+};
+
+// LK entries [0, consume) of the FIFO, consume <= 64, one per lane
+template <typename Real, int MODE>
+__device__ __forceinline__ void stream_lk(StreamLDS<Real, MODE>& L, int consume,
+                                          const GlobalParams<Real>& gp, const Real* wrow,
+                                          StreamEnergies& en, int lane, int odd) {
+  using C = RowCtx<Real, MODE>;
+  using V = typename V4<Real>::T;
+  if (lane >= consume) return;
+  const int e = L.lk[lane];
+  const int s1 = e & 31, s2 = (e >> 5) & 127;
+  const Real wcp = (e >> CODE_LJ) & 1 ? Real(0.2) : Real(1);
+  const V p1 = *(const V*)L.pos[s1], p2 = *(const V*)L.pos[s2];
+  const V q1 = *(const V*)L.prm[s1], q2 = *(const V*)L.prm[s2];
+  const int f1 = unpack_flags(L.lj2[s1][1]), f2 = unpack_flags(L.lj2[s2][1]);
+  const Real dx = p1.x - p2.x, dy = p1.y - p2.y, dz = p1.z - p2.z;
+  const Real d2 = dx * dx + dy * dy + dz * dz;
+  const Real inv_d = fast_rsqrt(d2);
+  const Real dist = d2 > Real(0) ? d2 * inv_d : Real(0);  // coincident atoms: d = 0
+  const Real sigma = lj_sigma(f1, f2, p1.w, p2.w, gp);
+  const bool cc = (f1 & F_CARBON_LK) && (f2 & F_CARBON_LK);
+  Real d_min, cdmin, cdmax;
+  lk_knots(sigma, cc, d_min, cdmin, cdmax);
+  const LkSide<Real> side[2] = {{-q2.z * q1.x, p1.w, q1.y}, {-q1.z * q2.x, p2.w, q2.y}};
+  Real v, dv;
+  lk_sides<Real, C::DERIV>(dist, d_min, cdmin, cdmax, side, gp, v, dv);
+  if (!C::NOE) en.lk.add(wcp * v);
+  if (C::DERIV && dist > Real(0)) {
+    Real gs = wcp * dv;
+    if (gs != Real(0)) {
+      gs *= inv_d;
+      if (C::WGRAD) gs *= wrow[2];
+      stream_scatter<Real, MODE>(L, C::DVDX ? 2 : 0, s1, s2, gs, dx, dy, dz, odd);
+    }
+  }
+}
+
+// pair entries [0, consume) of the FIFO, consume <= 64, one per lane: LJ (and
+// elec); returns whether this lane's entry (in *entry) goes on to LK
+template <typename Real, int MODE>
+__device__ __forceinline__ bool stream_pairs(StreamLDS<Real, MODE>& L, int consume,
+                                             const GlobalParams<Real>& gp,
+                                             const ElecConst<Real>& ek, const Real* wrow, Real wel,
+                                             StreamEnergies& en, int lane, int odd, int* entry) {
+  using C = RowCtx<Real, MODE>;
+  using V = typename V4<Real>::T;
+  if (lane >= consume) return false;
+  const int e = L.lj[lane];
+  *entry = e;
+  const int s1 = e & 31, s2 = (e >> 5) & 127;
+  const V p1 = *(const V*)L.pos[s1], p2 = *(const V*)L.pos[s2];
+  const Real se1 = L.lj2[s1][0], se2 = L.lj2[s2][0];
+  const int f1 = unpack_flags(L.lj2[s1][1]), f2 = unpack_flags(L.lj2[s2][1]);
+  const int code = C::ELEC ? (e >> CODE_LJ) & 3 : (e >> CODE_LJ) & 1;
+  const Real dx = p1.x - p2.x, dy = p1.y - p2.y, dz = p1.z - p2.z;
+  const Real d2 = dx * dx + dy * dy + dz * dz;
+  const Real inv_d = fast_rsqrt(d2);
+  const Real dist = d2 > Real(0) ? d2 * inv_d : Real(0);  // coincident atoms: d = 0
+  const Real sigma = lj_sigma(f1, f2, p1.w, p2.w, gp);
+  const Real wcp = C::ELEC ? code_weight<Real>(code) : (code ? Real(0.2) : Real(1));
+  Real atr, rep, dlj;
+  lj_pair<Real, C::DERIV>(dist, sigma, se1 * se2, wcp, gp, atr, rep, dlj);
+  if (!C::NOE) {
+    en.atr.add(atr);
+    en.rep.add(rep);
+  }
+  const bool inside = dist < sigma;
+  Real gs = dlj;
+  if (C::WGRAD) gs *= inside ? wrow[1] : wrow[0];
+  if (C::ELEC) {
+    const Real qq = code_weight<Real>(e >> CODE_EL) * (L.prm[s1][3] * L.prm[s2][3]);
+    Real v, dv;
+    elec_unit<Real, C::DERIV>(dist, ek, v, dv);
+    if (!C::NOE) en.el.add(qq * v);
+    if (C::DERIV) gs += wel * (qq * dv);
+  }
+  if (C::DERIV && gs != Real(0) && dist > Real(0))
+    stream_scatter<Real, MODE>(L, C::DVDX && inside ? 1 : 0, s1, s2, gs * inv_d, dx, dy, dz, odd);
+  return (f1 & f2 & F_HEAVY) && (!C::ELEC || code != CODE_NONE);
 }
 
 template <int MODE, int OCC>
@@ -218,28 +313,35 @@ __global__ __launch_bounds__(256, (stream_waves_per_simd<MODE, OCC>())) void sco
     ScoreArgs<Real> A) {
   using C = RowCtx<Real, MODE>;
   using V = typename V4<Real>::T;
-  static_assert(!C::BP && !C::ELEC, "block-pair and elec modes run the row kernel");
+  static_assert(!C::BP && !(C::ELEC && (C::DVDX || C::DET)), "modes of the row kernel");
   __shared__ StreamLDS<Real, MODE> lds_all[WAVES_PER_WG];
   const int lane = lane_id();
   StreamLDS<Real, MODE>& L = lds_all[uni(threadIdx.x / WAVE)];
   const GlobalParams<Real> gp = load_global_params(A.global_params);
+  const ElecConst<Real> ek = A.ek;
   const StackView& s = A.s;
   const BTView& bt = A.bt;
-  RowQueue queue(A.row_cursor, s.G, A.row_grab);
+  const int shift = A.part_shift;
+  RowQueue queue(A.row_cursor, int64_t(s.G) << shift, A.row_grab);
   const Real cull_pad = gp.max_dis + Real(1e-3);
+  const Real cut2 = C::ELEC && ek.cull2 > gp.max_dis2 ? ek.cull2 : gp.max_dis2;
   const int u = lane & (SCH - 1), half = lane >> 5;
+  const int odd = (lane & 1) ? SSLOTS : 0;
 
   if (C::DERIV) {
-    auto* g = &L.gring[0][0][0][0];
-    for (int i = lane; i < RINGCOPIES * L.NGP * 3 * SRING; i += WAVE) g[i] = 0;
-    auto* gb = &L.g1acc[0][0][0][0];
-    for (int i = lane; i < G1COPIES * L.NGP * 3 * TILE; i += WAVE) gb[i] = 0;
+    auto* g = &L.grad[0][0][0];
+    for (int i = lane; i < L.NGP * 3 * GROW; i += WAVE) g[i] = 0;
   }
   wave_sync();
 
-  for (int64_t row = queue.next(); row >= 0; row = queue.next()) {
-    const int n_items = uni((int)min<int64_t>(A.w.row_count[row], A.w.row_cap));
-    if (n_items == 0) continue;
+  for (int64_t unit = queue.next(); unit >= 0; unit = queue.next()) {
+    const int64_t row = unit >> shift;
+    const int n_row = uni((int)min<int64_t>(A.w.row_count[row], A.w.row_cap));
+    // this part's items [k_lo, n_items) of the row
+    const int64_t part = unit - (row << shift);
+    const int k_lo = int((n_row * part) >> shift);
+    const int n_items = int((n_row * (part + 1)) >> shift);
+    if (n_items == k_lo) continue;
     const int g1 = (int)row;
     const int t1 = uni(s.block_type[g1]);
     const int n1 = uni(bt.n_atoms[t1]);
@@ -254,63 +356,74 @@ __global__ __launch_bounds__(256, (stream_waves_per_simd<MODE, OCC>())) void sco
       wrow[1] = A.weights[s.P + p];
       wrow[2] = A.weights[2 * s.P + p];
     }
+    const Real wel = (C::ELEC && C::WGRAD) ? A.weights[3 * s.P + p] : Real(0);
     const Real reach1 = sph1.w + cull_pad;
     const Real reach1_2 = reach1 * reach1;
+    auto stage = [&](int slot, const AtomRegs<Real>& R) {
+      V pp, pq;
+      pp.x = R.x; pp.y = R.y; pp.z = R.z; pp.w = R.r0.x;
+      pq.x = R.r0.z; pq.y = R.r0.w; pq.z = R.vol; pq.w = C::ELEC ? R.q : Real(0);
+      *(V*)L.pos[slot] = pp;
+      *(V*)L.prm[slot] = pq;
+      L.lj2[slot][0] = R.r0.y;
+      L.lj2[slot][1] = pack_flags(R.flags, Real(0));
+    };
     // ---- stage g1 into slots 0..31
-    bool heavy1 = false;
     if (lane < n1) {
       AtomRegs<Real> R;
-      load_atom<Real, false>(R, A, t1, o1, lane);
-      V pp, qq;
-      pp.x = R.x; pp.y = R.y; pp.z = R.z; pp.w = R.r0.x;
-      qq.x = R.r0.y; qq.y = R.r0.z; qq.z = R.r0.w; qq.w = R.vol;
-      *(V*)L.pos[lane] = pp;
-      *(V*)L.prm[lane] = qq;
-      L.flg[lane] = (uint8_t)R.flags;
+      load_atom<Real, C::ELEC>(R, A, t1, o1, lane);
+      stage(lane, R);
       L.pd1[lane] = R.pd;
-      heavy1 = (R.flags & F_HEAVY) != 0;
+      if (C::ELEC) L.epd1[lane] = R.epd;
     }
-    const uint32_t hmask1 = (uint32_t)__ballot(heavy1);
-    LaneSum e_atr, e_rep, e_lk;
-    int n_lj = 0, n_lk = 0, seq_lj = 0, seq_lk = 0, done_lj = 0, done_lk = 0;
-    int end_lj[3] = {0, 0, 0}, end_lk[3] = {0, 0, 0};
+    StreamEnergies en;
+    int n_lj = 0, n_lk = 0, seq_lj = 0, done_lj = 0;
+    int end_lj[3] = {0, 0, 0};
     int cnt[3] = {0, 0, 0};  // atoms held by each ring chunk (0: free)
     int cur = 0;             // ring chunk being filled
     int fill = 0;            // its atoms so far
     bool cur_cp = false, cur_lig = false;  // it holds atoms within 4 bonds / ligand atoms
     wave_sync();
 
-    auto drain = [&](bool all) {
-      const int c1 = all ? n_lj : (n_lj & ~(WAVE - 1));
-      const int c2 = all ? n_lk : (n_lk & ~(WAVE - 1));
-      if (c1 > 0) eval_lj<Real, MODE>(L, c1, gp, wrow, e_atr, e_rep, lane);
-      if (c2 > 0) eval_lk<Real, MODE>(L, c2, gp, wrow, e_lk, lane);
+    auto drain_lk = [&]() {
+      const int c = min(n_lk, WAVE);
+      stream_lk<Real, MODE>(L, c, gp, wrow, en, lane, odd);
       wave_sync();
-      fifo_shift(L.lj, c1, n_lj, lane);
-      fifo_shift(L.lk, c2, n_lk, lane);
-      n_lj -= c1;
-      done_lj += c1;
-      n_lk -= c2;
-      done_lk += c2;
+      fifo_shift(L.lk, c, n_lk, lane);
+      n_lk -= c;
     };
-    auto drain_full = [&]() {
-      if (n_lj >= WAVE || n_lk >= WAVE) drain(false);
+    // one batch of the pair FIFO; its heavy-heavy entries join the LK FIFO
+    auto drain = [&]() {
+      const int c = min(n_lj, WAVE);
+      int e = 0;
+      const bool hv = stream_pairs<Real, MODE>(L, c, gp, ek, wrow, wel, en, lane, odd, &e);
+      const uint64_t m = __ballot(hv);
+      if (hv) L.lk[n_lk + lanes_below(m)] = (uint16_t)(e & ((1 << CODE_EL) - 1));
+      n_lk += __popcll(m);
+      wave_sync();
+      fifo_shift(L.lj, c, n_lj, lane);
+      n_lj -= c;
+      done_lj += c;
+      if (n_lk >= WAVE) drain_lk();
     };
-    auto append = [&](bool in, bool hv, int e) {
+    auto append = [&](bool in, int e) {
       const uint64_t m = __ballot(in);
       if (in) L.lj[n_lj + lanes_below(m)] = (uint16_t)e;
       n_lj += __popcll(m);
       seq_lj += __popcll(m);
-      const uint64_t mh = __ballot(hv);
-      if (hv) L.lk[n_lk + lanes_below(mh)] = (uint16_t)e;
-      n_lk += __popcll(mh);
-      seq_lk += __popcll(mh);
+      wave_sync();
+      if (n_lj >= WAVE) drain();
     };
     // ring chunk r no longer referenced: evaluate what still points at it,
-    // flush its atoms
+    // flush its atoms (LK entries are in ring order, so the oldest pending one
+    // tells whether any is left)
     auto retire = [&](int r) {
       if (cnt[r] == 0) return;
-      if (end_lj[r] > done_lj || end_lk[r] > done_lk) drain(true);
+      if (end_lj[r] > done_lj) drain();
+      if (n_lk > 0) {
+        const int head = (uni((int)L.lk[0]) >> 10) & 3;  // 0: intra-block, 1 + ring chunk
+        if (head == 0 || head == r + 1) drain_lk();
+      }
       flush_chunk<Real, MODE>(L, A, r, cnt[r], lane);
       cnt[r] = 0;
     };
@@ -319,31 +432,38 @@ __global__ __launch_bounds__(256, (stream_waves_per_simd<MODE, OCC>())) void sco
       const int r = cur;
       const int n = fill;
       const V tr = *(const V*)L.pos[TILE + SCH * r + u];
-      const uint32_t qb = L.tq[u];
-      const bool heavy2 = (qb & Q_HEAVY) != 0;
+      const uint32_t qb = L.tq()[u];
+      const uint32_t eqb = C::ELEC ? L.teq[u] : 0;
       const bool lig2 = (qb & Q_LIG) != 0;
       const bool ok_u = u < n;
       const int ebase = (TILE + SCH * r + u) << 5;
+      wave_sync();
       for (int t = 0; t < n1; t += 2) {
         const int ta = t + half;
-        const V P1 = *(const V*)L.pos[ta < n1 ? ta : t];
+        const int tl = ta < n1 ? ta : t;
+        const V P1 = *(const V*)L.pos[tl];
         const Real dx = P1.x - tr.x, dy = P1.y - tr.y, dz = P1.z - tr.z;
         const Real d2 = dx * dx + dy * dy + dz * dz;
-        bool in = ok_u && ta < n1 && d2 < gp.max_dis2;
-        bool w02 = false;
+        bool in = ok_u && ta < n1 && d2 < cut2;
+        int e = ebase | ta;
         if (cur_cp) {
-          int sep = min_sep_bytes(qb + L.pd1[ta < n1 ? ta : t]);
+          int sep = min_sep_bytes(qb + L.pd1[tl]);
           if (cur_lig && lig1 && lig2 && (sep == 3 || sep == 4)) sep = 5;
-          in = in && sep >= 4;
-          w02 = sep == 4;
+          const int code = sep > 4 ? 0 : (sep == 4 ? 1 : CODE_NONE);
+          if (C::ELEC) {
+            int sep_e = min_sep_bytes(eqb + L.epd1[tl]);
+            if (cur_lig && lig1 && lig2 && (sep_e == 3 || sep_e == 4)) sep_e = 5;
+            const int code_e = sep_e > 4 ? 0 : (sep_e == 4 ? 1 : CODE_NONE);
+            in = in && (code != CODE_NONE || code_e != CODE_NONE);
+            e |= code_e << CODE_EL;
+          } else {
+            in = in && code != CODE_NONE;
+          }
+          e |= code << CODE_LJ;
         }
-        const bool hv = in && heavy2 && ((hmask1 >> ta) & 1u);
-        append(in, hv, ebase | ta | (w02 ? (1 << 12) : 0));
-        wave_sync();
-        drain_full();
+        append(in, e);
       }
       end_lj[r] = seq_lj;
-      end_lk[r] = seq_lk;
       cnt[r] = n;
       cur = cur == 2 ? 0 : cur + 1;
       fill = 0;
@@ -351,28 +471,30 @@ __global__ __launch_bounds__(256, (stream_waves_per_simd<MODE, OCC>())) void sco
       retire(cur);  // the chunk two before: its entries are consumed by now
     };
 
-    int k0 = 0;
-    if (uni(A.w.row_items[row * A.w.row_cap]) == g1) {
-      // ---- intra-block pairs a1 < a2 of non-zero weight (prepared table)
-      const int n_ip = uni(A.intra_count[t1]);
-      const uint16_t* ip = A.intra_pairs + int64_t(t1) * INTRA_MAX;
-      for (int j0 = 0; j0 < n_ip; j0 += WAVE) {
-        bool in = false, hv = false, w02 = false;
-        int a1 = 0, a2 = 0;
-        if (j0 + lane < n_ip) {
-          const int e = ip[j0 + lane];
-          a1 = e & 31;
-          a2 = (e >> 5) & 31;
-          const V pa = *(const V*)L.pos[a1], pb = *(const V*)L.pos[a2];
-          const Real dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
-          in = dx * dx + dy * dy + dz * dz < gp.max_dis2;
-          w02 = (e >> 10) & 1;
-          hv = in && ((hmask1 >> a1) & (hmask1 >> a2) & 1u);
+    int k0 = k_lo;
+    if (k_lo == 0 && uni(A.w.row_items[row * A.w.row_cap]) == g1) {
+      // ---- intra-block pairs a1 < a2 of non-zero weight (prepared tables)
+      auto intra = [&](int n_ip, const uint16_t* ip, Real cut2, int code_other, int code_shift) {
+        for (int j0 = 0; j0 < n_ip; j0 += WAVE) {
+          bool in = false;
+          int e = 0;
+          if (j0 + lane < n_ip) {
+            const int w = ip[j0 + lane];
+            const int a1 = w & 31, a2 = (w >> 5) & 31;
+            const V pa = *(const V*)L.pos[a1], pb = *(const V*)L.pos[a2];
+            const Real dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
+            in = dx * dx + dy * dy + dz * dz < cut2;
+            e = a1 | (a2 << 5) | code_other | (((w >> 10) & 1) << code_shift);
+          }
+          append(in, e);
         }
-        append(in, hv, a1 | (a2 << 5) | (w02 ? (1 << 12) : 0));
-        wave_sync();
-        drain_full();
-      }
+      };
+      intra(uni(A.intra_count[t1]), A.intra_pairs + int64_t(t1) * INTRA_MAX, gp.max_dis2,
+            C::ELEC ? CODE_NONE << CODE_EL : 0, CODE_LJ);
+      // elec's own table (representative separations, charged atoms only)
+      if (C::ELEC)
+        intra(uni(A.e_intra_count[t1]), A.e_intra_pairs + int64_t(t1) * INTRA_MAX, ek.cull2,
+              CODE_NONE << CODE_LJ, CODE_EL);
       k0 = 1;
     }
 
@@ -406,11 +528,11 @@ __global__ __launch_bounds__(256, (stream_waves_per_simd<MODE, OCC>())) void sco
 
       for (int q0 = 0; q0 < total; q0 += WAVE) {
         // ---- raw chunk: lane -> (block, atom) through start markers
-        L.mark[lane] = 0;
+        L.mark()[lane] = 0;
         wave_sync();
-        if (d_n2 > 0 && d_pre >= q0 && d_pre < q0 + WAVE) L.mark[d_pre - q0] = 1;
+        if (d_n2 > 0 && d_pre >= q0 && d_pre < q0 + WAVE) L.mark()[d_pre - q0] = 1;
         wave_sync();
-        const uint64_t M = __ballot(L.mark[lane] != 0);
+        const uint64_t M = __ballot(L.mark()[lane] != 0);
         // blocks with atoms that start at or before q0, less one: the block
         // holding stream position q0 (in lane order over blocks with atoms)
         const int kfirst = __popcll(__ballot(d_n2 > 0 && d_pre <= q0)) - 1;
@@ -427,7 +549,7 @@ __global__ __launch_bounds__(256, (stream_waves_per_simd<MODE, OCC>())) void sco
         AtomRegs<Real> R;
         bool near = false;
         if (valid && a >= 0 && a < (info >> 8)) {
-          load_atom<Real, false>(R, A, t2, o2, a);
+          load_atom<Real, C::ELEC>(R, A, t2, o2, a);
           const Real ex = R.x - sph1.x, ey = R.y - sph1.y, ez = R.z - sph1.z;
           near = ex * ex + ey * ey + ez * ez < reach1_2;
         }
@@ -435,15 +557,17 @@ __global__ __launch_bounds__(256, (stream_waves_per_simd<MODE, OCC>())) void sco
         const int n_surv = __popcll(mnear);
         if (n_surv == 0) continue;
         // combined connection bytes q (count pair) for atoms within 4 bonds
-        uint32_t qv = Q_NONE;
+        uint32_t qv = Q_NONE, eqv = Q_NONE;
         const uint64_t mcp = __ballot(near && (info & 1));
         if (mcp) {
           uint32_t csk[MAX_CONN];
 #pragma unroll
           for (int c1 = 0; c1 < MAX_CONN; ++c1) csk[c1] = (uint32_t)__shfl((int)cs[c1], k, WAVE);
-          if (info & 1) qv = combine_q(csk, R.pd);
+          if (info & 1) {
+            qv = combine_q(csk, R.pd);
+            if (C::ELEC) eqv = combine_q(csk, R.epd);
+          }
         }
-        qv |= (near && (R.flags & F_HEAVY)) ? Q_HEAVY : 0u;
         qv |= (info & 2) ? Q_LIG : 0u;
         const bool any_lig = __ballot(near && (info & 2)) != 0;
         const int rk = lanes_below(mnear);
@@ -454,14 +578,9 @@ __global__ __launch_bounds__(256, (stream_waves_per_simd<MODE, OCC>())) void sco
           const bool mine = near && rk >= done && rk < done + take;
           if (mine) {
             const int pos = fill + rk - done;
-            const int slot = TILE + SCH * cur + pos;
-            V pp, pq;
-            pp.x = R.x; pp.y = R.y; pp.z = R.z; pp.w = R.r0.x;
-            pq.x = R.r0.y; pq.y = R.r0.z; pq.z = R.r0.w; pq.w = R.vol;
-            *(V*)L.pos[slot] = pp;
-            *(V*)L.prm[slot] = pq;
-            L.tq[pos] = qv;
-            L.flg[slot] = (uint8_t)R.flags;
+            stage(TILE + SCH * cur + pos, R);
+            L.tq()[pos] = qv;
+            if (C::ELEC) L.teq[pos] = eqv;
             L.atom[SCH * cur + pos] = o2 + a;
           }
           cur_cp = cur_cp || (__ballot(mine && (info & 1)) != 0);
@@ -475,7 +594,8 @@ __global__ __launch_bounds__(256, (stream_waves_per_simd<MODE, OCC>())) void sco
     }
     // ---- row end: test the partial chunk, evaluate the rest, flush
     if (fill > 0) test_chunk();
-    drain(true);
+    if (n_lj > 0) drain();
+    if (n_lk > 0) drain_lk();
     for (int r = 0; r < 3; ++r)
       if (cnt[r] > 0) {
         flush_chunk<Real, MODE>(L, A, r, cnt[r], lane);
@@ -483,9 +603,9 @@ __global__ __launch_bounds__(256, (stream_waves_per_simd<MODE, OCC>())) void sco
       }
     flush_g1<Real, MODE>(L, A, n1, o1, lane);
     if (!C::NOE) {
-      const double ea = wave_sum(e_atr.value());
-      const double er = wave_sum(e_rep.value());
-      const double el = wave_sum(e_lk.value());
+      const double ea = wave_sum(en.atr.value());
+      const double er = wave_sum(en.rep.value());
+      const double el = wave_sum(en.lk.value());
       if (lane == 0 && C::DET) {
         auto* e = (unsigned long long*)A.energies64;
         atomicAdd(&e[p], det_energy_enc(ea));
@@ -495,6 +615,10 @@ __global__ __launch_bounds__(256, (stream_waves_per_simd<MODE, OCC>())) void sco
         unsafeAtomicAdd(&A.energies64[p], ea);
         unsafeAtomicAdd(&A.energies64[s.P + p], er);
         unsafeAtomicAdd(&A.energies64[2 * s.P + p], el);
+      }
+      if (C::ELEC) {
+        const double ee = wave_sum(en.el.value());
+        if (lane == 0) unsafeAtomicAdd(&A.energies64[3 * s.P + p], ee);
       }
     }
     wave_sync();
