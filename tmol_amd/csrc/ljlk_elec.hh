@@ -51,6 +51,7 @@ struct ElecArgs {
   const uint16_t* intra_pairs;  // [T, INTRA_MAX]
   ElecConst<Real> k;
   uint32_t* row_cursor;
+  int part_shift;        // a row is 2^part_shift queue units (parts of its items)
   const Real* weights;   // [P] or [P, B, B] / [G, row_cap] (block pair)
   double* energies64;    // [P]
   Real* energies_bp;     // [P, B, B] / [G, row_cap]
@@ -241,7 +242,8 @@ elec_rows_kernel(ElecArgs<Real> A) {
   const ElecConst<Real> k = A.k;
   const StackView& s = A.s;
   const BTView& bt = A.bt;
-  RowQueue queue(A.row_cursor, s.G);
+  const int shift = A.part_shift;
+  RowQueue queue(A.row_cursor, int64_t(s.G) << shift);
   const Real cull_pad = k.hpe + Real(1e-3);
   constexpr bool CEN = MODE & M_CENSUS;
   ElecCensus cen;
@@ -251,9 +253,14 @@ elec_rows_kernel(ElecArgs<Real> A) {
     for (int i = lane; i < 3 * RSLOTS; i += WAVE) (&L.grad[0][0])[i] = 0;
   wave_sync();
 
-  for (int64_t row = queue.next(); row >= 0; row = queue.next()) {
-    const int n_items = uni((int)min<int64_t>(A.w.row_count[row], A.w.row_cap));
-    if (n_items == 0) continue;
+  for (int64_t unit = queue.next(); unit >= 0; unit = queue.next()) {
+    const int64_t row = unit >> shift;
+    const int n_row = uni((int)min<int64_t>(A.w.row_count[row], A.w.row_cap));
+    // this part's items [k_lo, n_items) of the row
+    const int64_t part = unit - (row << shift);
+    const int k_lo = int((n_row * part) >> shift);
+    const int n_items = int((n_row * (part + 1)) >> shift);
+    if (n_items == k_lo) continue;
     const int g1 = (int)row;
     const int t1 = uni(s.block_type[g1]);
     const int n1 = uni(bt.n_atoms[t1]);
@@ -300,7 +307,7 @@ elec_rows_kernel(ElecArgs<Real> A) {
         used0 = false;
     };
 
-    for (int c0 = 0; c0 < n_items; c0 += WAVE) {
+    for (int c0 = k_lo; c0 < n_items; c0 += WAVE) {
       const int n_chunk = min(WAVE, n_items - c0);
       // d_pk: n_atoms | n_conn << 8 | is_ligand << 12 | min block separation << 16
       int d_g2 = g1, d_t2 = t1, d_o2 = 0, d_pk = 0;

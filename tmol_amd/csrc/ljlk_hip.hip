@@ -168,71 +168,72 @@ static int resident_workgroups(K kernel) {
   return n;
 }
 
-// n_wg <= 0: one workgroup per resident slot (the row queue balances the load)
-template <typename Real, int MODE>
-static void launch_score(const ScoreArgs<Real>& a, bool general, int n_wg, hipStream_t stream) {
+// A row is one wave's serial work (about 25-45 us for a protein's 18 items), so
+// a batch with fewer rows than resident waves is bound by one row's latency and
+// leaves the chip idle: its rows are split into 2^shift parts, the most that
+// still gives every resident wave at most one part (each part stages g1 again
+// and ends in partial batches), up to 16, about one neighbor block each.
+static int row_part_shift(int64_t n_rows, int64_t resident_waves) {
+  int s = 0;
+  while (s < 4 && (n_rows << (s + 1)) <= resident_waves) ++s;
+  return s;
+}
+
+// a persistent row kernel over `a`'s rows: n_wg <= 0 launches one workgroup per
+// resident slot, or fewer where the queue holds fewer units (it balances the
+// load)
+template <typename K, typename Args>
+static void launch_persistent(K k, Args a, int n_wg, hipStream_t stream) {
   hipLaunchKernelGGL(fill_kernel<uint32_t>, dim3(2), dim3(256), 0, stream, a.row_cursor,
                      8 * QSTRIDE, 0u);
+  const int resident = resident_workgroups(k);
+  a.part_shift = row_part_shift(a.s.G, int64_t(resident) * WAVES_PER_WG);
+  const int64_t units = int64_t(a.s.G) << a.part_shift;
+  if (n_wg <= 0)
+    n_wg = (int)std::min<int64_t>(resident, (units + WAVES_PER_WG - 1) / WAVES_PER_WG);
+  hipLaunchKernelGGL(k, dim3(n_wg), dim3(256), 0, stream, a);
+}
+
+template <typename Real, int MODE>
+static void launch_score(const ScoreArgs<Real>& a, bool general, int n_wg, hipStream_t stream) {
   if (general) {
+    hipLaunchKernelGGL(fill_kernel<uint32_t>, dim3(2), dim3(256), 0, stream, a.row_cursor,
+                       8 * QSTRIDE, 0u);
     auto k = score_general_kernel<Real, MODE>;
     if (n_wg <= 0) n_wg = resident_workgroups(k);
     hipLaunchKernelGGL(k, dim3(n_wg), dim3(256), 0, stream, a);
   } else {
-    auto k = score_rows_kernel<Real, MODE>;
-    if (n_wg <= 0) n_wg = resident_workgroups(k);
-    hipLaunchKernelGGL(k, dim3(n_wg), dim3(256), 0, stream, a);
+    launch_persistent(score_rows_kernel<Real, MODE>, a, n_wg, stream);
   }
-}
-
-// rows kernel only (modes the general kernel does not implement)
-template <typename Real, int MODE>
-static void launch_rows(const ScoreArgs<Real>& a, int n_wg, hipStream_t stream) {
-  hipLaunchKernelGGL(fill_kernel<uint32_t>, dim3(2), dim3(256), 0, stream, a.row_cursor,
-                     8 * QSTRIDE, 0u);
-  auto k = score_rows_kernel<Real, MODE>;
-  if (n_wg <= 0) n_wg = resident_workgroups(k);
-  hipLaunchKernelGGL(k, dim3(n_wg), dim3(256), 0, stream, a);
 }
 
 // the rows kernel compiled for `occ` waves per SIMD (0: the mode's default;
 // float only -- other dtypes take the default)
 template <typename Real, int MODE>
 static void launch_rows_occ(const ScoreArgs<Real>& a, int occ, int n_wg, hipStream_t stream) {
-  hipLaunchKernelGGL(fill_kernel<uint32_t>, dim3(2), dim3(256), 0, stream, a.row_cursor,
-                     8 * QSTRIDE, 0u);
-  auto go = [&](auto k) {
-    if (n_wg <= 0) n_wg = resident_workgroups(k);
-    hipLaunchKernelGGL(k, dim3(n_wg), dim3(256), 0, stream, a);
-  };
   if constexpr (std::is_same<Real, float>::value) {
     switch (occ) {
-      case 3: go(score_rows_kernel<Real, MODE, 3>); return;
-      case 4: go(score_rows_kernel<Real, MODE, 4>); return;
-      case 5: go(score_rows_kernel<Real, MODE, 5>); return;
+      case 3: launch_persistent(score_rows_kernel<Real, MODE, 3>, a, n_wg, stream); return;
+      case 4: launch_persistent(score_rows_kernel<Real, MODE, 4>, a, n_wg, stream); return;
+      case 5: launch_persistent(score_rows_kernel<Real, MODE, 5>, a, n_wg, stream); return;
       default: break;
     }
   }
-  go(score_rows_kernel<Real, MODE>);
+  launch_persistent(score_rows_kernel<Real, MODE>, a, n_wg, stream);
 }
 
 // the stream kernel (whole-pose energies / WGRAD, blocks of <= 32 atoms),
 // compiled for `occ` waves per SIMD (float: 3, 4 or 5; 0 = 4)
 template <typename Real, int MODE>
 static void launch_stream(const ScoreArgs<Real>& a, int occ, int n_wg, hipStream_t stream) {
-  hipLaunchKernelGGL(fill_kernel<uint32_t>, dim3(2), dim3(256), 0, stream, a.row_cursor,
-                     8 * QSTRIDE, 0u);
-  auto go = [&](auto k) {
-    if (n_wg <= 0) n_wg = resident_workgroups(k);
-    hipLaunchKernelGGL(k, dim3(n_wg), dim3(256), 0, stream, a);
-  };
   if constexpr (std::is_same<Real, float>::value && !(MODE & M_ELEC)) {
     switch (occ) {
-      case 3: go(score_stream_kernel<Real, MODE, 3>); return;
-      case 5: go(score_stream_kernel<Real, MODE, 5>); return;
+      case 3: launch_persistent(score_stream_kernel<Real, MODE, 3>, a, n_wg, stream); return;
+      case 5: launch_persistent(score_stream_kernel<Real, MODE, 5>, a, n_wg, stream); return;
       default: break;
     }
   }
-  go(score_stream_kernel<Real, MODE>);
+  launch_persistent(score_stream_kernel<Real, MODE>, a, n_wg, stream);
 }
 
 // ek != nullptr: elec is scored in the same pass (M_ELEC; tables prepared in
@@ -302,9 +303,9 @@ static int run_score(const tmol_ljlk_stack* st, const tmol_ljlk_block_types* btp
           launch_stream<Real, M_WGRAD | M_NOE | M_DET>(a, occ, n_wg, stream);
       } else {
         switch (mode) {
-          case M_DVDX: launch_rows<Real, M_DVDX | M_DET>(a, n_wg, stream); break;
-          case M_WGRAD: launch_rows<Real, M_WGRAD | M_DET>(a, n_wg, stream); break;
-          case M_WGRAD | M_NOE: launch_rows<Real, M_WGRAD | M_NOE | M_DET>(a, n_wg, stream); break;
+          case M_DVDX: launch_rows_occ<Real, M_DVDX | M_DET>(a, 0, n_wg, stream); break;
+          case M_WGRAD: launch_rows_occ<Real, M_WGRAD | M_DET>(a, 0, n_wg, stream); break;
+          case M_WGRAD | M_NOE: launch_rows_occ<Real, M_WGRAD | M_NOE | M_DET>(a, 0, n_wg, stream); break;
           default: return TMOL_LJLK_ENOTSUP;
         }
       }
@@ -694,11 +695,7 @@ static int run_elec_neighbors(const tmol_ljlk_stack* st, const tmol_ljlk_block_t
 
 template <typename Real, int MODE>
 static void launch_elec(const ElecArgs<Real>& a, int n_wg, hipStream_t stream) {
-  hipLaunchKernelGGL(fill_kernel<uint32_t>, dim3(2), dim3(256), 0, stream, a.row_cursor,
-                     8 * QSTRIDE, 0u);
-  auto k = elec_rows_kernel<Real, MODE>;
-  if (n_wg <= 0) n_wg = resident_workgroups(k);
-  hipLaunchKernelGGL(k, dim3(n_wg), dim3(256), 0, stream, a);
+  launch_persistent(elec_rows_kernel<Real, MODE>, a, n_wg, stream);
 }
 
 template <typename Real>
