@@ -331,6 +331,7 @@ struct HbArgs {
   Real* energies_bp;             // block pairs
   Real* dxyz;                    // [NA, 3]
   unsigned long long* census;    // [3]
+  int part_shift;                // rows are not split into parts: 0
 };
 
 // a work-list item of the row: the other block, its type, first atom,

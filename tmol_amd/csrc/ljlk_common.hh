@@ -61,6 +61,18 @@ __device__ __forceinline__ int lanes_below(uint64_t mask) {
                                    __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
 }
 
+// four Reals moved as one 16-byte (float) or 32-byte (double) access
+template <typename Real>
+struct V4;
+template <>
+struct V4<float> {
+  using T = float4;
+};
+template <>
+struct V4<double> {
+  using T = double4;
+};
+
 // ------------------------------------------------------------------ workspace
 
 struct WsLayout {
@@ -216,6 +228,40 @@ __device__ __forceinline__ const int32_t* bonded_row(const StackView& s, int lo,
     if (g > hi) break;
   }
   return nullptr;
+}
+
+// Minimum bond separation of blocks g1 < g2 and, where it is at most 4, the
+// connection separations cs[c1] (byte c2; 6 where no path is shorter): one
+// search of the bonded table for both.  cs is 6 everywhere otherwise.
+__device__ __forceinline__ int pair_separations(const StackView& s, int g1, int g2, int nc1,
+                                                int nc2, uint32_t cs[MAX_CONN]) {
+#pragma unroll
+  for (int c1 = 0; c1 < MAX_CONN; ++c1) cs[c1] = 0x06060606u;
+  if (s.layout == TMOL_LJLK_PADDED) {
+    const int64_t cell = int64_t(g1) * s.B + (g2 - (g2 / s.B) * s.B);
+    const int ms = s.min_bondsep[cell];
+    if (ms <= 4) {
+#pragma unroll
+      for (int c1 = 0; c1 < MAX_CONN; ++c1) {
+        if (c1 >= nc1) break;
+        const int32_t* v = s.inter_block_bondsep + (cell * s.C + c1) * s.C;
+        uint32_t r = 0x06060606u;
+        for (int c2 = 0; c2 < nc2; ++c2)
+          r = (r & ~(255u << (8 * c2))) | ((uint32_t)min(v[c2], 6) << (8 * c2));
+        cs[c1] = r;
+      }
+    }
+    return ms;
+  }
+  const int32_t* e = bonded_row(s, g1, g2);
+  if (!e) return 6;
+  const int ms = e[1];
+  if (ms <= 4) {
+#pragma unroll
+    for (int c1 = 0; c1 < MAX_CONN; ++c1)
+      if (c1 < nc1) cs[c1] = (uint32_t)e[4 + c1];
+  }
+  return ms;
 }
 
 // bond separation between connection c1 of g1 and c2 of g2 (g1 != g2)
@@ -431,6 +477,13 @@ struct RowQueue {
       --left;
     }
     return -1;
+  }
+  // the next rows of one grab, first and count (wave-uniform); -1 at the end
+  __device__ int64_t next_range(int& count) {
+    const int64_t first = next();
+    count = first < 0 ? 0 : 1 + int(end - cur);
+    cur = end;
+    return first;
   }
 };
 

@@ -61,16 +61,12 @@ struct ElecArgs {
   unsigned long long* census;  // [16] with M_CENSUS
 };
 
-// Per block type: packed inter-block path distances and the intra-block
-// table (one wave per type, ballot-compacted in (a1, a2) order).
+// Block type t's packed inter-block path distances and intra-block table (by
+// one wave, ballot-compacted in (a1, a2) order).
 template <typename Real>
-__global__ __launch_bounds__(64) void elec_prepare_kernel(BTView bt, const Real* charge,
-                                                          const int32_t* inter_rpd,
-                                                          const int32_t* intra_rpd,
-                                                          uint32_t* epd, int32_t* count,
-                                                          uint16_t* pairs) {
-  const int t = blockIdx.x;
-  const int lane = lane_id();
+__device__ __forceinline__ void elec_prepare(const BTView& bt, int t, int lane, const Real* charge,
+                                             const int32_t* inter_rpd, const int32_t* intra_rpd,
+                                             uint32_t* epd, int32_t* count, uint16_t* pairs) {
   const int n = bt.n_atoms[t];
   const int nc = bt.n_conn[t];
   const int64_t A = bt.Amax;

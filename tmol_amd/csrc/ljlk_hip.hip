@@ -30,6 +30,7 @@
 #include "ljlk_elec_rotamer.hh"
 #include "ljlk_topology.hh"
 #include "ljlk_elec.hh"
+#include "ljlk_setup.hh"
 #include "lbfgs.hh"
 #include "lkball.hh"
 #include "hbond.hh"
@@ -75,41 +76,81 @@ static void fill(Real* p, int64_t n, hipStream_t stream, Real v = Real(0)) {
   hipLaunchKernelGGL(fill_kernel<Real>, dim3(grid_for(n)), dim3(256), 0, stream, p, n, v);
 }
 
+static void launch_clear(const ClearList& c, hipStream_t stream) {
+  int64_t n = 0;
+  for (int k = 0; k < c.used; ++k) n = std::max(n, c.n[k]);
+  if (n > 0)
+    hipLaunchKernelGGL(clear_kernel, dim3(grid_for(n)), dim3(256), 0, stream, c);
+}
+
+template <typename Real>
+static void launch_setup(SetupArgs<Real>& a, hipStream_t stream) {
+  a.type_jobs = a.records || a.epd ? a.bt.T : 0;
+  int64_t n = a.s.G;
+  for (int k = 0; k < a.clear.used; ++k) n = std::max(n, a.clear.n[k]);
+  hipLaunchKernelGGL(setup_kernel<Real>, dim3(a.type_jobs + grid_for(n)), dim3(256), 0, stream, a);
+}
+
+template <typename Real>
+static void setup_ljlk_tables(SetupArgs<Real>& a, const tmol_ljlk_block_types* btp, void* records,
+                              void* conn_pd, void* intra) {
+  a.type_params = (const Real*)btp->type_params;
+  a.n_atom_types = btp->n_atom_types;
+  a.records = (Real*)records;
+  a.conn_pd = (uint8_t*)conn_pd;
+  a.intra_count = (int32_t*)intra;
+  a.intra_pairs = (uint16_t*)((char*)intra + 4 * int64_t(btp->n_block_types));
+}
+
+template <typename Real>
+static void setup_elec_tables(SetupArgs<Real>& a, const tmol_ljlk_block_types* btp,
+                              const tmol_elec_tables* e, void* epd, void* intra) {
+  a.charge = (const Real*)e->partial_charge;
+  a.inter_rpd = e->inter_repr_path_distance;
+  a.intra_rpd = e->intra_repr_path_distance;
+  a.epd = (uint32_t*)epd;
+  a.e_intra_count = (int32_t*)intra;
+  a.e_intra_pairs = (uint16_t*)((char*)intra + 4 * int64_t(btp->n_block_types));
+}
+
+// Setup (the tables already named in `a`, spheres, clears) and the neighbor
+// rows; FULL: rows list both triangles (lk_ball), otherwise g2 >= g1.
+template <typename Real, bool FULL = false>
+static int launch_neighbors(SetupArgs<Real>& a, const tmol_ljlk_stack* st,
+                            const tmol_ljlk_block_types* btp, const void* coords, double max_dis,
+                            const int32_t* tiles, int64_t n_tiles, void* ws, int64_t row_cap,
+                            int32_t* dense, hipStream_t stream, const WsLayout& Lw) {
+  a.s = make_stack_view(st, btp->max_n_conn);
+  a.bt = make_bt_view(btp);
+  a.coords = (const Real*)coords;
+  char* w = (char*)ws;
+  a.spheres = (Real*)(w + Lw.spheres);
+  uint32_t* counters = (uint32_t*)(w + Lw.counters);
+  uint32_t* row_count = (uint32_t*)(w + Lw.row_count);
+  a.clear.add(counters, 64);
+  a.clear.add(row_count, 4 * int64_t(a.s.G));
+  if (dense) a.clear.add(dense, 4 * int64_t(a.s.P) * a.s.B * a.s.B);
+  launch_setup(a, stream);
+  if (n_tiles > 0) {
+    auto k = neighbor_rows_kernel<Real, FULL>;
+    hipLaunchKernelGGL(k, dim3((unsigned)n_tiles), dim3(256), 0, stream, a.s, (const int4*)tiles,
+                       n_tiles, (const Real*)a.spheres, (Real)max_dis, row_count,
+                       (int32_t*)(w + Lw.row_items), row_cap, counters, dense,
+                       st->pose_block_start);
+  }
+  return check(hipGetLastError());
+}
+
 template <typename Real>
 static int run_neighbors(const tmol_ljlk_stack* st, const tmol_ljlk_block_types* btp,
                          const void* coords, double max_dis, const int32_t* tiles,
                          int64_t n_tiles, void* ws, int64_t row_cap, int32_t* dense,
                          hipStream_t stream, const WsLayout& Lw) {
-  StackView s = make_stack_view(st, btp->max_n_conn);
-  BTView bt = make_bt_view(btp);
+  SetupArgs<Real> a{};
   char* w = (char*)ws;
-  uint32_t* counters = (uint32_t*)(w + Lw.counters);
-  Real* spheres = (Real*)(w + Lw.spheres);
-  Real* records = (Real*)(w + Lw.records);
-  uint8_t* conn_pd = (uint8_t*)(w + Lw.conn_pd);
-  uint32_t* row_count = (uint32_t*)(w + Lw.row_count);
-  int32_t* row_items = (int32_t*)(w + Lw.row_items);
-  hipLaunchKernelGGL(fill_kernel<uint32_t>, dim3(1), dim3(64), 0, stream, counters, 16,
-                     (uint32_t)0);
-  hipLaunchKernelGGL(fill_kernel<uint32_t>, dim3(grid_for(s.G)), dim3(256), 0, stream,
-                     row_count, int64_t(s.G), (uint32_t)0);
-  int nrec = bt.T * bt.Amax;
-  hipLaunchKernelGGL(prepare_records_kernel<Real>, dim3(grid_for(nrec)), dim3(256), 0, stream, bt,
-                     (const Real*)btp->type_params, btp->n_atom_types, records, conn_pd);
-  hipLaunchKernelGGL(prepare_intra_kernel, dim3(bt.T), dim3(64), 0, stream, bt,
-                     (int32_t*)(w + Lw.intra),
-                     (uint16_t*)(w + Lw.intra + 4 * int64_t(bt.T)));
-  hipLaunchKernelGGL(spheres_kernel<Real>, dim3(grid_for(s.G)), dim3(256), 0, stream, s, bt,
-                     (const Real*)coords, spheres);
-  if (dense) {
-    int64_t n = int64_t(s.P) * s.B * s.B;
-    hipLaunchKernelGGL(fill_kernel<int32_t>, dim3(grid_for(n)), dim3(256), 0, stream, dense, n, 0);
-  }
-  if (n_tiles > 0)
-    hipLaunchKernelGGL(neighbor_rows_kernel<Real>, dim3((unsigned)n_tiles), dim3(256), 0, stream, s,
-                       (const int4*)tiles, n_tiles, spheres, (Real)max_dis, row_count, row_items,
-                       row_cap, counters, dense);
-  return check(hipGetLastError());
+  setup_ljlk_tables(a, btp, w + Lw.records, w + Lw.conn_pd, w + Lw.intra);
+  return launch_neighbors(a, st, btp, coords, max_dis, tiles, n_tiles, ws, row_cap, dense, stream,
+                          Lw);
 }
 
 template <typename Real>
@@ -168,24 +209,25 @@ static int resident_workgroups(K kernel) {
   return n;
 }
 
-// A row is one wave's serial work (about 25-45 us for a protein's 18 items), so
-// a batch with fewer rows than resident waves is bound by one row's latency and
-// leaves the chip idle: its rows are split into 2^shift parts, the most that
-// still gives every resident wave at most one part (each part stages g1 again
-// and ends in partial batches), up to 16, about one neighbor block each.
+// A row is one wave's serial work, so a batch with fewer rows than resident
+// waves is bound by one row's latency and leaves the chip idle: its rows are
+// split into 2^shift parts, the most that still gives every resident wave at
+// most one part (each part stages g1 again and ends in partial batches), up to
+// 16, about one neighbor block each.  One 76-residue protein, per-term
+// derivatives: LJ+LK 150 -> 42 us, elec 121 -> 24 us; block-pair gradients of
+// 7 poses of 61-181 residues 265 -> 96 us.  At one part per wave or more
+// splitting only repeats the staging: 64 poses of 150-600 residues keep shift 0.
 static int row_part_shift(int64_t n_rows, int64_t resident_waves) {
   int s = 0;
   while (s < 4 && (n_rows << (s + 1)) <= resident_waves) ++s;
   return s;
 }
 
-// a persistent row kernel over `a`'s rows: n_wg <= 0 launches one workgroup per
-// resident slot, or fewer where the queue holds fewer units (it balances the
-// load)
+// a persistent row kernel over `a`'s rows (cursors cleared): n_wg <= 0 launches
+// one workgroup per resident slot, or fewer where the queue holds fewer units
+// (it balances the load)
 template <typename K, typename Args>
 static void launch_persistent(K k, Args a, int n_wg, hipStream_t stream) {
-  hipLaunchKernelGGL(fill_kernel<uint32_t>, dim3(2), dim3(256), 0, stream, a.row_cursor,
-                     8 * QSTRIDE, 0u);
   const int resident = resident_workgroups(k);
   a.part_shift = row_part_shift(a.s.G, int64_t(resident) * WAVES_PER_WG);
   const int64_t units = int64_t(a.s.G) << a.part_shift;
@@ -197,8 +239,6 @@ static void launch_persistent(K k, Args a, int n_wg, hipStream_t stream) {
 template <typename Real, int MODE>
 static void launch_score(const ScoreArgs<Real>& a, bool general, int n_wg, hipStream_t stream) {
   if (general) {
-    hipLaunchKernelGGL(fill_kernel<uint32_t>, dim3(2), dim3(256), 0, stream, a.row_cursor,
-                       8 * QSTRIDE, 0u);
     auto k = score_general_kernel<Real, MODE>;
     if (n_wg <= 0) n_wg = resident_workgroups(k);
     hipLaunchKernelGGL(k, dim3(n_wg), dim3(256), 0, stream, a);
@@ -264,26 +304,28 @@ static int run_score(const tmol_ljlk_stack* st, const tmol_ljlk_block_types* btp
   const bool general = (flags & TMOL_LJLK_GENERAL_KERNEL) || btp->max_n_atoms > TILE;
   const int P = st->n_poses;
   const int64_t NA3 = st->n_atoms_total * 3;
+  ClearList c{};
+  c.add(a.row_cursor, 4 * 8 * QSTRIDE);
   if (det) {
     // float32 whole-pose DVDX / WGRAD (stream or row kernel; not the general one)
     if (!std::is_same<Real, float>::value || general || bp || ek) return TMOL_LJLK_ENOTSUP;
     if (!(flags & (TMOL_LJLK_DVDX | TMOL_LJLK_WGRAD))) return TMOL_LJLK_ENOTSUP;
     const int planes = (flags & TMOL_LJLK_DVDX) ? 3 : 1;
     a.fixed = (unsigned long long*)((char*)ws + Lw.fixed);
-    fill<unsigned long long>(a.fixed, planes * NA3, stream);
+    c.add(a.fixed, 8 * planes * NA3);
   }
   if (!noe) {
     if (bp)
-      fill<Real>((Real*)energies,
-                 3 * (st->layout == TMOL_LJLK_PADDED
-                          ? int64_t(P) * st->max_n_blocks * st->max_n_blocks
-                          : int64_t(st->n_blocks_total) * row_cap),
-                 stream);
+      c.add(energies, int64_t(sizeof(Real)) * 3 *
+                          (st->layout == TMOL_LJLK_PADDED
+                               ? int64_t(P) * st->max_n_blocks * st->max_n_blocks
+                               : int64_t(st->n_blocks_total) * row_cap));
     else
-      fill<double>(a.energies64, int64_t(n_terms) * P, stream);
+      c.add(a.energies64, 8 * int64_t(n_terms) * P);
   }
-  if ((flags & TMOL_LJLK_DVDX) && !acc && !det) fill<Real>((Real*)dvdx, 3 * NA3, stream);
-  if ((flags & TMOL_LJLK_WGRAD) && !acc && !det) fill<Real>((Real*)grad, NA3, stream);
+  if ((flags & TMOL_LJLK_DVDX) && !acc && !det) c.add(dvdx, int64_t(sizeof(Real)) * 3 * NA3);
+  if ((flags & TMOL_LJLK_WGRAD) && !acc && !det) c.add(grad, int64_t(sizeof(Real)) * NA3);
+  launch_clear(c, stream);
   const int n_wg = n_wave_groups;
   int mode = flags & (TMOL_LJLK_DVDX | TMOL_LJLK_WGRAD | TMOL_LJLK_BLOCK_PAIR | TMOL_LJLK_NO_ENERGY);
   // launch variants (autotuner): waves per SIMD and rows per queue grab
@@ -477,26 +519,21 @@ static int run_rot_neighbors(const tmol_ljlk_rotamer_set* r, const tmol_ljlk_blo
   Real* rsph = (Real*)(w + Lw.rot_spheres);
   Real* bsph = (Real*)(w + Lw.block_spheres);
   const int64_t G = int64_t(v.P) * v.B;
-  const int nrec = bt.T * bt.Amax;
-  if (elec)
-    hipLaunchKernelGGL(elec_prepare_kernel<Real>, dim3(bt.T), dim3(64), 0, stream, bt,
-                       (const Real*)elec->partial_charge, elec->inter_repr_path_distance,
-                       elec->intra_repr_path_distance, (uint32_t*)(w + Lw.e_pd),
-                       (int32_t*)(w + Lw.e_intra),
-                       (uint16_t*)(w + Lw.e_intra + 4 * int64_t(bt.T)));
-  else
-    hipLaunchKernelGGL(prepare_records_kernel<Real>, dim3(grid_for(nrec)), dim3(256), 0, stream,
-                       bt, (const Real*)btp->type_params, btp->n_atom_types,
-                       (Real*)(w + Lw.records), (uint8_t*)(w + Lw.conn_pd));
-  if (v.R > 0) {
-    // rotamer spheres: the block-sphere pass with rotamers as blocks
-    StackView s{};
-    s.G = v.R;
-    s.block_atom_offset = v.rot_coord_offset;
-    s.block_type = v.block_type_for_rot;
-    hipLaunchKernelGGL(spheres_kernel<Real>, dim3((unsigned)((v.R + 255) / 256)), dim3(256), 0,
-                       stream, s, bt, (const Real*)coords, rsph);
+  // rotamer spheres: the block-sphere pass with rotamers as blocks
+  SetupArgs<Real> a{};
+  a.s.G = v.R;
+  a.s.block_atom_offset = v.rot_coord_offset;
+  a.s.block_type = v.block_type_for_rot;
+  a.bt = bt;
+  a.coords = (const Real*)coords;
+  a.spheres = rsph;
+  if (elec) {
+    setup_elec_tables(a, btp, elec, w + Lw.e_pd, w + Lw.e_intra);
+  } else {
+    setup_ljlk_tables(a, btp, w + Lw.records, w + Lw.conn_pd, w);
+    a.intra_count = nullptr;  // self pairs take the block type's path distances
   }
+  launch_setup(a, stream);
   hipLaunchKernelGGL(rot_block_spheres_kernel<Real>, dim3((unsigned)((G + 255) / 256)),
                      dim3(256), 0, stream, v, (const Real*)rsph, bsph);
   int64_t* rp = (int64_t*)(w + Lw.row_pairs);
@@ -665,32 +702,10 @@ static int run_elec_neighbors(const tmol_ljlk_stack* st, const tmol_ljlk_block_t
                               const tmol_elec_tables* e, const void* coords, double max_dis,
                               const int32_t* tiles, int64_t n_tiles, void* ws, int64_t row_cap,
                               int32_t* dense, hipStream_t stream, const WsLayout& Lw) {
-  StackView s = make_stack_view(st, btp->max_n_conn);
-  BTView bt = make_bt_view(btp);
-  char* w = (char*)ws;
-  uint32_t* counters = (uint32_t*)(w + Lw.counters);
-  Real* spheres = (Real*)(w + Lw.spheres);
-  uint32_t* row_count = (uint32_t*)(w + Lw.row_count);
-  int32_t* row_items = (int32_t*)(w + Lw.row_items);
-  hipLaunchKernelGGL(fill_kernel<uint32_t>, dim3(1), dim3(64), 0, stream, counters, 16,
-                     (uint32_t)0);
-  hipLaunchKernelGGL(fill_kernel<uint32_t>, dim3(grid_for(s.G)), dim3(256), 0, stream,
-                     row_count, int64_t(s.G), (uint32_t)0);
-  hipLaunchKernelGGL(elec_prepare_kernel<Real>, dim3(bt.T), dim3(64), 0, stream, bt,
-                     (const Real*)e->partial_charge, e->inter_repr_path_distance,
-                     e->intra_repr_path_distance, (uint32_t*)(w + Lw.conn_pd),
-                     (int32_t*)(w + Lw.intra), (uint16_t*)(w + Lw.intra + 4 * int64_t(bt.T)));
-  hipLaunchKernelGGL(spheres_kernel<Real>, dim3(grid_for(s.G)), dim3(256), 0, stream, s, bt,
-                     (const Real*)coords, spheres);
-  if (dense) {
-    int64_t n = int64_t(s.P) * s.B * s.B;
-    hipLaunchKernelGGL(fill_kernel<int32_t>, dim3(grid_for(n)), dim3(256), 0, stream, dense, n, 0);
-  }
-  if (n_tiles > 0)
-    hipLaunchKernelGGL(neighbor_rows_kernel<Real>, dim3((unsigned)n_tiles), dim3(256), 0, stream, s,
-                       (const int4*)tiles, n_tiles, spheres, (Real)max_dis, row_count, row_items,
-                       row_cap, counters, dense);
-  return check(hipGetLastError());
+  SetupArgs<Real> a{};
+  setup_elec_tables(a, btp, e, (char*)ws + Lw.conn_pd, (char*)ws + Lw.intra);
+  return launch_neighbors(a, st, btp, coords, max_dis, tiles, n_tiles, ws, row_cap, dense, stream,
+                          Lw);
 }
 
 template <typename Real, int MODE>
@@ -727,8 +742,10 @@ static int run_elec_score(const tmol_ljlk_stack* st, const tmol_ljlk_block_types
   a.n_atoms = st->n_atoms_total;
   a.census = census;
   if (census) {
-    hipLaunchKernelGGL(fill_kernel<unsigned long long>, dim3(1), dim3(64), 0, stream, census, 16,
-                       0ull);
+    ClearList c{};
+    c.add(a.row_cursor, 4 * 8 * QSTRIDE);
+    c.add(census, 8 * 16);
+    launch_clear(c, stream);
     launch_elec<Real, M_CENSUS>(a, n_wg, stream);
     return check(hipGetLastError());
   }
@@ -737,18 +754,20 @@ static int run_elec_score(const tmol_ljlk_stack* st, const tmol_ljlk_block_types
   const bool acc = flags & TMOL_LJLK_ACCUMULATE;
   const int P = st->n_poses;
   const int64_t NA3 = st->n_atoms_total * 3;
+  ClearList c{};
+  c.add(a.row_cursor, 4 * 8 * QSTRIDE);
   if (!noe) {
     if (bp)
-      fill<Real>((Real*)energies,
-                 st->layout == TMOL_LJLK_PADDED
-                     ? int64_t(P) * st->max_n_blocks * st->max_n_blocks
-                     : int64_t(st->n_blocks_total) * row_cap,
-                 stream);
+      c.add(energies, int64_t(sizeof(Real)) *
+                          (st->layout == TMOL_LJLK_PADDED
+                               ? int64_t(P) * st->max_n_blocks * st->max_n_blocks
+                               : int64_t(st->n_blocks_total) * row_cap));
     else
-      fill<double>(a.energies64, P, stream);
+      c.add(a.energies64, 8 * int64_t(P));
   }
-  if ((flags & TMOL_LJLK_DVDX) && !acc) fill<Real>((Real*)dvdx, NA3, stream);
-  if ((flags & TMOL_LJLK_WGRAD) && !acc) fill<Real>((Real*)grad, NA3, stream);
+  if ((flags & TMOL_LJLK_DVDX) && !acc) c.add(dvdx, int64_t(sizeof(Real)) * NA3);
+  if ((flags & TMOL_LJLK_WGRAD) && !acc) c.add(grad, int64_t(sizeof(Real)) * NA3);
+  launch_clear(c, stream);
   const int mode = flags & (TMOL_LJLK_DVDX | TMOL_LJLK_WGRAD | TMOL_LJLK_BLOCK_PAIR |
                             TMOL_LJLK_NO_ENERGY);
   switch (mode) {
@@ -833,36 +852,13 @@ static int run_lkb_neighbors(const tmol_ljlk_stack* st, const tmol_ljlk_block_ty
                              const void* coords, double max_dis, const int32_t* tiles,
                              int64_t n_tiles, void* ws, int64_t row_cap, int32_t* dense,
                              hipStream_t stream, const WsLayout& Lw) {
-  StackView s = make_stack_view(st, btp->max_n_conn);
-  BTView bt = make_bt_view(btp);
-  char* w = (char*)ws;
-  uint32_t* counters = (uint32_t*)(w + Lw.counters);
-  Real* spheres = (Real*)(w + Lw.spheres);
-  uint32_t* row_count = (uint32_t*)(w + Lw.row_count);
-  int32_t* row_items = (int32_t*)(w + Lw.row_items);
-  hipLaunchKernelGGL(fill_kernel<uint32_t>, dim3(1), dim3(64), 0, stream, counters, 16,
-                     (uint32_t)0);
-  hipLaunchKernelGGL(fill_kernel<uint32_t>, dim3(grid_for(s.G)), dim3(256), 0, stream,
-                     row_count, int64_t(s.G), (uint32_t)0);
-  hipLaunchKernelGGL(spheres_kernel<Real>, dim3(grid_for(s.G)), dim3(256), 0, stream, s, bt,
-                     (const Real*)coords, spheres);
-  if (dense) {
-    int64_t n = int64_t(s.P) * s.B * s.B;
-    hipLaunchKernelGGL(fill_kernel<int32_t>, dim3(grid_for(n)), dim3(256), 0, stream, dense, n, 0);
-  }
-  if (n_tiles > 0) {
-    auto k = neighbor_rows_kernel<Real, FULL>;
-    hipLaunchKernelGGL(k, dim3((unsigned)n_tiles), dim3(256), 0, stream, s, (const int4*)tiles,
-                       n_tiles, spheres, (Real)max_dis, row_count, row_items, row_cap, counters,
-                       dense, st->pose_block_start);
-  }
-  return check(hipGetLastError());
+  SetupArgs<Real> a{};
+  return launch_neighbors<Real, FULL>(a, st, btp, coords, max_dis, tiles, n_tiles, ws, row_cap,
+                                      dense, stream, Lw);
 }
 
 template <typename Real, int MODE>
 static void launch_lkb(const LkbArgs<Real>& a, int n_wg, hipStream_t stream) {
-  hipLaunchKernelGGL(fill_kernel<uint32_t>, dim3(2), dim3(256), 0, stream, a.row_cursor,
-                     8 * QSTRIDE, 0u);
   auto k = lkb_gather_kernel<Real, MODE>;
   if (n_wg <= 0) n_wg = resident_workgroups(k);
   hipLaunchKernelGGL(k, dim3(n_wg), dim3(256), 0, stream, a);
@@ -908,9 +904,11 @@ static int run_lkb_score(const tmol_ljlk_stack* st, const tmol_ljlk_block_types*
                        (const Real*)coords, (int4*)(w + Lk.info), (float4*)(w + Lk.opos),
                        (int32_t*)(w + Lk.oatom));
   }
+  ClearList c{};
+  c.add(a.row_cursor, 4 * 8 * QSTRIDE);
   if (census) {
-    hipLaunchKernelGGL(fill_kernel<unsigned long long>, dim3(1), dim3(64), 0, stream, census, 4,
-                       0ull);
+    c.add(census, 8 * 4);
+    launch_clear(c, stream);
     launch_lkb<Real, M_CENSUS>(a, n_wg, stream);
     return check(hipGetLastError());
   }
@@ -920,18 +918,18 @@ static int run_lkb_score(const tmol_ljlk_stack* st, const tmol_ljlk_block_types*
   const int P = st->n_poses;
   if (!noe) {
     if (bp)
-      fill<Real>((Real*)energies,
-                 4 * (st->layout == TMOL_LJLK_PADDED
-                          ? int64_t(P) * st->max_n_blocks * st->max_n_blocks
-                          : int64_t(st->n_blocks_total) * row_cap),
-                 stream);
+      c.add(energies, int64_t(sizeof(Real)) * 4 *
+                          (st->layout == TMOL_LJLK_PADDED
+                               ? int64_t(P) * st->max_n_blocks * st->max_n_blocks
+                               : int64_t(st->n_blocks_total) * row_cap));
     else
-      fill<double>(a.energies64, 4 * int64_t(P), stream);
+      c.add(a.energies64, 8 * 4 * int64_t(P));
   }
   if ((flags & TMOL_LJLK_WGRAD) && !acc) {
-    fill<Real>((Real*)dxyz, st->n_atoms_total * 3, stream);
-    fill<Real>((Real*)dwat, st->n_atoms_total * 12, stream);
+    c.add(dxyz, int64_t(sizeof(Real)) * st->n_atoms_total * 3);
+    c.add(dwat, int64_t(sizeof(Real)) * st->n_atoms_total * 12);
   }
+  launch_clear(c, stream);
   const int mode = flags & (TMOL_LJLK_WGRAD | TMOL_LJLK_BLOCK_PAIR | TMOL_LJLK_NO_ENERGY);
   switch (mode) {
     case 0: launch_lkb<Real, 0>(a, n_wg, stream); break;
@@ -999,11 +997,7 @@ static int run_hb_bases(const tmol_ljlk_stack* st, const tmol_ljlk_block_types* 
 
 template <typename Real, int MODE>
 static void launch_hb(const HbArgs<Real>& a, int n_wg, hipStream_t stream) {
-  hipLaunchKernelGGL(fill_kernel<uint32_t>, dim3(2), dim3(256), 0, stream, a.row_cursor,
-                     8 * QSTRIDE, 0u);
-  auto k = hb_score_kernel<Real, MODE>;
-  if (n_wg <= 0) n_wg = resident_workgroups(k);
-  hipLaunchKernelGGL(k, dim3(n_wg), dim3(256), 0, stream, a);
+  launch_persistent(hb_score_kernel<Real, MODE>, a, n_wg, stream);
 }
 
 template <typename Real>
@@ -1043,9 +1037,11 @@ static int run_hb_score(const tmol_ljlk_stack* st, const tmol_ljlk_block_types* 
   a.energies_bp = (Real*)energies;
   a.dxyz = (Real*)dxyz;
   a.census = census;
+  ClearList c{};
+  c.add(a.row_cursor, 4 * 8 * QSTRIDE);
   if (census) {
-    hipLaunchKernelGGL(fill_kernel<unsigned long long>, dim3(1), dim3(64), 0, stream, census, 3,
-                       0ull);
+    c.add(census, 8 * 3);
+    launch_clear(c, stream);
     launch_hb<Real, M_CENSUS>(a, n_wg, stream);
     return check(hipGetLastError());
   }
@@ -1055,11 +1051,13 @@ static int run_hb_score(const tmol_ljlk_stack* st, const tmol_ljlk_block_types* 
   const int P = st->n_poses;
   if (!noe) {
     if (bp)
-      fill<Real>((Real*)energies, int64_t(P) * st->max_n_blocks * st->max_n_blocks, stream);
+      c.add(energies, int64_t(sizeof(Real)) * P * st->max_n_blocks * st->max_n_blocks);
     else
-      fill<double>(a.energies64, int64_t(P), stream);
+      c.add(a.energies64, 8 * int64_t(P));
   }
-  if ((flags & TMOL_LJLK_WGRAD) && !acc) fill<Real>((Real*)dxyz, st->n_atoms_total * 3, stream);
+  if ((flags & TMOL_LJLK_WGRAD) && !acc)
+    c.add(dxyz, int64_t(sizeof(Real)) * st->n_atoms_total * 3);
+  launch_clear(c, stream);
   const int mode = flags & (TMOL_LJLK_WGRAD | TMOL_LJLK_BLOCK_PAIR | TMOL_LJLK_NO_ENERGY);
   switch (mode) {
     case 0: launch_hb<Real, 0>(a, n_wg, stream); break;
@@ -1225,10 +1223,12 @@ int tmol_ljlk_census(const tmol_ljlk_stack* s, const tmol_ljlk_block_types* bt,
   WsLayout L = ws_layout(s, bt, row_capacity, dtype);
   if (ws_bytes < L.total) return TMOL_LJLK_EINVAL;
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(fill_kernel<unsigned long long>, dim3(1), dim3(64), 0, st,
-                     (unsigned long long*)census, 16, 0ull);
   ScoreArgs<float> a = make_args<float>(s, bt, coords, workspace, row_capacity, L);
   a.census = (unsigned long long*)census;
+  ClearList c{};
+  c.add(a.row_cursor, 4 * 8 * QSTRIDE);
+  c.add(census, 8 * 16);
+  launch_clear(c, st);
   launch_score<float, M_CENSUS>(a, true, 0, st);
   return check(hipGetLastError());
 }
@@ -1685,16 +1685,15 @@ int tmol_ljlk_elec_prepare(const tmol_ljlk_stack* s, const tmol_ljlk_block_types
   BTView b = make_bt_view(bt);
   char* w = (char*)workspace;
   hipStream_t st = (hipStream_t)stream;
+  auto prepare = [&](auto a) {
+    a.bt = b;
+    setup_elec_tables(a, bt, e, w + L.e_pd, w + L.e_intra);
+    launch_setup(a, st);
+  };
   if (dtype == TMOL_LJLK_F32)
-    hipLaunchKernelGGL(elec_prepare_kernel<float>, dim3(b.T), dim3(64), 0, st, b,
-                       (const float*)e->partial_charge, e->inter_repr_path_distance,
-                       e->intra_repr_path_distance, (uint32_t*)(w + L.e_pd),
-                       (int32_t*)(w + L.e_intra), (uint16_t*)(w + L.e_intra + 4 * int64_t(b.T)));
+    prepare(SetupArgs<float>{});
   else
-    hipLaunchKernelGGL(elec_prepare_kernel<double>, dim3(b.T), dim3(64), 0, st, b,
-                       (const double*)e->partial_charge, e->inter_repr_path_distance,
-                       e->intra_repr_path_distance, (uint32_t*)(w + L.e_pd),
-                       (int32_t*)(w + L.e_intra), (uint16_t*)(w + L.e_intra + 4 * int64_t(b.T)));
+    prepare(SetupArgs<double>{});
   return check(hipGetLastError());
 }
 

@@ -9,14 +9,13 @@ namespace tmol_ljlk {
 
 // ------------------------------------------------------------------ prepare
 
+// record and connection path distances of atom a of block type t
 template <typename Real>
-__global__ void prepare_records_kernel(BTView bt, const Real* __restrict__ type_params,
-                                       int n_atom_types, Real* __restrict__ records,
-                                       uint8_t* __restrict__ conn_pd) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  int n = bt.T * bt.Amax;
-  if (i >= n) return;
-  int t = i / bt.Amax, a = i - t * bt.Amax;
+__device__ __forceinline__ void prepare_record(const BTView& bt, int t, int a,
+                                               const Real* __restrict__ type_params,
+                                               int n_atom_types, Real* __restrict__ records,
+                                               uint8_t* __restrict__ conn_pd) {
+  const int i = t * bt.Amax + a;
   int at = bt.atom_types[i];
   Real* r = records + int64_t(i) * REC;
   if (at < 0 || at >= n_atom_types || a >= bt.n_atoms[t]) {
@@ -56,16 +55,14 @@ __global__ void prepare_records_kernel(BTView bt, const Real* __restrict__ type_
   }
 }
 
-// Intra-block pairs of every block type with at most 32 atoms that carry
-// count-pair weight (path distance >= 4; the others score exactly zero),
-// a1 < a2 in the order (a1, a2), one wave per type (lanes over a2, ballot
-// compaction keeps the order):
+// Intra-block pairs of block type t (at most 32 atoms) that carry count-pair
+// weight (path distance >= 4; the others score exactly zero), a1 < a2 in the
+// order (a1, a2), by one wave (lanes over a2, ballot compaction keeps the
+// order):
 //   pairs[t * INTRA_MAX + k] = a1 | a2 << 5 | (path distance == 4) << 10
-__global__ __launch_bounds__(64) void prepare_intra_kernel(BTView bt, int32_t* __restrict__ count,
-                                                           uint16_t* __restrict__ pairs) {
-  const int t = blockIdx.x;
-  if (t >= bt.T) return;
-  const int lane = threadIdx.x;
+__device__ __forceinline__ void prepare_intra(const BTView& bt, int t, int lane,
+                                              int32_t* __restrict__ count,
+                                              uint16_t* __restrict__ pairs) {
   const int n = bt.n_atoms[t];
   int k = 0;
   if (n <= TILE)
@@ -90,11 +87,10 @@ __global__ __launch_bounds__(64) void prepare_intra_kernel(BTView bt, int32_t* _
 // order, divided by n, radius = sqrt(max d^2) with ((dx*dx + dy*dy) + dz*dz);
 // no contraction, IEEE division and square root.
 template <typename Real>
-__global__ void spheres_kernel(StackView s, BTView bt, const Real* __restrict__ coords,
-                               Real* __restrict__ spheres) {
+__device__ __forceinline__ void block_sphere(const StackView& s, const BTView& bt, int g,
+                                             const Real* __restrict__ coords,
+                                             Real* __restrict__ spheres) {
 #pragma clang fp contract(off)
-  int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= s.G) return;
   int t = s.block_type[g];
   Real* out = spheres + int64_t(g) * 4;
   if (t < 0) {
@@ -142,22 +138,78 @@ __global__ void spheres_kernel(StackView s, BTView bt, const Real* __restrict__ 
 // registers, so the lists need no atomics and come out sorted by g2.
 // The pair test is the reference's (sphere_overlap.impl.hh:287-351):
 // d^2 < ((r1 + r2) + reach)^2 with its association, no contraction.
+// Bound: latency of the column loop.  Each wave keeps its 64 columns in
+// registers, one per lane, loads the next chunk's before testing this one's,
+// and reduces the boxes with DPP, so the loop has no barrier and no LDS round
+// trip (512 poses: 207 us with columns staged in LDS behind two barriers).
+
+// v moved across lanes by a DPP control (every lane of the wave active)
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+  const int i = __float_as_int(v);
+  return __int_as_float(__builtin_amdgcn_update_dpp(i, i, CTRL, 0xf, 0xf, false));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = int(b & 0xffffffffll), hi = int(b >> 32);
+  const uint32_t l = uint32_t(__builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xf, 0xf, false));
+  const uint32_t h = uint32_t(__builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, false));
+  return __longlong_as_double((long long)((uint64_t(h) << 32) | l));
+}
+__device__ __forceinline__ float wave_lane(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ double wave_lane(double v, int l) {
+  const long long b = __double_as_longlong(v);
+  const uint32_t lo = __builtin_amdgcn_readlane(int(b & 0xffffffffll), l);
+  const uint32_t hi = __builtin_amdgcn_readlane(int(b >> 32), l);
+  return __longlong_as_double((long long)((uint64_t(hi) << 32) | lo));
+}
+
+// smallest v of the wave: within rows of 16 lanes by quad permutes (xor 1, 2)
+// and mirrors (half row, row), then across the four rows
 template <typename Real>
-__device__ __forceinline__ void chunk_box(const Real (*sph)[4], const int* typ, int lane,
-                                          Real* lo, Real* hi) {
-  const bool ok = typ[lane] >= 0;
+__device__ __forceinline__ Real wave_min(Real v) {
+  v = fmin(v, dpp_move<0xB1>(v));
+  v = fmin(v, dpp_move<0x4E>(v));
+  v = fmin(v, dpp_move<0x141>(v));
+  v = fmin(v, dpp_move<0x140>(v));
+  return fmin(fmin(wave_lane(v, 0), wave_lane(v, 16)), fmin(wave_lane(v, 32), wave_lane(v, 48)));
+}
+
+// one block's sphere and type, as a lane of the neighbor pass holds it
+template <typename Real>
+struct NbrSphere {
+  Real x, y, z, r;
+  int type;
+};
+
+template <typename Real>
+__device__ __forceinline__ NbrSphere<Real> load_sphere(const StackView& s, const Real* spheres,
+                                                       int g, int end) {
+  NbrSphere<Real> q{Real(0), Real(0), Real(0), Real(0), -1};
+  if (g < end) {
+    const Real* p = spheres + int64_t(g) * 4;
+    q.x = p[0];
+    q.y = p[1];
+    q.z = p[2];
+    q.r = p[3];
+    q.type = s.block_type[g];
+  }
+  return q;
+}
+
+// bounding box of the wave's spheres
+template <typename Real>
+__device__ __forceinline__ void chunk_box(const NbrSphere<Real>& q, Real* lo, Real* hi) {
+  const bool ok = q.type >= 0;
   const Real big = Real(1e30);
+  const Real c[3] = {q.x, q.y, q.z};
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    Real l = ok ? sph[lane][k] - sph[lane][3] : big;
-    Real h = ok ? sph[lane][k] + sph[lane][3] : -big;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      l = fmin(l, __shfl_xor(l, o, WAVE));
-      h = fmax(h, __shfl_xor(h, o, WAVE));
-    }
-    lo[k] = l;
-    hi[k] = h;
+    lo[k] = wave_min(ok ? c[k] - q.r : big);
+    hi[k] = -wave_min(ok ? -(c[k] + q.r) : big);
   }
 }
 
@@ -173,67 +225,60 @@ __global__ __launch_bounds__(256) void neighbor_rows_kernel(
     int32_t* __restrict__ dense, const int32_t* __restrict__ pose_start = nullptr) {
 #pragma clang fp contract(off)
   __shared__ Real sph_r[NBR_TILE][4];
-  __shared__ Real sph_c[NBR_TILE][4];
   __shared__ int typ_r[NBR_TILE];
-  __shared__ int typ_c[NBR_TILE];
   const int64_t tile_id = blockIdx.x;
   if (tile_id >= n_tiles) return;
   const int4 tl = tiles[tile_id];
   if (tl.x != tl.y) return;
   const int row0 = tl.x, end = tl.z;
-  const int tid = threadIdx.x;
   const int lane = lane_id();
-  const int wave = tid / WAVE;
-  if (tid < NBR_TILE) {
-    const int g = row0 + tid;
-    const bool ok = g < end;
-    for (int k = 0; k < 4; ++k) sph_r[tid][k] = ok ? spheres[int64_t(g) * 4 + k] : Real(0);
-    typ_r[tid] = ok ? s.block_type[g] : -1;
+  const int wave = threadIdx.x / WAVE;
+  const NbrSphere<Real> mine = load_sphere(s, spheres, row0 + lane, end);
+  const int col_begin =
+      !FULL ? row0 : (s.layout == TMOL_LJLK_PADDED ? tl.w * s.B : pose_start[tl.w]);
+  NbrSphere<Real> next = load_sphere(s, spheres, col_begin + lane, end);
+  if (wave == 0) {
+    sph_r[lane][0] = mine.x;
+    sph_r[lane][1] = mine.y;
+    sph_r[lane][2] = mine.z;
+    sph_r[lane][3] = mine.r;
+    typ_r[lane] = mine.type;
   }
   __syncthreads();
   Real rlo[3], rhi[3];
-  chunk_box(sph_r, typ_r, lane, rlo, rhi);
+  chunk_box(mine, rlo, rhi);
   const Real pad = reach + Real(1e-3);
   uint32_t cnt[16];
 #pragma unroll
   for (int r = 0; r < 16; ++r) cnt[r] = 0;
   bool overflow = false;
-  const int col_begin =
-      !FULL ? row0 : (s.layout == TMOL_LJLK_PADDED ? tl.w * s.B : pose_start[tl.w]);
   for (int col0 = col_begin; col0 < end; col0 += NBR_TILE) {
-    __syncthreads();  // the previous column chunk is no longer read
-    if (tid < NBR_TILE) {
-      const int g = col0 + tid;
-      const bool ok = g < end;
-      for (int k = 0; k < 4; ++k) sph_c[tid][k] = ok ? spheres[int64_t(g) * 4 + k] : Real(0);
-      typ_c[tid] = ok ? s.block_type[g] : -1;
-    }
-    __syncthreads();
+    const NbrSphere<Real> col = next;
+    next = load_sphere(s, spheres, col0 + NBR_TILE + lane, end);
     Real clo[3], chi[3];
-    chunk_box(sph_c, typ_c, lane, clo, chi);
+    chunk_box(col, clo, chi);
     Real gap2 = Real(0);
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
       const Real gk = fmax(Real(0), fmax(clo[k] - rhi[k], rlo[k] - chi[k]));
       gap2 += gk * gk;
     }
-    if (gap2 > pad * pad) continue;  // uniform across the workgroup
+    if (gap2 > pad * pad) continue;  // uniform across the wave
     const int g2 = col0 + lane;
-    const Real c0 = sph_c[lane][0], c1 = sph_c[lane][1], c2 = sph_c[lane][2], c3 = sph_c[lane][3];
-    const bool col_ok = typ_c[lane] >= 0;
+    const bool col_ok = col.type >= 0;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int lr = wave * 16 + r;
       const int g1 = row0 + lr;
       const bool ok = col_ok && typ_r[lr] >= 0 && (FULL || g1 <= g2);
-      const Real dx = sph_r[lr][0] - c0;
-      const Real dy = sph_r[lr][1] - c1;
-      const Real dz = sph_r[lr][2] - c2;
+      const Real dx = sph_r[lr][0] - col.x;
+      const Real dy = sph_r[lr][1] - col.y;
+      const Real dz = sph_r[lr][2] - col.z;
       const Real dxx = dx * dx;
       const Real dyy = dy * dy;
       const Real dzz = dz * dz;
       const Real d2 = (dxx + dyy) + dzz;
-      const Real thr = (sph_r[lr][3] + c3) + reach;
+      const Real thr = (sph_r[lr][3] + col.r) + reach;
       const Real thr2 = thr * thr;
       const bool hit = ok && (d2 < thr2);
       const uint64_t m = __ballot(hit);
@@ -261,6 +306,32 @@ __global__ __launch_bounds__(256) void neighbor_rows_kernel(
   }
   if (__ballot(overflow) != 0 && lane == 0) atomicOr(&counters[1], 1u);
   if (total > 0 && lane == 0) atomicAdd(&counters[0], total);
+}
+
+// ------------------------------------------------------------------ setup
+
+// Clears of one call, done by one launch instead of one each: up to CLEAR_N
+// ranges of 4-byte words set to 0.
+constexpr int CLEAR_N = 6;
+struct ClearList {
+  uint32_t* p[CLEAR_N];
+  int64_t n[CLEAR_N];
+  int used;
+  void add(void* q, int64_t bytes) {
+    p[used] = (uint32_t*)q;
+    n[used++] = bytes / 4;
+  }
+};
+
+__device__ __forceinline__ void clear_ranges(const ClearList& c, int64_t i0, int64_t stride) {
+  for (int k = 0; k < c.used; ++k) {
+    uint32_t* p = c.p[k];
+    for (int64_t i = i0; i < c.n[k]; i += stride) p[i] = 0;
+  }
+}
+
+__global__ __launch_bounds__(256) void clear_kernel(ClearList c) {
+  clear_ranges(c, int64_t(blockIdx.x) * 256 + threadIdx.x, int64_t(gridDim.x) * 256);
 }
 
 // ------------------------------------------------------------------ small kernels

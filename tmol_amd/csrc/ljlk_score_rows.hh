@@ -58,18 +58,6 @@ __device__ __forceinline__ double lane_val(double v, int j) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// four Reals moved as one 16-byte (float) or 32-byte (double) access
-template <typename Real>
-struct V4;
-template <>
-struct V4<float> {
-  using T = float4;
-};
-template <>
-struct V4<double> {
-  using T = double4;
-};
-
 // one lane's atom of a block, held in registers between its global load and
 // its LDS staging: coordinates, prepared record, connection path distances
 template <typename Real>

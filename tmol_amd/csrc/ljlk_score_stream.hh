@@ -121,27 +121,6 @@ __device__ __forceinline__ uint32_t combine_q(const uint32_t cs[MAX_CONN], uint3
   return q;
 }
 
-// packed connection separations cs[c1] (byte c2) of the pair (g1, g2), g1 < g2
-__device__ __forceinline__ void conn_rows(const StackView& s, int g1, int g2, int nc1, int nc2,
-                                          uint32_t cs[MAX_CONN]) {
-#pragma unroll
-  for (int c1 = 0; c1 < MAX_CONN; ++c1) cs[c1] = 0x06060606u;
-  if (s.layout == TMOL_LJLK_PADDED) {
-    for (int c1 = 0; c1 < nc1; ++c1) {
-      uint32_t r = 0x06060606u;
-      for (int c2 = 0; c2 < nc2; ++c2) {
-        const uint32_t v = (uint32_t)min(conn_sep(s, g1, g2, c1, c2), 6);
-        r = (r & ~(255u << (8 * c2))) | (v << (8 * c2));
-      }
-      cs[c1] = r;
-    }
-    return;
-  }
-  const int32_t* e = bonded_row(s, g1, g2);
-  if (!e) return;
-  for (int c1 = 0; c1 < nc1; ++c1) cs[c1] = (uint32_t)e[4 + c1];
-}
-
 // gradient gs (x1 - x2) of an entry's pair: + to the g1 atom's slot s1 (odd
 // lanes: its second copy), - to slot s2 (a ring slot, or a g1 slot for
 // intra-block pairs)
@@ -502,7 +481,7 @@ __global__ __launch_bounds__(256, (stream_waves_per_simd<MODE, OCC>())) void sco
       // ---- descriptors: one neighbor block per lane
       const int nb = min(WAVE, n_items - c0);
       int d_t2 = 0, d_o2 = 0, d_n2 = 0, d_info = 0;
-      uint32_t cs[MAX_CONN] = {Q_NONE, Q_NONE, Q_NONE, Q_NONE};
+      uint32_t cs[MAX_CONN] = {0, 0, 0, 0};  // read for blocks within 4 bonds only
       if (lane < nb) {
         const int g2 = A.w.row_items[row * A.w.row_cap + c0 + lane];
         if (g2 != g1) {
@@ -510,10 +489,9 @@ __global__ __launch_bounds__(256, (stream_waves_per_simd<MODE, OCC>())) void sco
           d_o2 = s.block_atom_offset[g2];
           d_n2 = bt.n_atoms[d_t2];
           const int nc2 = bt.n_conn[d_t2];
-          const int ms = min_block_sep(s, g1, g2, nc1, nc2);
+          const int ms = pair_separations(s, g1, g2, nc1, nc2, cs);
           const bool lig2 = lig1 && bt.is_ligand[d_t2] != 0;
           d_info = (ms <= 4 ? 1 : 0) | (lig2 ? 2 : 0) | (d_n2 << 8);
-          if (ms <= 4) conn_rows(s, g1, g2, nc1, nc2, cs);
         }
       }
       // exclusive scan of the atom counts: the stream position of each block
