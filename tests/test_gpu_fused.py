@@ -111,3 +111,42 @@ def test_fused_on_the_512_pose_batch():
     assert (e4[3] - e1).abs().max().item() < 1e-4
     g = g3 + g1
     assert ((g4 - g).norm() / g.norm()).item() < 1e-6
+
+
+@pytest.mark.parametrize("n,lo,hi", [(1, 2, 2), (1, 9, 9), (2, 33, 35), (9, 40, 90), (220, 2, 7)])
+def test_split_rows_equal_the_oracles(n, lo, hi):
+    """Rows are split into parts when a batch has fewer rows than resident
+    waves: per-pose energies, the weighted gradient and the drop-in ops'
+    per-term derivatives from one residue pair to more rows than waves."""
+    poses = generate_poses(n, (lo, hi), seed=11 + n)
+    _say("split rows %d x %d-%d" % (n, lo, hi))
+    ps = PoseStack(poses, dtype=torch.float64)
+    a = pose_op_args(ps, LJLKEnergyTerm())
+    b = elec_op_args(ps, ElecEnergyTerm())
+    a[23], a[24] = a[23].double(), a[24].double()
+    b[16], b[22] = b[16].double(), b[22].double()
+    s3, _, dv3, _ = orc.oracle_pose_scores(*a, require_grad=True)
+    s1, _, dv1, _ = orc.oracle_elec_scores(*b, require_grad=True)
+    keep = numpy.concatenate([p * ps.max_n_atoms + numpy.arange(q.n_atoms)
+                              for p, q in enumerate(poses)])
+    st, fused, _, _ = _scorers(poses, torch.float64)
+    e4, g4 = [t.cpu().numpy() for t in fused.energy_and_grad(st.coords.to(DEV), torch.tensor(W4))]
+    oe = numpy.concatenate([s3, s1], axis=0)
+    og = (dv3 * W4[:3, None, None]).sum(0) + W4[3] * dv1[0]
+    # float64 on both sides, the bounds of the fused test above
+    assert (numpy.abs(e4 - oe) / numpy.maximum(1.0, numpy.abs(oe))).max() < 1e-9
+    assert numpy.abs(g4 - og[keep]).max() / max(1.0, numpy.abs(og).max()) < 1e-9
+    from tmol_amd.ops import elec_pose_scores, ljlk_pose_scores
+
+    for op, args, want, w in ((ljlk_pose_scores, a, dv3, W4[:3]),
+                              (elec_pose_scores, b, dv1, W4[3:])):
+        for bp in (False, True):
+            d = [t.to(DEV) if torch.is_tensor(t) else t for t in args[:-1]] + [bp]
+            x = d[0].clone().requires_grad_(True)
+            out = op(x, *d[1:])
+            scores = out[0] if isinstance(out, (tuple, list)) else out
+            wt = torch.tensor(w, device=DEV).view([-1] + [1] * (scores.dim() - 1))
+            (scores * wt).sum().backward()
+            go = (want * w[:, None, None]).sum(0)
+            err = numpy.abs(x.grad.cpu().numpy() - go).max()
+            assert err <= 1e-9 * max(1.0, numpy.abs(go).max()), (op, bp, err)

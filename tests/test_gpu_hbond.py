@@ -158,3 +158,30 @@ def test_single_block_and_glycine_poses(term):
     E, _ = hbond_pose_scores(*_dev(score_op_args(ps, term, D, I), "cuda"))
     Eo, _, _ = orc.oracle_hb_score(score_op_args(ps, term, D.cpu(), I.cpu()), ba)
     assert numpy.abs(E.cpu().numpy() - Eo).max() <= 1e-10 * max(1.0, numpy.abs(Eo).max())
+
+
+@pytest.mark.parametrize("n,lo,hi", [(1, 2, 2), (1, 17, 17), (3, 31, 34), (300, 2, 9), (70, 3, 60)])
+def test_rows_walked_together_across_poses(term, n, lo, hi):
+    """A wave walks several rows at once and carries passing pairs from row
+    to row: poses of a few residues (pairs of several poses evaluated
+    together), one pose (rows split into parts) and ragged ends, per-pose
+    energies and gradient in float64 against the oracle."""
+    from tmol_amd.hbond import HBondRaggedScorer
+
+    print("hbond rows", n, lo, hi, flush=True)
+    poses = generate_poses(n, (lo, hi), seed=31 + n)
+    rs = RaggedPoseStack(poses, dtype=torch.float64)
+    sc = HBondRaggedScorer(rs, term, device="cuda", dtype=torch.float64)
+    w = torch.linspace(0.5, 1.5, n, dtype=torch.float64)
+    E, G = sc.energy_and_grad(rs.coords.cuda(), w.cuda())
+    ps = PoseStack(poses, dtype=torch.float64)
+    ba = bases_op_args(ps, term)
+    Do, Io = orc.oracle_hb_bases(*ba)
+    sa = score_op_args(ps, term, torch.tensor(Do), torch.tensor(Io))
+    Eo, _, dX = orc.oracle_hb_score(sa, ba, dTdV=w.numpy()[None, :])
+    # the same formulas summed in another order (TOL's float64 bounds)
+    assert numpy.abs(E.cpu().numpy() - Eo[0]).max() <= 1e-10 * max(1.0, numpy.abs(Eo).max())
+    keep = numpy.concatenate([p * ps.max_n_atoms + numpy.arange(q.n_atoms)
+                              for p, q in enumerate(poses)])
+    go = dX[keep]
+    assert numpy.abs(G.cpu().numpy() - go).max() <= 1e-9 * max(1.0, numpy.abs(go).max())

@@ -16,8 +16,11 @@ constexpr int HB_POLY = 16;     // c10..c0, pad, xmin, xmax, min_val, max_val (d
 constexpr int HB_DW = TMOL_HBOND_DON_WIDTH;
 constexpr int HB_AW = TMOL_HBOND_ACC_WIDTH;
 constexpr int HB_CHUNK = 64;    // work-list items staged per pass
+constexpr int HB_ROWS = 4;      // rows walked together, 16 lanes each
+constexpr int HB_SUB = WAVE / HB_ROWS;
 constexpr int HB_FIFO = 128;    // passing donor x acceptor pairs awaiting evaluation
 constexpr int HB_MAX_SEP = 4;   // pairs below separation 5 score 0
+constexpr int HB_PD_CAP = 255;  // packed path distances (a separation above 4 needs no more)
 
 // ------------------------------------------------------------------ bases
 
@@ -331,40 +334,71 @@ struct HbArgs {
   Real* energies_bp;             // block pairs
   Real* dxyz;                    // [NA, 3]
   unsigned long long* census;    // [3]
-  int part_shift;                // rows are not split into parts: 0
+  int part_shift;                // a row is 2^part_shift queue units
 };
 
 // a work-list item of the row: the other block, its type, first atom,
 // donor / acceptor / connection counts, minimum separation from the row's
 // block and its candidate donor x acceptor pairs
 struct HbItem {
-  int g2, bt2, off2, nd2, na2, nc2, msep, cand;
+  int row, g2, bt2, off2, nd2, na2, nc2, msep;
+  uint32_t cs[MAX_CONN];  // connection separations to the row's block (msep <= 4)
+};
+
+// the row of a lane group
+struct HbRow {
+  int g1, bt1, off1, nd1, na1, nc1;
 };
 
 struct HbLDS {
   HbItem it[HB_CHUNK];
+  HbRow row[HB_ROWS];
+  uint32_t pd1[HB_ROWS][TILE];  // path distances from its connections, by list position
   int32_t cend[HB_CHUNK];  // inclusive prefix sums of cand
-  int32_t qh[HB_FIFO], qa[HB_FIFO], qt[HB_FIFO], qb[HB_FIFO];  // H, A, types, other block
+  // H, A, types, the row's block and the other block
+  int32_t qh[HB_FIFO], qa[HB_FIFO], qt[HB_FIFO], qg[HB_FIFO], qb[HB_FIFO];
 };
 
-// evaluate n (<= 64) FIFO entries from head
+// energies of one pose summed by a wave's lanes, added to the pose's total
+// when an entry of another pose comes
+struct HbEnergy {
+  LaneSum sum;
+  int pose = -1;  // wave-uniform
+  __device__ __forceinline__ void flush(double* energies64) {
+    if (pose < 0) return;
+    const double v = wave_sum(sum.value());
+    if (lane_id() == 0 && v != 0.0) unsafeAtomicAdd(&energies64[pose], v);
+    sum = LaneSum();
+  }
+};
+
+// evaluate n (<= 64) FIFO entries from head; they may come from several rows
 template <typename Real, int MODE>
-__device__ __forceinline__ void hb_phase_b(HbLDS& L, const HbArgs<Real>& a, int g1, int head,
-                                           int n, int lane, Real w_row, LaneSum& esum,
-                                           unsigned long long& n_eval) {
+__device__ __forceinline__ void hb_phase_b(HbLDS& L, const HbArgs<Real>& a, int head, int n,
+                                           int lane, HbEnergy& en, unsigned long long& n_eval) {
   constexpr bool DERIV = (MODE & M_WGRAD) != 0;
   constexpr bool BP = (MODE & M_BP) != 0;
   constexpr bool NOE = (MODE & M_NOE) != 0;
   constexpr bool CENSUS = (MODE & M_CENSUS) != 0;
-  if (lane >= n) return;
+  if (CENSUS) {
+    n_eval += lane < n;
+    return;
+  }
   const int e = (head + lane) & (HB_FIFO - 1);
+  const int pose = !BP && lane < n ? a.s.pose_of(L.qg[e]) : 0;
+  bool mixed = false;
+  if (!BP && !NOE) {
+    const int first = __builtin_amdgcn_readfirstlane(pose);
+    mixed = __ballot(lane < n && pose != first) != 0;
+    if (mixed || first != en.pose) {
+      en.flush(a.energies64);
+      en.pose = first;
+    }
+  }
+  if (lane >= n) return;
   const int64_t h = L.qh[e], x = L.qa[e];
   const int ty = L.qt[e];
   const int dt = ty & 0xffff, at = ty >> 16;
-  if (CENSUS) {
-    ++n_eval;
-    return;
-  }
   const int64_t pi = int64_t(dt) * a.n_acc_types + at;
   const Vec3<Real> D = v3(a.derived + 9 * h), H = v3(a.coords + 3 * h), A = v3(a.coords + 3 * x);
   const Vec3<Real> B = v3(a.derived + 9 * x + 3), B0 = v3(a.derived + 9 * x + 6);
@@ -373,24 +407,27 @@ __device__ __forceinline__ void hb_phase_b(HbLDS& L, const HbArgs<Real>& a, int 
                                         a.polys + 3 * HB_POLY * pi, a.gp, g);
   int64_t cell = 0;
   if (BP) {
-    const int g2 = L.qb[e];
+    const int g1 = L.qg[e], g2 = L.qb[e];
     const int lo = g1 < g2 ? g1 : g2, hi = g1 < g2 ? g2 : g1;
     const int p = lo / a.s.B;
     cell = (int64_t(p) * a.s.B + (lo - p * a.s.B)) * a.s.B + (hi - p * a.s.B);
-    if (!NOE && E != Real(0)) atomicAdd(&a.energies_bp[cell], E);
+    if (!NOE && E != Real(0)) unsafeAtomicAdd(&a.energies_bp[cell], E);
   } else if (!NOE) {
-    esum.add(E);
+    if (pose == en.pose)
+      en.sum.add(E);
+    else
+      unsafeAtomicAdd(&a.energies64[pose], double(E));
   }
   if (DERIV) {
-    const Real w = BP ? a.weights[cell] : w_row;
+    const Real w = a.weights[BP ? cell : pose];
     const int64_t atoms[5] = {a.dinds[3 * h], h, x, a.dinds[3 * x + 1], a.dinds[3 * x + 2]};
 #pragma unroll
     for (int j = 0; j < 5; ++j) {
       if (atoms[j] < 0) continue;
       const Real gx = w * g[j].x, gy = w * g[j].y, gz = w * g[j].z;
-      if (gx != Real(0)) atomicAdd(&a.dxyz[3 * atoms[j]], gx);
-      if (gy != Real(0)) atomicAdd(&a.dxyz[3 * atoms[j] + 1], gy);
-      if (gz != Real(0)) atomicAdd(&a.dxyz[3 * atoms[j] + 2], gz);
+      if (gx != Real(0)) unsafeAtomicAdd(&a.dxyz[3 * atoms[j]], gx);
+      if (gy != Real(0)) unsafeAtomicAdd(&a.dxyz[3 * atoms[j] + 1], gy);
+      if (gz != Real(0)) unsafeAtomicAdd(&a.dxyz[3 * atoms[j] + 2], gz);
     }
   }
 }
@@ -405,19 +442,26 @@ __device__ __forceinline__ void hb_phase_b(HbLDS& L, const HbArgs<Real>& a, int 
 // reference's lookup with the donor's and acceptor's list positions as atom
 // indices; intra-block pairs: the atoms' path distance), then the H-A
 // distance against max_ha_dis.  Passing pairs are compacted into an LDS
-// FIFO and evaluated 64 at a time.  Energies: per-pose FP64 sums (one
-// atomic per row) or block-pair cells; gradients through the derived atoms'
-// indices with global atomics (few pairs pass).
-// waves per SIMD the scoring kernel is compiled for: it is latency-bound
-// (the per-item loads form dependent chains), so occupancy pays until the
-// register cap spills.  Measured on the 512-pose batch: gradients 3 / 4 / 5 /
-// 6 waves 1.07 / 0.91 / 1.03 / 1.10 ms (5 and 6 spill); energies 4 / 5 / 6 / 8
-// waves 0.74 / 0.68 / 0.67 / 0.67 ms (6 and 8 spill)
+// FIFO and evaluated 64 at a time.  Energies: per-pose FP64 sums or block-pair
+// cells; gradients through the derived atoms' indices with global atomics
+// (few pairs pass).
+// The kernel is bound by the latency of its dependent loads (row, item, type,
+// list entry, coordinates: 80% of the wave cycles waited), not by arithmetic
+// (VALU 25-28% busy), so a wave walks HB_ROWS rows at once, 16 lanes each: a
+// protein row has 10-20 items, which filled a quarter of the lanes of a wave
+// of its own.  The FIFO is carried from row to row: a row has about 2.5
+// passing pairs, and draining them at its end ran the evaluation with 4% of
+// its lanes.  256 poses of 50-600 residues with gradients: one row per wave
+// 312 us, the carried FIFO alone 320 us, four rows 234 us, and 203 us with
+// the registers of three waves per SIMD.
+// Waves per SIMD: the fewest that spill nothing.  Same batch, gradients at
+// 3 / 4 / 5 waves 203 / 234 / 247 us (4 and 5 spill), energies at 4 / 5 / 6
+// waves 187 / 193 / 200 us.
 #ifndef TMOL_HB_WAVES_GRAD
-#define TMOL_HB_WAVES_GRAD 4
+#define TMOL_HB_WAVES_GRAD 3
 #endif
 #ifndef TMOL_HB_WAVES_ENERGY
-#define TMOL_HB_WAVES_ENERGY 5
+#define TMOL_HB_WAVES_ENERGY 4
 #endif
 template <int MODE>
 constexpr int hb_waves_per_simd() {
@@ -430,52 +474,78 @@ __global__ __launch_bounds__(256, hb_waves_per_simd<MODE>()) void hb_score_kerne
   constexpr bool BP = (MODE & M_BP) != 0;
   constexpr bool NOE = (MODE & M_NOE) != 0;
   constexpr bool CENSUS = (MODE & M_CENSUS) != 0;
+  using V = typename V4<Real>::T;
   __shared__ HbLDS lds_all[WAVES_PER_WG];
   const int wave = threadIdx.x >> 6, lane = lane_id();
   HbLDS& L = lds_all[wave];
   const Real max_ha = a.gp[5];
   unsigned long long n_cand = 0, n_cp = 0, n_eval = 0;
-  RowQueue rq(a.row_cursor, a.s.G);
-  for (int64_t row = rq.next(); row >= 0; row = rq.next()) {
-    const int g1 = int(row);
-    const int bt1 = a.s.block_type[g1];
-    if (bt1 < 0) continue;
-    const int n_items = int(min<int64_t>(a.w.row_count[g1], a.w.row_cap));
-    const int nd1 = a.n_don[bt1], na1 = a.n_acc[bt1];
-    if (n_items == 0 || (nd1 == 0 && na1 == 0)) continue;
-    const int pose = a.s.pose_of(g1);
-    const int64_t off1 = a.s.block_atom_offset[g1];
-    const int nc1 = a.n_conn[bt1];
-    const int32_t* items = a.w.row_items + int64_t(g1) * a.w.row_cap;
-    const Real w_row = (DERIV && !BP) ? a.weights[pose] : Real(0);
-    LaneSum esum;
-    int head = 0, tail = 0;
-    for (int k0 = 0; k0 < n_items; k0 += HB_CHUNK) {
-      const int n = n_items - k0 < HB_CHUNK ? n_items - k0 : HB_CHUNK;
+  HbEnergy en;
+  int head = 0, tail = 0;
+  const int shift = a.part_shift;
+  RowQueue rq(a.row_cursor, int64_t(a.s.G) << shift, HB_ROWS);
+  const int grp = lane / HB_SUB, sl = lane % HB_SUB;
+  for (bool last = false; !last;) {
+    int n_units = 0;
+    const int64_t u0 = rq.next_range(n_units);
+    last = u0 < 0;  // nothing left but the FIFO
+    // this lane group's row and its items [k, n_items)
+    HbRow R{0, -1, 0, 0, 0, 0};
+    int k = 0, n_items = 0;
+    if (grp < n_units) {
+      const int64_t unit = u0 + grp, row = unit >> shift;
+      R.g1 = int(row);
+      R.bt1 = a.s.block_type[row];
+      const int n_row = int(min<int64_t>(a.w.row_count[row], a.w.row_cap));
+      R.off1 = a.s.block_atom_offset[row];
+      if (R.bt1 >= 0) {
+        R.nd1 = a.n_don[R.bt1];
+        R.na1 = a.n_acc[R.bt1];
+        R.nc1 = a.n_conn[R.bt1];
+        if (R.nd1 + R.na1 > 0) {
+          const int64_t part = unit - (row << shift);
+          k = int((n_row * part) >> shift) + sl;
+          n_items = int((n_row * (part + 1)) >> shift);
+        }
+      }
+    }
+    const int32_t* items = a.w.row_items + int64_t(R.g1) * a.w.row_cap;
+    const V s1 = *(const V*)(a.spheres + 4 * int64_t(R.g1));
+    if (sl == 0) L.row[grp] = R;
+    if (R.bt1 >= 0)
+      for (int x = sl; x < a.Am; x += HB_SUB) {
+        uint32_t pk = 0;
+        for (int c = 0; c < R.nc1; ++c) {
+          const int ca = a.conn_atoms[R.bt1 * a.s.C + c];
+          const int v = a.path_distance[(int64_t(R.bt1) * a.Am + ca) * a.Am + x];
+          pk |= (uint32_t)min(v, HB_PD_CAP) << (8 * c);
+        }
+        L.pd1[grp][x] = pk;
+      }
+    for (; __ballot(k < n_items) != 0 || (last && tail > head); k += HB_SUB) {
       int cand = 0;
-      if (lane < n) {
-        HbItem it;
-        it.g2 = items[k0 + lane];
+      HbItem it;
+      it.row = grp;
+      if (k < n_items) {
+        it.g2 = items[k];
         it.bt2 = a.s.block_type[it.g2];
         it.off2 = a.s.block_atom_offset[it.g2];
+        const V s2 = *(const V*)(a.spheres + 4 * int64_t(it.g2));
         it.nd2 = it.bt2 >= 0 ? a.n_don[it.bt2] : 0;
         it.na2 = it.bt2 >= 0 ? a.n_acc[it.bt2] : 0;
         it.nc2 = it.bt2 >= 0 ? a.n_conn[it.bt2] : 0;
         it.msep = 6;
-        if (it.g2 == g1) {
-          cand = nd1 * na1;
+        if (it.g2 == R.g1) {
+          cand = R.nd1 * R.na1;
         } else if (it.bt2 >= 0) {
           // blocks whose spheres stay farther apart than max_ha_dis (with
           // a margin for rounding) hold no pair within it
-          const Real* s1 = a.spheres + 4 * int64_t(g1);
-          const Real* s2 = a.spheres + 4 * int64_t(it.g2);
-          const Vec3<Real> dc = {s1[0] - s2[0], s1[1] - s2[1], s1[2] - s2[2]};
-          if (norm3(dc) <= s1[3] + s2[3] + max_ha + Real(1e-3)) {
-            it.msep = min_block_sep(a.s, g1, it.g2, nc1, it.nc2);
-            cand = nd1 * it.na2 + na1 * it.nd2;
+          const Vec3<Real> dc = {s1.x - s2.x, s1.y - s2.y, s1.z - s2.z};
+          if (norm3(dc) <= s1.w + s2.w + max_ha + Real(1e-3)) {
+            it.msep = pair_separations(a.s, R.g1, it.g2, R.nc1, it.nc2, it.cs);
+            cand = R.nd1 * it.na2 + R.na1 * it.nd2;
           }
         }
-        it.cand = cand;
         L.it[lane] = it;
       }
       // inclusive prefix sum of the candidate counts
@@ -485,16 +555,16 @@ __global__ __launch_bounds__(256, hb_waves_per_simd<MODE>()) void hb_score_kerne
         const int v = __shfl_up(incl, o, WAVE);
         if (lane >= o) incl += v;
       }
-      if (lane < n) L.cend[lane] = incl;
+      L.cend[lane] = incl;
       const int total = __shfl(incl, WAVE - 1, WAVE);
       if (CENSUS) n_cand += uint64_t(lane == 0 ? total : 0);
       wave_sync();
-      for (int base = 0; base < total; base += WAVE) {
+      for (int base = 0; base < total || (last && tail > head); base += WAVE) {
         const int c = base + lane;
         bool pass = false;
-        int32_t qh = 0, qa = 0, qt = 0, qb = 0;
+        int32_t qh = 0, qa = 0, qt = 0, qg = 0, qb = 0;
         if (c < total) {
-          int lo = 0, hi = n - 1;
+          int lo = 0, hi = WAVE - 1;
           while (lo < hi) {
             const int mid = (lo + hi) >> 1;
             if (L.cend[mid] > c)
@@ -503,10 +573,12 @@ __global__ __launch_bounds__(256, hb_waves_per_simd<MODE>()) void hb_score_kerne
               lo = mid + 1;
           }
           const HbItem& it = L.it[lo];
+          const HbRow& rw = L.row[it.row];
+          const int bt1 = rw.bt1, na1 = rw.na1;
           const int pp = c - (lo ? L.cend[lo - 1] : 0);
           int hl, al, dt, at, sep;
           int64_t ho, ao;
-          if (it.g2 == g1) {
+          if (it.g2 == rw.g1) {
             const int i = pp / na1, j = pp - i * na1;
             const int32_t* dr = a.don + (int64_t(bt1) * a.Dmax + i) * HB_DW;
             const int32_t* ar = a.acc + (int64_t(bt1) * a.Xmax + j) * HB_AW;
@@ -514,10 +586,10 @@ __global__ __launch_bounds__(256, hb_waves_per_simd<MODE>()) void hb_score_kerne
             dt = dr[2];
             al = ar[0];
             at = ar[3];
-            ho = ao = off1;
+            ho = ao = rw.off1;
             sep = a.path_distance[(int64_t(bt1) * a.Am + hl) * a.Am + al];
           } else {
-            const int nA = nd1 * it.na2;
+            const int nA = rw.nd1 * it.na2;
             int r1, r2;  // positions in g1's and g2's lists (the count-pair lookup)
             if (pp < nA) {  // g1 donates, g2 accepts
               const int i = pp / it.na2, j = pp - i * it.na2;
@@ -527,7 +599,7 @@ __global__ __launch_bounds__(256, hb_waves_per_simd<MODE>()) void hb_score_kerne
               dt = dr[2];
               al = ar[0];
               at = ar[3];
-              ho = off1;
+              ho = rw.off1;
               ao = it.off2;
               r1 = i;
               r2 = j;
@@ -541,20 +613,19 @@ __global__ __launch_bounds__(256, hb_waves_per_simd<MODE>()) void hb_score_kerne
               al = ar[0];
               at = ar[3];
               ho = it.off2;
-              ao = off1;
+              ao = rw.off1;
               r1 = j;
               r2 = i;
             }
             sep = it.msep;
             if (sep <= HB_MAX_SEP) {
               int best = HB_MAX_SEP + 1;
-              for (int c1 = 0; c1 < nc1; ++c1) {
-                const int ca1 = a.conn_atoms[bt1 * a.s.C + c1];
-                const int pd1 = a.path_distance[(int64_t(bt1) * a.Am + ca1) * a.Am + r1];
-                for (int c2 = 0; c2 < it.nc2; ++c2) {
-                  const int ca2 = a.conn_atoms[it.bt2 * a.s.C + c2];
-                  const int pd2 = a.path_distance[(int64_t(it.bt2) * a.Am + ca2) * a.Am + r2];
-                  const int v = pd1 + conn_sep(a.s, g1, it.g2, c1, c2) + pd2;
+              for (int c2 = 0; c2 < it.nc2; ++c2) {
+                const int ca2 = a.conn_atoms[it.bt2 * a.s.C + c2];
+                const int pd2 = a.path_distance[(int64_t(it.bt2) * a.Am + ca2) * a.Am + r2];
+                for (int c1 = 0; c1 < rw.nc1; ++c1) {
+                  const int v = int((L.pd1[it.row][r1] >> (8 * c1)) & 255u) +
+                                int((it.cs[c1] >> (8 * c2)) & 255u) + pd2;
                   best = v < best ? v : best;
                 }
               }
@@ -568,6 +639,7 @@ __global__ __launch_bounds__(256, hb_waves_per_simd<MODE>()) void hb_score_kerne
             qh = int32_t(hg);
             qa = int32_t(ag);
             qt = dt | (at << 16);
+            qg = rw.g1;
             qb = it.g2;
           } else if (CENSUS) {
             ++n_cp;
@@ -579,29 +651,22 @@ __global__ __launch_bounds__(256, hb_waves_per_simd<MODE>()) void hb_score_kerne
           L.qh[e] = qh;
           L.qa[e] = qa;
           L.qt[e] = qt;
+          L.qg[e] = qg;
           L.qb[e] = qb;
         }
         tail += __popcll(mask);
-        if (tail - head >= WAVE) {
+        if (tail - head >= WAVE || (last && tail > head)) {
+          const int m = tail - head < WAVE ? tail - head : WAVE;
           wave_sync();
-          hb_phase_b<Real, MODE>(L, a, g1, head, WAVE, lane, w_row, esum, n_eval);
-          head += WAVE;
+          hb_phase_b<Real, MODE>(L, a, head, m, lane, en, n_eval);
+          head += m;
         }
       }
       wave_sync();
     }
-    while (tail > head) {
-      const int n = tail - head < WAVE ? tail - head : WAVE;
-      wave_sync();
-      hb_phase_b<Real, MODE>(L, a, g1, head, n, lane, w_row, esum, n_eval);
-      head += n;
-    }
     wave_sync();
-    if (!BP && !NOE && !CENSUS) {
-      const double v = wave_sum(esum.value());
-      if (lane == 0 && v != 0.0) atomicAdd(&a.energies64[pose], v);
-    }
   }
+  if (!BP && !NOE && !CENSUS) en.flush(a.energies64);
   if (CENSUS) {
     const unsigned long long c1 = wave_sum(n_cp), c2 = wave_sum(n_eval);
     if (lane == 0) {
