@@ -210,6 +210,16 @@ int tmol_ljlk_backward_combine(const void* dvdx, const void* grad_scores,
                                int32_t n_poses, int32_t dtype, void* grad,
                                void* stream);
 
+/* Totals of several terms under weights known at the forward pass: weights
+ * [T, P] = w[(t + first) % T] / scale for a weighted-gradient pass (scale: the
+ * power of two of the largest weight), and the gradient of the totals,
+ *   out[a, k] = up[atom_pose[a]] * scale * grad[a, k]. */
+int tmol_total_weights(const float* w, int32_t n_terms, int32_t first, int32_t n_poses,
+                       int32_t dtype, void* out, void* scale, void* stream);
+int tmol_total_backward(const void* grad, const void* up, const void* scale,
+                        const int32_t* atom_pose, int64_t n_atoms, int32_t dtype, void* out,
+                        void* stream);
+
 /* Copy the work-list counters to the host (synchronises the stream):
  *   counters_host[0] = block pairs found (including any beyond row capacity)
  *   counters_host[1] = row capacity overflow flag */

@@ -1233,6 +1233,44 @@ int tmol_ljlk_census(const tmol_ljlk_stack* s, const tmol_ljlk_block_types* bt,
   return check(hipGetLastError());
 }
 
+int tmol_total_weights(const float* w, int32_t n_terms, int32_t first, int32_t n_poses,
+                       int32_t dtype, void* out, void* scale, void* stream) {
+  if (!w || !out || !scale || n_terms <= 0 || n_terms > 4 || first < 0 || first >= n_terms ||
+      n_poses <= 0)
+    return TMOL_LJLK_EINVAL;
+  const unsigned nb = (unsigned)((int64_t(n_terms) * n_poses + 255) / 256);
+  hipStream_t st = (hipStream_t)stream;
+  if (dtype == TMOL_LJLK_F32)
+    hipLaunchKernelGGL(total_weights_kernel<float>, dim3(nb), dim3(256), 0, st, w, n_terms, first,
+                       n_poses, (float*)out, (float*)scale);
+  else if (dtype == TMOL_LJLK_F64)
+    hipLaunchKernelGGL(total_weights_kernel<double>, dim3(nb), dim3(256), 0, st, w, n_terms, first,
+                       n_poses, (double*)out, (double*)scale);
+  else
+    return TMOL_LJLK_EINVAL;
+  return check(hipGetLastError());
+}
+
+int tmol_total_backward(const void* grad, const void* up, const void* scale,
+                        const int32_t* atom_pose, int64_t n_atoms, int32_t dtype, void* out,
+                        void* stream) {
+  if (!grad || !up || !scale || !atom_pose || !out || n_atoms < 0) return TMOL_LJLK_EINVAL;
+  if (n_atoms == 0) return TMOL_LJLK_OK;
+  const unsigned nb = (unsigned)((n_atoms * 3 + 255) / 256);
+  hipStream_t st = (hipStream_t)stream;
+  if (dtype == TMOL_LJLK_F32)
+    hipLaunchKernelGGL(total_backward_kernel<float>, dim3(nb), dim3(256), 0, st,
+                       (const float*)grad, (const float*)up, (const float*)scale, atom_pose,
+                       n_atoms, (float*)out);
+  else if (dtype == TMOL_LJLK_F64)
+    hipLaunchKernelGGL(total_backward_kernel<double>, dim3(nb), dim3(256), 0, st,
+                       (const double*)grad, (const double*)up, (const double*)scale, atom_pose,
+                       n_atoms, (double*)out);
+  else
+    return TMOL_LJLK_EINVAL;
+  return check(hipGetLastError());
+}
+
 int tmol_ljlk_backward_combine(const void* dvdx, const void* grad_scores,
                                const int32_t* atom_pose, int64_t n_atoms, int32_t n_poses,
                                int32_t dtype, void* grad, void* stream) {

@@ -385,6 +385,46 @@ __global__ void combine_kernel(const Real* __restrict__ dvdx, const Real* __rest
   grad[i] = v;
 }
 
+// Weights of a pose's total as the weighted-gradient pass takes them: out
+// [T, P] = w[(t + first) % T] / scale, scale the power of two that brings the
+// largest weight into [1, 2).  The pass sums in fixed point, whose range and
+// resolution suit contributions of weight about 1; dividing by a power of two
+// changes no digit.  A weight that is not finite makes the scale (and with it
+// the gradient) NaN.
+template <typename Real>
+__global__ __launch_bounds__(256) void total_weights_kernel(const float* __restrict__ w,
+                                                            int n_terms, int first, int n_poses,
+                                                            Real* __restrict__ out,
+                                                            Real* __restrict__ scale) {
+  float m = 0.0f;
+  bool finite = true;
+  for (int t = 0; t < n_terms; ++t) {
+    finite = finite && isfinite(w[t]);
+    m = fmaxf(m, fabsf(w[t]));
+  }
+  // ilogb of the smallest subnormal is -149: 2^149 and its inverse need the
+  // double range for the division
+  const int e = finite && m > 0.0f ? ilogbf(m) : 0;
+  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i == 0) scale[0] = finite ? Real(ldexp(1.0, e)) : Real(__builtin_nanf(""));
+  if (i >= int64_t(n_terms) * n_poses) return;
+  const int t = int(i / n_poses);
+  out[i] = Real(ldexp(double(w[(t + first) % n_terms]), -e));
+}
+
+// gradient of the poses' totals: out[a, k] = up[pose(a)] scale grad[a, k]
+template <typename Real>
+__global__ __launch_bounds__(256) void total_backward_kernel(const Real* __restrict__ grad,
+                                                             const Real* __restrict__ up,
+                                                             const Real* __restrict__ scale,
+                                                             const int32_t* __restrict__ atom_pose,
+                                                             int64_t n_atoms,
+                                                             Real* __restrict__ out) {
+  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= n_atoms * 3) return;
+  out[i] = up[atom_pose[i / 3]] * scale[0] * grad[i];
+}
+
 // Count-pair separations of listed block pairs (first tiles), computed with
 // the scoring kernels' count-pair function (one wave per item).
 __global__ __launch_bounds__(64) void debug_sep_kernel(StackView s, BTView bt,

@@ -25,6 +25,7 @@ import threading
 from typing import List, Optional
 
 import torch
+from torch.autograd.function import once_differentiable
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libtmol_ljlk_hip.so")
@@ -129,6 +130,12 @@ def lib():
             ]
             L.tmol_ljlk_backward_combine.argtypes = [
                 _VP, _VP, _VP, ctypes.c_int64, ctypes.c_int32, ctypes.c_int32, _VP, _VP,
+            ]
+            L.tmol_total_weights.argtypes = [
+                _VP, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, _VP, _VP, _VP,
+            ]
+            L.tmol_total_backward.argtypes = [
+                _VP, _VP, _VP, _VP, ctypes.c_int64, ctypes.c_int32, _VP, _VP,
             ]
             L.tmol_ljlk_read_counters.argtypes = [_VP, ctypes.POINTER(ctypes.c_int64), _VP]
             L.tmol_ljlk_work_list.argtypes = [
@@ -438,10 +445,7 @@ def _(rot_coords, rot_coord_offset, pose_ind_for_atom, first_rot_for_block, *res
     return [score, nbr, dv]
 
 
-@torch.library.custom_op("tmol_amd::ljlk_backward_combine", mutates_args=())
-def ljlk_backward_combine(dV_dx: torch.Tensor, grad_score: torch.Tensor,
-                          pose_ind_for_atom: torch.Tensor) -> torch.Tensor:
-    """grad[a] = sum_t grad_score[t, pose(a)] * dV_dx[t, a] (hand-written kernel)."""
+def _backward_combine(dV_dx, grad_score, pose_ind_for_atom):
     _require_device(dV_dx)
     dev = dV_dx.device
     NA = dV_dx.shape[1]
@@ -452,6 +456,23 @@ def ljlk_backward_combine(dV_dx: torch.Tensor, grad_score: torch.Tensor,
                                             gs.shape[1], _dtype_code(dV_dx.dtype), _p(grad),
                                             _stream(dev)), "backward combine")
     return grad
+
+
+def _block_pair_backward(grad_score, args):
+    coords = args[0]
+    call = PaddedCall(args, coords.dtype)
+    call.neighbors(None)
+    grad = torch.empty_like(call.coords)
+    w = grad_score.to(coords.dtype).contiguous()
+    call.score(BLOCK_PAIR | WGRAD | NO_ENERGY, weights=w, grad=grad)
+    return grad
+
+
+@torch.library.custom_op("tmol_amd::ljlk_backward_combine", mutates_args=())
+def ljlk_backward_combine(dV_dx: torch.Tensor, grad_score: torch.Tensor,
+                          pose_ind_for_atom: torch.Tensor) -> torch.Tensor:
+    """grad[a] = sum_t grad_score[t, pose(a)] * dV_dx[t, a] (hand-written kernel)."""
+    return _backward_combine(dV_dx, grad_score, pose_ind_for_atom)
 
 
 @ljlk_backward_combine.register_fake
@@ -487,12 +508,7 @@ def ljlk_block_pair_backward(
             block_type_atom_types, block_type_n_interblock_bonds,
             block_type_atoms_forming_chemical_bonds, block_type_path_distance,
             block_type_is_ligand_fragment, type_params, global_params, max_dis, True)
-    call = PaddedCall(args, rot_coords.dtype)
-    call.neighbors(None)
-    grad = torch.empty_like(call.coords)
-    w = grad_score.to(rot_coords.dtype).contiguous()
-    call.score(BLOCK_PAIR | WGRAD | NO_ENERGY, weights=w, grad=grad)
-    return grad
+    return _block_pair_backward(grad_score, args)
 
 
 @ljlk_block_pair_backward.register_fake
@@ -590,7 +606,153 @@ def ljlk_pose_scores(*args):
     ``[score, block_neighbors]``."""
     if len(args) != 27:
         raise TypeError("ljlk_pose_scores takes 27 arguments (%d given)" % len(args))
+    if _plain_call(args) and args[0].is_cuda:
+        require = args[0].requires_grad and torch.is_grad_enabled() and not args[-1]
+        return list(LJLKPoseScoreFunction.apply(require, *args))
     return torch.ops.tmol_ljlk.ljlk_pose_scores(*args)
+
+
+def _plain_call(args) -> bool:
+    """An eager call of plain tensors that only autograd has to see: nothing
+    compiles, traces, transforms or intercepts it, so the registered op's
+    dispatch (0.4 ms of host time per forward of a 27-argument op, the
+    larger part of a small pose's call) would reach the same kernels."""
+    if (torch.compiler.is_compiling() or torch.jit.is_tracing()
+            or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0):
+        return False
+    for a in args:
+        t = type(a)
+        if t is torch.Tensor or t is torch.nn.Parameter:
+            if torch._is_functional_tensor(a):
+                return False
+        elif t is not int and t is not float and t is not bool:
+            return False
+    # the schema's scalars: int max_n_rots_per_pose, float max_dis, bool block pairs
+    return type(args[12]) is int and type(args[-2]) is not bool and type(args[-1]) is bool
+
+
+class LJLKPoseScoreFunction(torch.autograd.Function):
+    """The eager form of the op and its registered autograd: whole-pose mode
+    saves dV/dx and pose_ind_for_atom, block-pair mode re-walks the neighbor
+    list (compiled.ops.cpp:29-279)."""
+
+    @staticmethod
+    def forward(ctx, require, *args):
+        ctx.set_materialize_grads(False)
+        score, nbr, dvdx, call = _forward_impl(args, require)
+        ctx.mark_non_differentiable(nbr)
+        ctx.n_args = len(args) + 1
+        ctx.block_pair = call.block_pair
+        if call.block_pair:
+            ctx.args = args[1:]
+            ctx.save_for_backward(args[0])
+        else:
+            ctx.save_for_backward(dvdx, args[2])
+        return score, nbr
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, grad_score, grad_nbr):
+        none = (None,) * ctx.n_args
+        if grad_score is None:
+            return none
+        if ctx.block_pair:
+            (coords,) = ctx.saved_tensors
+            grad = _block_pair_backward(grad_score, (coords,) + ctx.args)
+        else:
+            dvdx, atom_pose = ctx.saved_tensors
+            if dvdx is None:
+                return none
+            grad = _backward_combine(dvdx, grad_score, atom_pose)
+        return (None, grad) + none[2:]
+
+
+class WholePoseTotalFunction(torch.autograd.Function):
+    """sum_t w_t V_t per pose of LJ+LK (t = atr, rep, lk) and, with elec's
+    argument tail, elec: one neighbor pass and one scoring pass that also
+    takes the weighted gradient, which the backward scales by each pose's
+    incoming gradient.  The weights are known at the forward pass, so per-term
+    derivatives need not be kept.  elec_first: the weights' first row is
+    elec's."""
+
+    @staticmethod
+    def forward(ctx, coords, weights, tail, elec_tail, elec_first, require):
+        ctx.set_materialize_grads(False)
+        dtype, dev = coords.dtype, coords.device
+        call = PaddedCall((coords,) + tail, dtype)
+        elec = None
+        if elec_tail is not None:
+            (_, _, n_atoms, charge, n_conn, conn_atoms, inter_rpd, intra_rpd, is_ligand,
+             global_params, _) = elec_tail
+            elec = ElecTypeTables(n_atoms, n_conn, conn_atoms, is_ligand, charge, inter_rpd,
+                                  intra_rpd, global_params, dtype, dev)
+        T, P = (4 if elec else 3), call.P
+        stream = _stream(dev)
+        call.neighbors(None)
+        energies = torch.empty((T, P), dtype=dtype, device=dev)
+        w = torch.empty((T * P + 1,), dtype=dtype, device=dev)  # [T, P], then the scale
+        scale = w[T * P:]
+        _check(lib().tmol_total_weights(_p(weights), T, 1 if elec_first else 0, P, call.dcode,
+                                        _p(w), _p(scale), stream), "total weights")
+        grad = torch.empty_like(call.coords) if require else None
+        flags = WGRAD if require else 0
+        if elec:
+            L = _elec_lib()
+            where = (ctypes.byref(call.cstack), ctypes.byref(call.bt.c), ctypes.byref(elec.celec))
+            ws = (_p(call.ws.buf), call.ws.nbytes, call.ws.capacity)
+            _check(L.tmol_ljlk_elec_prepare(*where, *ws, call.dcode, stream), "elec prepare")
+            _check(L.tmol_ljlk_elec_score(*where, _p(call.coords), call.dcode, *ws, flags, _p(w),
+                                          _p(energies), _p(grad), 0, stream), "ljlk+elec score")
+        else:
+            call.score(flags, weights=w, energies=energies, grad=grad)
+        ctx.save_for_backward(grad, scale, call.keep["atom_pose"])
+        order = weights.roll(-1, 0) if elec_first else weights
+        return (order * energies).sum(dim=0)
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, grad_total):
+        grad, scale, atom_pose = ctx.saved_tensors
+        if grad_total is None or grad is None:
+            return (None,) * 6
+        up = grad_total.to(grad.dtype).contiguous()
+        out = torch.empty_like(grad)
+        _check(lib().tmol_total_backward(_p(grad.contiguous()), _p(up), _p(scale.contiguous()),
+                                         _p(atom_pose.contiguous()), grad.shape[0],
+                                         _dtype_code(grad.dtype), _p(out), _stream(grad.device)),
+               "total backward")
+        return (out,) + (None,) * 5
+
+
+def whole_pose_total(coords, weights, tail, elec_tail=None, elec_first=False):
+    """[P] weighted totals (``WholePoseTotalFunction``), or None where the
+    terms have to be scored one by one: block types above 32 atoms, terms of
+    other pose stacks, an elec reach beyond LJ+LK's work list, weights that
+    are not one plain float32 number per term (or need a gradient), or a
+    call that more than autograd has to see."""
+    args = (coords,) + tail
+    n_terms = 3 if elec_tail is None else 4
+    if not (_plain_call(args) and coords.is_cuda and coords.dim() == 2
+            and type(weights) in (torch.Tensor, torch.nn.Parameter)
+            and tuple(weights.shape) == (n_terms, 1) and weights.dtype == torch.float32
+            and weights.device == coords.device and weights.is_contiguous()
+            and not weights.requires_grad and not tail[-1] and tail[17].shape[1] <= 32):
+        return None
+    if elec_tail is not None:
+        common, terms = elec_tail[:12], elec_tail[12:-1]
+        # LJ+LK's places of elec's stack and block-type tables
+        shared = (tail[12], tail[13], tail[14], tail[18], tail[19], tail[21])
+        if not (_plain_call((coords,) + elec_tail)
+                and all(a is b for a, b in zip(common, tail[:12]) if torch.is_tensor(a))
+                and all(a is terms[i] for a, i in zip(shared, (0, 1, 2, 4, 5, 8)))
+                and terms[10] <= tail[24] and not elec_tail[-1]):
+            return None
+    else:
+        terms = None
+    require = coords.requires_grad and torch.is_grad_enabled()
+    return WholePoseTotalFunction.apply(coords, weights, tail, terms, elec_first, require)
 
 
 def debug_pair_separations(args, items: torch.Tensor) -> torch.Tensor:

@@ -126,13 +126,11 @@ class ElecEnergyTerm:
             q[i, :n] = qi
             inter[i, :n, :n] = ei
             intra[i, :n, :n] = ai
-        lig = numpy.array([int(bt.is_ligand_fragment) for bt in pbt.active_block_types],
-                          dtype=numpy.int32)
         cache = {
             "partial_charge": torch.tensor(q, device=pbt.device),
             "inter_repr_path_distance": torch.tensor(inter, device=pbt.device),
             "intra_repr_path_distance": torch.tensor(intra, device=pbt.device),
-            "is_ligand_fragment": torch.tensor(lig, device=pbt.device),
+            "is_ligand_fragment": pbt.ljlk_is_ligand_fragment,
         }
         pbt._elec_tables = cache
         return cache

@@ -5,7 +5,9 @@ their creation order, and each contributes its score types in its own order.
 """
 
 import torch
+from torch.nn.modules.module import _has_any_global_hook as _any_global_hook
 
+from ..ops import whole_pose_total
 from .elec_energy_term import ElecEnergyTerm
 from .ljlk_energy_term import LJLKEnergyTerm
 from .score_types import ScoreType
@@ -58,7 +60,12 @@ class ScoreFunction:
     def render_whole_pose_scoring_module(self, pose_stack):
         self.pre_work_initialization(pose_stack)
         mods = [t.render_whole_pose_scoring_module(pose_stack) for t in self.all_terms()]
-        return WholePoseScoringModule(self.weights_tensor(), mods)
+        module = WholePoseScoringModule(self.weights_tensor(), mods)
+        kinds = [type(t) for t in self.all_terms()]
+        if kinds in ([LJLKEnergyTerm], [LJLKEnergyTerm, ElecEnergyTerm],
+                     [ElecEnergyTerm, LJLKEnergyTerm]):
+            module._one_pass = dict(zip(kinds, mods))
+        return module
 
     def render_block_pair_scoring_module(self, pose_stack):
         self.pre_work_initialization(pose_stack)
@@ -79,14 +86,35 @@ class WholePoseScoringModule:
     def __init__(self, weights, term_modules):
         self.weights = torch.nn.Parameter(weights.unsqueeze(1), requires_grad=False)
         self.term_modules = term_modules
+        self._one_pass = None  # the modules of terms that one pass can score together
 
     def __call__(self, coords, sum_terms=True, apply_weights=True):
+        if sum_terms and apply_weights and self._one_pass:
+            total = self._total(coords)
+            if total is not None:
+                return total
         unweighted = self.unweighted_scores(coords)
         weighted = self.weights * unweighted if apply_weights else unweighted
         return torch.sum(weighted, dim=0) if sum_terms else weighted
 
     def unweighted_scores(self, coords):
         return torch.cat([term(coords) for term in self.term_modules], dim=0)
+
+    def _total(self, coords):
+        """The weighted sum from one pass over all terms, or None where the
+        terms have to be called one by one.  Separate passes keep dV/dx of
+        every term for weights that come with the backward; a total's weights
+        are known here."""
+        mods = list(self.term_modules)
+        if (type(self) is not WholePoseScoringModule or "unweighted_scores" in self.__dict__
+                or len(mods) != len(self._one_pass) or _any_global_hook()
+                or any(m is not q or not m.is_plain()
+                       for m, q in zip(mods, self._one_pass.values()))):
+            return None
+        f64 = coords.dtype == torch.float64
+        lj, elec = self._one_pass[LJLKEnergyTerm], self._one_pass.get(ElecEnergyTerm)
+        return whole_pose_total(coords.flatten(start_dim=0, end_dim=-2), self.weights,
+                                lj.tail(f64), elec.tail(f64) if elec else None, mods[0] is elec)
 
 
 class BlockPairScoringModule:

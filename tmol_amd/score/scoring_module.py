@@ -36,10 +36,19 @@ class TermPoseScoringModule(torch.nn.Module):
         self.n_poses = ps.first_rot_for_block.shape[0]
         self.max_n_blocks = ps.first_rot_for_block.shape[1]
 
+    def tail(self, f64):
+        return self._tail_f64 if f64 else self._tail_f32
+
+    def is_plain(self):
+        """Called as it was rendered: no hook or replaced forward that a
+        caller scoring the term by other means would pass by."""
+        return (type(self) is TermWholePoseScoringModule and "forward" not in self.__dict__
+                and not (self._forward_hooks or self._forward_pre_hooks or self._backward_hooks
+                         or self._backward_pre_hooks))
+
     def forward(self, coords):
         flat = coords.flatten(start_dim=0, end_dim=-2)
-        tail = self._tail_f64 if coords.dtype == torch.float64 else self._tail_f32
-        scores, _ = self.term_score_poses(flat, *tail)
+        scores, _ = self.term_score_poses(flat, *self.tail(coords.dtype == torch.float64))
         return scores
 
 
