@@ -737,6 +737,13 @@ typedef struct {
   const void* bt_atom_icoors_backup;          /* [T, Amax, 3] */
 } tmol_leaf_atoms_args;
 
+/* Bits of *failed (device, zeroed by the caller) for the tables that index
+ * outside one another (T = n_block_types): 1 block_type, 2 bt_n_atoms,
+ * 4 downstream, 8 / 16 ancestors / backup ancestors, 32 connections, 64 block
+ * offsets, 128 connections naming a padding block. */
+int tmol_leaf_atoms_check(const tmol_leaf_atoms_args* args, int32_t n_block_types,
+                          uint32_t* failed, void* stream);
+
 /* new_coords [P, NA, 3] from orig_coords [P, NA, 3]. */
 int tmol_leaf_atoms_build(const tmol_leaf_atoms_args* args, const void* orig_coords,
                           int32_t dtype, void* new_coords, void* stream);

@@ -211,3 +211,40 @@ def test_pose_stack_from_pdb(co):
         co, *ingest.canonical_form_from_pdb(_pdb("1ubq.pdb"), co)))
     for b in range(1, 29):
         assert numpy.allclose(ps.poses[0].coords[b], full.poses[0].coords[b + 10], atol=1e-4)
+
+
+@pytest.mark.parametrize("key,value", [
+    ("btype", "T"), ("btype", -2), ("bt_n", "A1"), ("bt_n", -1), ("down", "n"), ("down", -2),
+    ("anc0", "n"), ("anc1", "C"), ("anc2", "A"), ("anc_b0", -2), ("anc_b1", -2), ("irc0", "B"),
+    ("irc0", -2), ("irc1", "C"), ("boff", "NA"), ("boff", -1), ("pad", 0)])
+@pytest.mark.parametrize("at", [0, -1])
+def test_table_check_equals_the_tensor_checks(co, key, value, at):
+    """One table entry out of range, first or last of its table: the kernel's
+    check raises what the tensor form of the checks raises on the host."""
+    _, args = _random_missing(co, torch.float64)
+    keys = ("orig", "bmiss", "pmiss", "boff", "btype", "irc", "bt_n", "down", "anc",
+            "geom", "anc_b", "geom_b")
+    k = {n: (torch.as_tensor(t).clone()) for n, t in zip(keys, args)}
+    P, NA = k["orig"].shape[:2]
+    B, A = k["bmiss"].shape[1:]
+    C, T = k["irc"].shape[2], k["bt_n"].shape[0]
+    name = key.rstrip("012")
+    v = {"T": T, "A1": A + 1, "n": A, "A": A, "C": C, "B": B, "NA": NA}.get(value, value)
+    if key == "pad":  # a connection to a block that does not exist
+        pose = int((k["btype"] < 0).any(dim=1).nonzero()[0, 0])
+        k["irc"][pose, 0, 0, 0] = int((k["btype"][pose] < 0).nonzero()[at, 0])
+        k["irc"][pose, 0, 0, 1] = 0
+    elif key == "boff":
+        b = (k["btype"].view(-1) >= 0).nonzero()[at, 0]
+        k["boff"].view(-1)[b] = v
+    elif key[-1] in "012":
+        row = k[name].view(-1, k[name].shape[-1])[at]
+        row[1 if key.startswith("anc") and key[-1] == "2" else 0] = 0
+        row[int(key[-1])] = v
+    else:
+        k[name].view(-1)[at] = v
+    with pytest.raises(ingest.ops.LJLKLibraryError) as want:
+        ingest._validate_leaf_tables(k, P, NA, B, A, C)
+    with pytest.raises(ingest.ops.LJLKLibraryError) as got:
+        ingest.gen_pose_leaf_atoms(*[k[n].cuda() for n in keys])
+    assert str(got.value) == str(want.value)

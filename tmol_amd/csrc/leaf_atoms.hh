@@ -28,6 +28,58 @@ struct LeafArgs {
   const void* geom_backup;
 };
 
+// Bits of *failed, in the order the host reports them: every index that the
+// kernels below follow lies inside its table.  The last two index with values
+// that the first ones check, so they are tested only where those are sound
+// (and reported only when none of the first failed).
+//
+// Bound by the two launches and the read-back of one word: the tables of
+// 256 poses of 50-600 residues are 5 MB, read once.  The same checks as
+// elementwise tensor operations took 60 launches, 300 us of device time and
+// two read-backs per call.
+constexpr uint32_t LEAF_BAD_TYPE = 1, LEAF_BAD_N = 2, LEAF_BAD_DOWN = 4, LEAF_BAD_ANC = 8,
+                   LEAF_BAD_CONN = 32, LEAF_BAD_OFFSET = 64, LEAF_BAD_PARTNER = 128;
+
+__device__ __forceinline__ bool leaf_outside(int v, int lo, int n) { return v < lo || v >= n; }
+
+__global__ __launch_bounds__(256) void leaf_check_kernel(LeafArgs a, int T, uint32_t* failed) {
+  const int64_t i0 = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int64_t step = int64_t(gridDim.x) * blockDim.x;
+  uint32_t bad = 0;
+  for (int64_t t = i0; t < T; t += step)
+    if (leaf_outside(a.n_atoms[t], 0, a.Amax + 1)) bad |= LEAF_BAD_N;
+  for (int64_t i = i0; i < int64_t(T) * a.C * a.Amax; i += step)
+    if (leaf_outside(a.downstream[i], -1, a.n_atoms[i / (int64_t(a.C) * a.Amax)]))
+      bad |= LEAF_BAD_DOWN;
+  for (int64_t i = i0; i < int64_t(T) * a.Amax * 3; i += step) {
+    const int n = a.n_atoms[i / (int64_t(a.Amax) * 3)];
+    for (int k = 0; k < 2; ++k) {
+      const int32_t* u = (k ? a.anc_backup : a.anc) + 3 * i;
+      if (leaf_outside(u[0], -1, n) || leaf_outside(u[1], -1, a.C) ||
+          (u[1] >= 0 && leaf_outside(u[2], 0, a.Amax)))
+        bad |= LEAF_BAD_ANC << k;
+    }
+  }
+  for (int64_t q = i0; q < int64_t(a.P) * a.B; q += step) {
+    const int bt = a.block_type[q];
+    if (leaf_outside(bt, -1, T)) {
+      bad |= LEAF_BAD_TYPE;
+    } else if (bt >= 0) {
+      const int off = a.block_offset[q];
+      if (off < 0 || int64_t(off) + a.n_atoms[bt] > a.NA) bad |= LEAF_BAD_OFFSET;
+    }
+    const int32_t* row = a.block_type + (q / a.B) * a.B;
+    for (int c = 0; c < a.C; ++c) {
+      const int ob = a.irc[(q * a.C + c) * 2], oc = a.irc[(q * a.C + c) * 2 + 1];
+      if (leaf_outside(ob, -1, a.B) || (ob >= 0 && leaf_outside(oc, 0, a.C)))
+        bad |= LEAF_BAD_CONN;
+      else if (ob >= 0 && row[ob] < 0)
+        bad |= LEAF_BAD_PARTNER;
+    }
+  }
+  if (bad) atomicOr(failed, bad);
+}
+
 // pose-wide index of an unresolved atom id of block b (-1: none)
 __device__ __forceinline__ int leaf_resolve(const LeafArgs& a, int p, int b, const int32_t* u) {
   if (u[0] != -1) return a.block_offset[p * a.B + b] + u[0];
@@ -296,9 +348,9 @@ __global__ __launch_bounds__(LEAF_WAVE) void leaf_atoms_backward_remote_kernel(
         for (int j = 0; j < 3; ++j) {
           if (slot[j] >= 0) continue;
           Real* d = dorig + 3 * (base + anc[j]);
-          atomicAdd(&d[0], gs[j].x);
-          atomicAdd(&d[1], gs[j].y);
-          atomicAdd(&d[2], gs[j].z);
+          unsafeAtomicAdd(&d[0], gs[j].x);
+          unsafeAtomicAdd(&d[1], gs[j].y);
+          unsafeAtomicAdd(&d[2], gs[j].z);
         }
       }
     }

@@ -2046,6 +2046,19 @@ static unsigned leaf_grid(const LeafArgs& a) {
   return (unsigned)std::max<int64_t>(1, std::min<int64_t>(waves, 65536));
 }
 
+int tmol_leaf_atoms_check(const tmol_leaf_atoms_args* x, int32_t n_block_types, uint32_t* failed,
+                          void* stream) {
+  LeafArgs a;
+  int v = leaf_args(x, TMOL_LJLK_F32, a);
+  if (v) return v;
+  if (n_block_types < 0 || !failed) return TMOL_LJLK_EINVAL;
+  const int64_t n = std::max({int64_t(a.P) * a.B, int64_t(n_block_types) * a.C * a.Amax,
+                              int64_t(n_block_types) * a.Amax * 3});
+  hipLaunchKernelGGL(leaf_check_kernel, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 1024)),
+                     dim3(256), 0, (hipStream_t)stream, a, (int)n_block_types, failed);
+  return check(hipGetLastError());
+}
+
 int tmol_leaf_atoms_build(const tmol_leaf_atoms_args* x, const void* orig, int32_t dtype,
                           void* out, void* stream) {
   LeafArgs a;

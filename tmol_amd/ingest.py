@@ -220,59 +220,70 @@ def _leaf_lib():
         if not _bound:
             A = ctypes.POINTER(CLeafArgs)
             V = ctypes.c_void_p
+            L.tmol_leaf_atoms_check.argtypes = [A, ctypes.c_int32, V, V]
             L.tmol_leaf_atoms_build.argtypes = [A, V, ctypes.c_int32, V, V]
             L.tmol_leaf_atoms_backward.argtypes = [A, V, ctypes.c_int32, V, V, V]
             _bound = True
     return L
 
 
-def _failed(checks):
-    """The messages of the checks whose condition holds anywhere; the
-    conditions are reduced on their device and read back together (one
-    synchronization)."""
-    if not checks:
-        return []
-    flags = torch.stack([c.any() for _, c in checks]).tolist()
-    return [m for (m, _), f in zip(checks, flags) if f]
+# the checks of tmol_leaf_atoms_check by bit; the last two are reported when
+# none of the others failed
+_RANGE_CHECKS = (
+    "block_type outside [-1, n_block_types)",
+    "bt_n_atoms outside [0, max_n_block_atoms]",
+    "atom_downstream_of_conn outside [-1, n_atoms of its block type)",
+    "anc outside the block-type tables",
+    "anc_b outside the block-type tables",
+    "inter_block_connections outside [0, max_n_blocks) x [0, max_n_conn)",
+)
+_INDEXED_CHECKS = (
+    "block_coord_offset + n_atoms outside the pose",
+    "inter_block_connections naming a padding block",
+)
+
+
+def _failed(messages, conditions):
+    """The messages of the conditions that hold anywhere."""
+    return [m for m, c in zip(messages, conditions) if bool(c.any())]
 
 
 def _validate_leaf_tables(k, P, NA, B, Amax, C):
     """Every index the kernels follow stays inside its table: block types,
     block offsets plus sizes inside the pose, connection partners, ancestor
-    ids and the downstream atoms.  Two read-backs: the range checks, then
-    the checks that index with the values the first ones cleared."""
+    ids and the downstream atoms: the range checks, then the checks that
+    index with the values the first ones cleared.  Tables on the device are
+    tested by ``_LeafCall.check`` in one kernel and one read-back."""
     T = int(k["bt_n"].shape[0])
     bt = k["btype"]
     if tuple(k["down"].shape) != (T, C, Amax) or tuple(k["anc"].shape) != (T, Amax, 3, 3) \
             or tuple(k["anc_b"].shape) != (T, Amax, 3, 3) \
             or tuple(k["geom"].shape) != (T, Amax, 3) or tuple(k["geom_b"].shape) != (T, Amax, 3):
         raise ops.LJLKLibraryError("leaf-atom op: block-type table shapes")
+    if int(k["boff"].numel()) != P * B or (C > 0 and tuple(k["irc"].shape) != (P, B, C, 2)):
+        raise ops.LJLKLibraryError("leaf-atom op: inconsistent pose shapes")
+    if bt.is_cuda:
+        return
     n_of_type = k["bt_n"].view(T, 1, 1)
-    checks = [("block_type outside [-1, n_block_types)", (bt < -1) | (bt >= T)),
-              ("bt_n_atoms outside [0, max_n_block_atoms]", (k["bt_n"] < 0) | (k["bt_n"] > Amax)),
-              ("atom_downstream_of_conn outside [-1, n_atoms of its block type)",
-               (k["down"] < -1) | (k["down"] >= n_of_type))]
+    checks = [(bt < -1) | (bt >= T), (k["bt_n"] < 0) | (k["bt_n"] > Amax),
+              (k["down"] < -1) | (k["down"] >= n_of_type)]
     for key in ("anc", "anc_b"):
         u = k[key]
-        checks.append(("%s outside the block-type tables" % key,
-                       (u[..., 0] < -1) | (u[..., 0] >= n_of_type) | (u[..., 1] < -1)
-                       | (u[..., 1] >= C) | ((u[..., 1] >= 0) & ((u[..., 2] < 0) | (u[..., 2] >= Amax)))))
+        checks.append((u[..., 0] < -1) | (u[..., 0] >= n_of_type) | (u[..., 1] < -1)
+                      | (u[..., 1] >= C) | ((u[..., 1] >= 0) & ((u[..., 2] < 0) | (u[..., 2] >= Amax))))
     if C > 0:
         ob, oc = k["irc"][..., 0], k["irc"][..., 1]
-        checks.append(("inter_block_connections outside [0, max_n_blocks) x [0, max_n_conn)",
-                       (ob < -1) | (ob >= B) | ((ob >= 0) & ((oc < 0) | (oc >= C)))))
-    bad = _failed(checks)
+        checks.append((ob < -1) | (ob >= B) | ((ob >= 0) & ((oc < 0) | (oc >= C))))
+    bad = _failed(_RANGE_CHECKS, checks)
     if not bad:
         real = bt >= 0
         n = torch.where(real, k["bt_n"][bt.clamp(min=0).long()], torch.zeros_like(bt))
-        checks = [("block_coord_offset + n_atoms outside the pose",
-                   real & ((k["boff"] < 0) | (k["boff"] + n > NA)))]
+        checks = [real & ((k["boff"] < 0) | (k["boff"] + n > NA))]
         if C > 0:
             ob = k["irc"][..., 0]
             partner = bt.gather(1, ob.clamp(min=0).view(P, -1).long()).view(ob.shape)
-            checks.append(("inter_block_connections naming a padding block",
-                           (ob >= 0) & (partner < 0)))
-        bad = _failed(checks)
+            checks.append((ob >= 0) & (partner < 0))
+        bad = _failed(_INDEXED_CHECKS, checks)
     if bad:
         raise ops.LJLKLibraryError("leaf-atom op: " + "; ".join(bad))
 
@@ -288,7 +299,10 @@ class _LeafCall:
         P2, B, Amax = (int(x) for x in bmiss.shape)
         if P2 != P or tuple(pmiss.shape) != (P, NA) or tuple(btype.shape) != (P, B):
             raise ops.LJLKLibraryError("leaf-atom op: inconsistent pose shapes")
-        u8 = lambda t: t.to(device=dev, dtype=torch.uint8).contiguous()  # noqa: E731
+        def u8(t):  # a bool is a byte of 0 or 1 already
+            t = t.to(device=dev).contiguous()
+            return t.view(torch.uint8) if t.dtype == torch.bool else t.to(torch.uint8)
+
         i32 = lambda t: ops._i32(torch.as_tensor(t), dev)  # noqa: E731
         f = lambda t: torch.as_tensor(t).to(device=dev, dtype=orig.dtype).contiguous()  # noqa
         self.keep = dict(bmiss=u8(bmiss), pmiss=u8(pmiss), boff=i32(boff), btype=i32(btype),
@@ -311,6 +325,19 @@ class _LeafCall:
         self.orig = orig.contiguous()
         self.dcode = ops._dtype_code(orig.dtype)
         self.device = dev
+        self.check(int(k["bt_n"].shape[0]))
+
+    def check(self, n_types):
+        failed = torch.zeros(1, dtype=torch.int32, device=self.device)
+        ops._check(_leaf_lib().tmol_leaf_atoms_check(
+            ctypes.byref(self.cargs), n_types, ops._p(failed), ops._stream(self.device)),
+            "leaf atoms check")
+        bits = failed.item()
+        n = len(_RANGE_CHECKS)
+        bad = [m for i, m in enumerate(_RANGE_CHECKS) if bits >> i & 1] or \
+            [m for i, m in enumerate(_INDEXED_CHECKS) if bits >> (n + i) & 1]
+        if bad:
+            raise ops.LJLKLibraryError("leaf-atom op: " + "; ".join(bad))
 
     def build(self):
         out = torch.empty_like(self.orig)
