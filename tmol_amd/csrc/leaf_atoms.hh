@@ -93,29 +93,64 @@ __device__ __forceinline__ int leaf_resolve(const LeafArgs& a, int p, int b, con
   return a.block_offset[p * a.B + ob] + idx;
 }
 
-// the three ancestors and geometry (phi, theta, d) of atom slot `at` of a
-// block of type bt: the primary set, else the backup, else none (false)
+// a row of an ancestor table: three atom ids (atom, conn, bonds from conn),
+// loaded whole (two 16-byte loads and one word instead of nine words)
+struct LeafRow {
+  int32_t v[9];
+  // an ancestor named across a connection
+  __device__ __forceinline__ bool remote() const {
+    return (v[0] == -1 && v[1] != -1) || (v[3] == -1 && v[4] != -1) || (v[6] == -1 && v[7] != -1);
+  }
+};
+__device__ __forceinline__ LeafRow leaf_row(const int32_t* table, int64_t row) {
+  LeafRow r;
+  __builtin_memcpy(&r, table + row * 9, sizeof r);
+  return r;
+}
+
+// the three ancestors (pose-local indices) of atom slot `at` of a block of
+// type bt, for each its atom slot in the same block or -1 when named across a
+// connection, and the geometry (phi, theta, d): the primary set, else the
+// backup, else none (false)
 template <typename Real>
-__device__ __forceinline__ bool leaf_ancestors(const LeafArgs& a, int p, int b, int bt, int at,
-                                               int* anc, Real* geom) {
-  const int64_t row = int64_t(bt) * a.Amax + at;
-  const int32_t* sets[2] = {a.anc + row * 9, a.anc_backup + row * 9};
-  const Real* geoms[2] = {(const Real*)a.geom + row * 3, (const Real*)a.geom_backup + row * 3};
+__device__ __forceinline__ bool leaf_ancestors(const LeafArgs& a, int p, int b, int64_t row,
+                                               const LeafRow& primary, int* anc, int* slot,
+                                               Real* geom) {
+  LeafRow u = primary;
   for (int k = 0; k < 2; ++k) {
+    if (k) u = leaf_row(a.anc_backup, row);
     bool ok = true;
+#pragma unroll
     for (int j = 0; j < 3; ++j) {
-      anc[j] = leaf_resolve(a, p, b, sets[k] + 3 * j);
-      ok = ok && anc[j] != -1 && !a.pose_missing[int64_t(p) * a.NA + anc[j]];
+      anc[j] = leaf_resolve(a, p, b, u.v + 3 * j);
+      slot[j] = u.v[3 * j];
+      ok = ok && anc[j] != -1;
     }
-    if (ok) {
-      geom[0] = geoms[k][0];
-      geom[1] = geoms[k][1];
-      geom[2] = geoms[k][2];
-      return true;
-    }
+    if (!ok) continue;
+    const uint8_t* miss = a.pose_missing + int64_t(p) * a.NA;
+    __builtin_memcpy(geom, (const Real*)(k ? a.geom_backup : a.geom) + row * 3, 3 * sizeof(Real));
+    if (!(miss[anc[0]] | miss[anc[1]] | miss[anc[2]])) return true;
   }
   return false;
 }
+
+// what an atom slot's work starts from: loads that need the block's type
+// alone, issued together (the kernels wait on chains of loads, not on
+// bandwidth), and held by `ready` before the first branch on them
+struct LeafSlot {
+  int n_at, off, miss;
+  LeafRow row;
+  __device__ __forceinline__ LeafSlot(const LeafArgs& a, int q, int bt, int at) {
+    n_at = a.n_atoms[bt];
+    off = a.block_offset[q];
+    miss = a.block_missing[int64_t(q) * a.Amax + at];
+    row = leaf_row(a.anc, int64_t(bt) * a.Amax + at);
+  }
+  __device__ __forceinline__ void ready() {
+    asm volatile("" : "+v"(n_at), "+v"(off), "+v"(miss), "+v"(row.v[0]), "+v"(row.v[4]),
+                 "+v"(row.v[8]));
+  }
+};
 
 template <typename Real>
 __device__ __forceinline__ bool any_nan(Vec3<Real> v) {
@@ -128,11 +163,15 @@ __device__ __forceinline__ bool any_nan(Vec3<Real> v) {
 // (pose, block) grid: it loads their types, keeps the real ones (a ballot)
 // and takes them G = 64 / Amax at a time (Amax <= 64: lane = g * Amax + atom
 // slot), or one at a time with lanes striding over the atom slots (Amax >
-// 64).  Padding blocks cost one load per 64.
+// 64).  Padding blocks cost one load per LEAF_BPW.
 constexpr int LEAF_WAVE = 64;
-// blocks whose types one wave loads: fewer than 64 keeps one or two passes
-// per wave, so the dependent loads of many waves overlap
-constexpr int LEAF_BPW = 16;
+// blocks whose types one wave loads.  The kernels wait on chains of dependent
+// loads, so two passes per wave keep more chains in flight than sixteen
+// blocks' eight; fewer repeat the launch and the type load.  Build / backward
+// local / remote, 256 poses of 50-600 residues: 2 blocks 42 / 59 / 42 us, 4
+// 38 / 54 / 39, 8 41 / 56 / 43, 16 46 / 59 / 54 (one after another with their
+// loads instead of together: 51 / 64 / 52).
+constexpr int LEAF_BPW = 4;
 constexpr int LEAF_MAX_ATOMS = 2048;  // larger block types: ENOTSUP
 
 struct LeafPass {
@@ -188,21 +227,22 @@ __global__ __launch_bounds__(LEAF_WAVE) void leaf_atoms_kernel(LeafArgs a, const
       real = leaf_drop(a, real);
       if (r.g < 0) continue;
       const int p = r.q / a.B, b = r.q - p * a.B;
-      const int n_at = a.n_atoms[r.bt];
-      const int64_t off = int64_t(p) * a.NA + a.block_offset[r.q];
-      for (int at = r.at0; at < n_at; at += r.stride) {
-        const int64_t dst = off + at;
+      for (int at = r.at0; at < a.Amax; at += r.stride) {
+        LeafSlot s(a, r.q, r.bt, at);
+        s.ready();
+        if (at >= s.n_at) continue;
+        const int64_t dst = int64_t(p) * a.NA + s.off + at;
         Real* o = out + 3 * dst;
-        if (!a.block_missing[int64_t(r.q) * a.Amax + at]) {
+        if (!s.miss) {
           o[0] = orig[3 * dst];
           o[1] = orig[3 * dst + 1];
           o[2] = orig[3 * dst + 2];
           continue;
         }
-        int anc[3];
+        int anc[3], slot[3];
         Real g[3];
         Vec3<Real> W = {Real(NAN), Real(NAN), Real(NAN)};
-        if (leaf_ancestors(a, p, b, r.bt, at, anc, g)) {
+        if (leaf_ancestors(a, p, b, int64_t(r.bt) * a.Amax + at, s.row, anc, slot, g)) {
           const Real* base = orig + 3 * int64_t(p) * a.NA;
           const Vec3<Real> A = v3(base + 3 * anc[0]), B = v3(base + 3 * anc[1]),
                            C = v3(base + 3 * anc[2]);
@@ -223,50 +263,24 @@ __global__ __launch_bounds__(LEAF_WAVE) void leaf_atoms_kernel(LeafArgs a, const
   }
 }
 
-// the ancestors of a built atom (pose-local indices) with, for each, its
-// atom slot in the same block or -1 when named across a connection; false
-// when no complete ancestor set exists
-template <typename Real>
-__device__ __forceinline__ bool leaf_ancestor_slots(const LeafArgs& a, int p, int b, int bt,
-                                                    int at, int* anc, int* slot, Real* g) {
-  const int64_t row = int64_t(bt) * a.Amax + at;
-  const int32_t* sets[2] = {a.anc + row * 9, a.anc_backup + row * 9};
-  const Real* geoms[2] = {(const Real*)a.geom + row * 3, (const Real*)a.geom_backup + row * 3};
-  for (int k = 0; k < 2; ++k) {
-    bool ok = true;
-    for (int j = 0; j < 3; ++j) {
-      const int32_t* u = sets[k] + 3 * j;
-      anc[j] = leaf_resolve(a, p, b, u);
-      slot[j] = u[0];
-      ok = ok && anc[j] != -1 && !a.pose_missing[int64_t(p) * a.NA + anc[j]];
-    }
-    if (ok) {
-      g[0] = geoms[k][0];
-      g[1] = geoms[k][1];
-      g[2] = geoms[k][2];
-      return true;
-    }
-  }
-  return false;
-}
-
 // the ancestor shares of the atom at slot `at` of block q if it is built
 // (false otherwise, or without ancestors or with an absent coordinate; with
 // REMOTE_ONLY also when every ancestor is in the same block)
 template <typename Real, bool REMOTE_ONLY>
 __device__ __forceinline__ bool leaf_shares(const LeafArgs& a, const Real* orig,
-                                            const Real* dnew, int q, int bt, int at, int* anc,
-                                            int* slot, Vec3<Real>* gs) {
-  if (!a.block_missing[int64_t(q) * a.Amax + at]) return false;
+                                            const Real* dnew, int q, int bt, int at,
+                                            const LeafSlot& s, int* anc, int* slot,
+                                            Vec3<Real>* gs) {
+  if (!s.miss) return false;
   const int p = q / a.B, b = q - p * a.B;
   Real g[3];
-  if (!leaf_ancestor_slots(a, p, b, bt, at, anc, slot, g)) return false;
+  if (!leaf_ancestors(a, p, b, int64_t(bt) * a.Amax + at, s.row, anc, slot, g)) return false;
   if (REMOTE_ONLY && slot[0] >= 0 && slot[1] >= 0 && slot[2] >= 0) return false;
   const int64_t base = int64_t(p) * a.NA;
   const Vec3<Real> A = v3(orig + 3 * (base + anc[0])), B = v3(orig + 3 * (base + anc[1])),
                    C = v3(orig + 3 * (base + anc[2]));
   if (any_nan(A) || any_nan(B) || any_nan(C)) return false;
-  const int64_t dst = base + a.block_offset[q] + at;
+  const int64_t dst = base + s.off + at;
   build_coord_vjp(A, B, C, water_coef(g[2], g[1], g[0]), v3(dnew + 3 * dst), gs[0], gs[1],
                   gs[2]);
   return true;
@@ -294,12 +308,15 @@ __global__ __launch_bounds__(LEAF_WAVE) void leaf_atoms_backward_local_kernel(
       real = leaf_drop(a, real);
       for (int i = lane; i < 3 * W; i += LEAF_WAVE) acc[i] = Real(0);
       __syncthreads();
-      const int n_at = r.g < 0 ? 0 : a.n_atoms[r.bt];
       const int gbase = r.g < 0 ? 0 : r.g * a.Amax;
-      for (int at = r.at0; at < n_at; at += r.stride) {
+      const int n_slots = r.g < 0 ? 0 : a.Amax;
+      for (int at = r.at0; at < n_slots; at += r.stride) {
+        LeafSlot s(a, r.q, r.bt, at);
+        s.ready();
+        if (at >= s.n_at) continue;
         int anc[3], slot[3];
         Vec3<Real> gs[3];
-        if (!leaf_shares<Real, false>(a, orig, dnew, r.q, r.bt, at, anc, slot, gs)) continue;
+        if (!leaf_shares<Real, false>(a, orig, dnew, r.q, r.bt, at, s, anc, slot, gs)) continue;
         for (int j = 0; j < 3; ++j) {
           if (slot[j] < 0) continue;
           const int e = gbase + slot[j];
@@ -312,6 +329,7 @@ __global__ __launch_bounds__(LEAF_WAVE) void leaf_atoms_backward_local_kernel(
       if (r.g >= 0) {
         const int p = r.q / a.B;
         const int64_t off = int64_t(p) * a.NA + a.block_offset[r.q];
+        const int n_at = a.n_atoms[r.bt];
         for (int at = r.at0; at < n_at; at += r.stride) {
           const int64_t dst = off + at;
           const int e = gbase + at;
@@ -339,12 +357,17 @@ __global__ __launch_bounds__(LEAF_WAVE) void leaf_atoms_backward_remote_kernel(
       const LeafPass r = leaf_pass(a, real, q0, bt_lane, lane);
       real = leaf_drop(a, real);
       if (r.g < 0) continue;
-      const int n_at = a.n_atoms[r.bt];
       const int64_t base = int64_t(r.q / a.B) * a.NA;
-      for (int at = r.at0; at < n_at; at += r.stride) {
+      for (int at = r.at0; at < a.Amax; at += r.stride) {
+        LeafSlot s(a, r.q, r.bt, at);
+        const LeafRow backup = leaf_row(a.anc_backup, int64_t(r.bt) * a.Amax + at);
+        s.ready();
+        // most atoms hang from their own block whichever set they take: the
+        // tables say so before any ancestor is looked up
+        if (at >= s.n_at || !(s.row.remote() || backup.remote())) continue;
         int anc[3], slot[3];
         Vec3<Real> gs[3];
-        if (!leaf_shares<Real, true>(a, orig, dnew, r.q, r.bt, at, anc, slot, gs)) continue;
+        if (!leaf_shares<Real, true>(a, orig, dnew, r.q, r.bt, at, s, anc, slot, gs)) continue;
         for (int j = 0; j < 3; ++j) {
           if (slot[j] >= 0) continue;
           Real* d = dorig + 3 * (base + anc[j]);
