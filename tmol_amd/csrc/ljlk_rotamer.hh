@@ -28,7 +28,20 @@
 
 namespace tmol_ljlk {
 
-constexpr int UNIT_R1 = 4;  // b1 rotamers per work unit
+// b1 rotamers per work unit of a cell with nr2 rotamers in b2.  A unit is one
+// wave's serial work and grows with the rotamer pairs in it, so a cell of two
+// long side chains made units of hundreds of pairs and the launch ended in a
+// few of them (2.8 waves per SIMD resident on average where 7 fit).  About 32
+// pairs per unit end together; smaller units stage b2's list for too few b1
+// rotamers.  Energies of 8 x 200 residues / elec forward / backward of 5 x
+// 151: always 4 rotamers 2.85 / 1.03 / 1.67 ms, 128 pairs 2.81 / 1.03 / 1.67,
+// 64 pairs 2.54 / 0.77 / 1.34, 32 pairs 2.47 / 0.69 / 1.20, 16 pairs 2.61 /
+// 0.73 / 1.25.
+constexpr int UNIT_R1 = 4;      // most b1 rotamers of a unit
+constexpr int UNIT_PAIRS = 32;  // rotamer pairs of a unit, where that is at least one b1 rotamer
+__device__ __forceinline__ int unit_r1(int nr2, bool diag) {
+  return diag ? UNIT_R1 : max(1, min(UNIT_R1, UNIT_PAIRS / max(nr2, 1)));
+}  // b1 rotamers per work unit
 
 struct RotView {
   int P, B, R, C;
@@ -140,12 +153,12 @@ __global__ __launch_bounds__(256) void rot_rows_count_kernel(RotView v,
     const Real s0 = bsph[g1 * 4 + 0], s1 = bsph[g1 * 4 + 1], s2 = bsph[g1 * 4 + 2],
                s3 = bsph[g1 * 4 + 3];
     const int64_t nr1 = v.n_rots_for_block[g1];
-    const int64_t nu = (nr1 + UNIT_R1 - 1) / UNIT_R1;
     for (int b2 = b1 + lane; b2 < v.B; b2 += WAVE) {
       const int64_t g2 = int64_t(p) * v.B + b2;
       if (rot_cell_hit(v, bsph, s0, s1, s2, s3, g2, reach)) {
-        pairs += b2 == b1 ? nr1 : nr1 * int64_t(v.n_rots_for_block[g2]);
-        units += nu;
+        const int nr2 = v.n_rots_for_block[g2], ur = unit_r1(nr2, b2 == b1);
+        pairs += b2 == b1 ? nr1 : nr1 * int64_t(nr2);
+        units += (nr1 + ur - 1) / ur;
       }
     }
   }
@@ -211,7 +224,6 @@ __global__ __launch_bounds__(256) void rot_rows_fill_kernel(
   const Real s0 = bsph[g1 * 4 + 0], s1 = bsph[g1 * 4 + 1], s2 = bsph[g1 * 4 + 2],
              s3 = bsph[g1 * 4 + 3];
   const int nr1 = v.n_rots_for_block[g1], off1 = v.rot_offset_for_block[g1];
-  const int nu = (nr1 + UNIT_R1 - 1) / UNIT_R1;
   int64_t e = pair_off[g1], u = unit_off[g1];
   for (int c0 = b1; c0 < v.B; c0 += WAVE) {
     const int b2l = c0 + lane;
@@ -245,13 +257,14 @@ __global__ __launch_bounds__(256) void rot_rows_fill_kernel(
         indices[n_pairs + e + k] = v1;
         indices[2 * n_pairs + e + k] = v2;
       }
+      const int ur = unit_r1(nr2, diag), nu = (nr1 + ur - 1) / ur;
       for (int k = lane; k < nu; k += WAVE) {
         RotUnit U;
         U.g1 = int(g1);
         U.b2 = b2;
-        U.r1_first = off1 + k * UNIT_R1;
-        U.r1_count = (ok ? 1 : -1) * min(UNIT_R1, nr1 - k * UNIT_R1);
-        U.entry = e + (diag ? int64_t(k) * UNIT_R1 : int64_t(k) * UNIT_R1 * nr2);
+        U.r1_first = off1 + k * ur;
+        U.r1_count = (ok ? 1 : -1) * min(ur, nr1 - k * ur);
+        U.entry = e + (diag ? int64_t(k) * ur : int64_t(k) * ur * nr2);
         U.pad = 0;
         units[u + k] = U;
       }
