@@ -173,8 +173,9 @@ __device__ void elec_rot_intra(const ElecRotArgs<Real>& A, ElecRotLDS<Real>& L, 
 // Culling and compaction (the structure of the LJ+LK rotamer energy kernel),
 // for the energies and for the dTdV-weighted backward.  Per b1 rotamer r1 of
 // a unit:
-//   cull      every atom of b2's rotamers (the candidates, 64 at a time in
-//             rotamer order, over windows of up to 64 b2 rotamers) is tested
+//   cull      every atom of b2's rotamers whose spheres r1's reaches (the
+//             candidates, 64 at a time in rotamer order, over windows of up
+//             to 64 b2 rotamers) is tested
 //             against r1's sphere; charged survivors are compacted, in order,
 //             into a 64-lane chunk
 //   phase A   for a full (or the last) chunk: r1's atoms come from the
@@ -210,13 +211,13 @@ struct ElecRotLDS2 {
 };
 
 template <typename Real, bool BWD>
-__device__ __forceinline__ void elec_chunk_eval(ElecRotLDS2<Real, BWD>& L, int consume,
+__device__ __forceinline__ void elec_chunk_eval(ElecRotLDS2<Real, BWD>& L, int head, int consume,
                                                 const ElecConst<Real>& k, int lane) {
   using V = typename V4<Real>::T;
   using Acc = LdsAcc<Real>;
   using T = typename Acc::T;
   if (lane < consume) {
-    const int en = L.fifo[lane];
+    const int en = L.fifo[(head + lane) & (2 * WAVE - 1)];
     const int j = en & 31, l2 = (en >> 5) & 63;
     const Real wcp = (en >> 11) & 1 ? Real(0.2) : Real(1);
     const V p1 = *(const V*)L.r1.pos[j], p2 = *(const V*)L.pos2[l2];
@@ -241,12 +242,12 @@ __device__ __forceinline__ void elec_chunk_eval(ElecRotLDS2<Real, BWD>& L, int c
   }
 }
 
-// phase A + B over the chunk's nb lanes against r1 (n1 atoms held in the
-// registers R1 of lanes 0..n1-1), then (forward) the fold into the window's
+// phase A + B over the chunk's nb lanes against r1 (its charged atoms, a lane
+// mask, held in the registers R1), then (forward) the fold into the window's
 // sums or (backward) the flush of the chunk atoms' gradient
 template <typename Real, bool BWD>
-__device__ void elec_chunk(ElecRotLDS2<Real, BWD>& L, const ElecConst<Real>& k, int nb, int n1,
-                           bool cp, int min_sep, int nc1, bool lig1, const ElecAtom<Real>& R1,
+__device__ void elec_chunk(ElecRotLDS2<Real, BWD>& L, const ElecConst<Real>& k, int nb,
+                           uint64_t charged1, bool cp, int min_sep, int nc1, bool lig1, const ElecAtom<Real>& R1,
                            Real* grad, int lane) {
   using V = typename V4<Real>::T;
   using Acc = LdsAcc<Real>;
@@ -266,9 +267,9 @@ __device__ void elec_chunk(ElecRotLDS2<Real, BWD>& L, const ElecConst<Real>& k, 
     L.lacc[lane] = 0;
   else
     L.acc2[0][lane] = L.acc2[1][lane] = L.acc2[2][lane] = 0;
-  int n_f = 0;
-  for (int j = 0; j < n1; ++j) {
-    if (lane_val(R1.q, j) == Real(0)) continue;  // uncharged b1 atom
+  int hf = 0, tf = 0;  // FIFO ring: head and tail (wave-uniform)
+  for (uint64_t js = charged1; js; js &= js - 1) {
+    const int j = __builtin_ctzll(js);
     const Real dx = lane_val(R1.x, j) - p2.x, dy = lane_val(R1.y, j) - p2.y,
                dz = lane_val(R1.z, j) - p2.z;
     bool in = valid && dx * dx + dy * dy + dz * dz < k.cull2;
@@ -281,17 +282,18 @@ __device__ void elec_chunk(ElecRotLDS2<Real, BWD>& L, const ElecConst<Real>& k, 
       w02 = sep == 4;
     }
     const uint64_t m = __ballot(in);
-    if (in) L.fifo[n_f + lanes_below(m)] = (uint16_t)(j | (lane << 5) | (w02 ? (1 << 11) : 0));
-    n_f += __popcll(m);
-    if (n_f >= WAVE) {
+    if (in)
+      L.fifo[(tf + lanes_below(m)) & (2 * WAVE - 1)] =
+          (uint16_t)(j | (lane << 5) | (w02 ? (1 << 11) : 0));
+    tf += __popcll(m);
+    if (tf - hf >= WAVE) {
       wave_sync();
-      elec_chunk_eval(L, WAVE, k, lane);
-      fifo_shift(L.fifo, WAVE, n_f, lane);
-      n_f -= WAVE;
+      elec_chunk_eval(L, hf, WAVE, k, lane);
+      hf += WAVE;
     }
   }
   wave_sync();
-  if (n_f > 0) elec_chunk_eval(L, n_f, k, lane);
+  if (tf > hf) elec_chunk_eval(L, hf, tf - hf, k, lane);
   wave_sync();
   if constexpr (BWD) {
     if (valid) {
@@ -348,21 +350,15 @@ __device__ void elec_rot_inter_chunked(const ElecRotArgs<Real>& A, ElecRotLDS2<R
   for (int w0 = 0; w0 < nr2; w0 += WAVE) {
     const int wn = min(WAVE, nr2 - w0);
     // the window's rotamers (lane = rotamer): type, first atom, atom count,
-    // first candidate; candidates fetch theirs by lane shuffle
-    int nat = 0, t2l = -1, o2l = 0;
+    // sphere; candidates fetch theirs by lane shuffle
+    int nat2 = 0, t2l = -1, o2l = 0;
+    V s2 = {};
     if (lane < wn) {
       t2l = v.block_type_for_rot[off2 + w0 + lane];
       o2l = v.rot_coord_offset[off2 + w0 + lane];
-      nat = t2l >= 0 ? A.bt.n_atoms[t2l] : 0;
+      nat2 = t2l >= 0 ? A.bt.n_atoms[t2l] : 0;
+      s2 = *(const V*)(A.rot_spheres + 4 * int64_t(off2 + w0 + lane));
     }
-    int incl = nat;
-#pragma unroll
-    for (int o = 1; o < WAVE; o <<= 1) {
-      const int t = __shfl_up(incl, o, WAVE);
-      if (lane >= o) incl += t;
-    }
-    const int excl = incl - nat;
-    const int total = lane_val(incl, wn - 1);
     for (int i = 0; i < r1_count; ++i) {
       const int r1 = r1_first + i;
       const int t1 = uni(v.block_type_for_rot[r1]);
@@ -377,6 +373,12 @@ __device__ void elec_rot_inter_chunked(const ElecRotArgs<Real>& A, ElecRotLDS2<R
       const V sph = *(const V*)(A.rot_spheres + 4 * int64_t(r1));
       const Real reach = sph.w + k.hpe + Real(1e-3);
       const Real reach2 = reach * reach;
+      // candidates: the atoms of the rotamers whose sphere r1's reaches (one
+      // that is not a number stays)
+      const int nat = rot_sphere_far(sph, s2, reach) ? 0 : nat2;
+      const int incl = wave_prefix(nat);
+      const int excl = incl - nat;
+      const int total = lane_val(incl, wn - 1);
       ElecAtom<Real> R1;
       R1.x = R1.y = R1.z = R1.q = Real(0);
       R1.pd = 0;
@@ -390,6 +392,7 @@ __device__ void elec_rot_inter_chunked(const ElecRotArgs<Real>& A, ElecRotLDS2<R
         p.w = R1.q;
         *(V*)L.r1.pos[lane] = p;
       }
+      const uint64_t charged1 = __ballot(R1.q != Real(0));
       if constexpr (!BWD)
         L.sum[lane] = 0;
       else if (lane < TILE)
@@ -424,7 +427,7 @@ __device__ void elec_rot_inter_chunked(const ElecRotArgs<Real>& A, ElecRotLDS2<R
         const int nk = __popcll(mk);
         if (nk == 0) continue;
         if (nb + nk > WAVE) {
-          elec_chunk(L, k, nb, n1, cp, min_sep, nc1, lig1, R1, A.grad, lane);
+          elec_chunk(L, k, nb, charged1, cp, min_sep, nc1, lig1, R1, A.grad, lane);
           nb = 0;
         }
         if (keep) {
@@ -444,7 +447,7 @@ __device__ void elec_rot_inter_chunked(const ElecRotArgs<Real>& A, ElecRotLDS2<R
         }
         nb += nk;
       }
-      if (nb > 0) elec_chunk(L, k, nb, n1, cp, min_sep, nc1, lig1, R1, A.grad, lane);
+      if (nb > 0) elec_chunk(L, k, nb, charged1, cp, min_sep, nc1, lig1, R1, A.grad, lane);
       wave_sync();
       if constexpr (!BWD) {
         if (lane < wn) A.energies[entry + int64_t(i) * nr2 + w0 + lane] = L.sum[lane];
@@ -464,8 +467,8 @@ __device__ void elec_rot_inter_chunked(const ElecRotArgs<Real>& A, ElecRotLDS2<R
 // written, zero for pairs that are not scored); BWD true: grad [NA, 3] +=
 // sum_i dTdV[i] dV(pair i)/dx.  Float builds are held to 7 waves per SIMD:
 // the kernel is latency-bound, and the few spilled registers cost less than
-// the waves gained (forward 5.76 -> 4.77 ms on the 16 x 300-residue
-// repacking set).
+// the waves gained (5 x 151 residues, forward / backward at 5 waves 0.65 /
+// 1.20 ms, 6 and 7 0.63 / 1.16, 8 0.65 / 1.16).
 template <typename Real, bool BWD>
 __global__ __launch_bounds__(256, sizeof(Real) == 4 ? 7 : 2) void elec_rotamer_kernel(
     ElecRotArgs<Real> A) {

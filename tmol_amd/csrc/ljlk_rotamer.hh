@@ -385,15 +385,55 @@ __device__ __forceinline__ void stage_rot_chunk(RotLDS<Real>& L, const RotArgs<R
   wave_sync();
 }
 
+// x of another lane by a DPP control for the rows (of 16 lanes) of the mask;
+// zero elsewhere and where the control reaches over a row's edge (every lane
+// of the wave active)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_or_zero(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_or_zero(float x) {
+  return __int_as_float(dpp_or_zero<CTRL, ROWS>(__float_as_int(x)));
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_or_zero(double x) {
+  const long long b = __double_as_longlong(x);
+  const uint32_t lo = uint32_t(dpp_or_zero<CTRL, ROWS>(int(b & 0xffffffffll)));
+  const uint32_t hi = uint32_t(dpp_or_zero<CTRL, ROWS>(int(b >> 32)));
+  return __longlong_as_double((long long)((uint64_t(hi) << 32) | lo));
+}
+
+// inclusive prefix sum over the wave: four shifts within rows of 16 lanes,
+// then the row ends 15 and 47 into rows 1 and 3 and lane 31 into rows 2 and 3
+__device__ __forceinline__ int wave_prefix(int x) {
+  x += dpp_or_zero<0x111, 0xf>(x);
+  x += dpp_or_zero<0x112, 0xf>(x);
+  x += dpp_or_zero<0x114, 0xf>(x);
+  x += dpp_or_zero<0x118, 0xf>(x);
+  x += dpp_or_zero<0x142, 0xa>(x);
+  x += dpp_or_zero<0x143, 0xc>(x);
+  return x;
+}
+
 // Sum of the lanes of each segment [seg_start, ...] of contiguous lanes,
-// left in each segment's last lane (inclusive segmented scan).
+// left in each segment's last lane (inclusive segmented scan: the steps of
+// wave_prefix where they stay inside the segment).
 template <typename T>
 __device__ __forceinline__ T segment_scan(T x, int seg_start, int lane) {
-#pragma unroll
-  for (int o = 1; o < WAVE; o <<= 1) {
-    const T t = __shfl_up(x, o, WAVE);
-    if (lane - o >= seg_start) x += t;
-  }
+  const int d = lane - seg_start;
+  T t = dpp_or_zero<0x111, 0xf>(x);
+  if (d >= 1) x += t;
+  t = dpp_or_zero<0x112, 0xf>(x);
+  if (d >= 2) x += t;
+  t = dpp_or_zero<0x114, 0xf>(x);
+  if (d >= 4) x += t;
+  t = dpp_or_zero<0x118, 0xf>(x);
+  if (d >= 8) x += t;
+  t = dpp_or_zero<0x142, 0xa>(x);
+  if (seg_start < (lane & 48)) x += t;
+  t = dpp_or_zero<0x143, 0xc>(x);
+  if (seg_start < 32) x += t;
   return x;
 }
 
@@ -747,8 +787,8 @@ rotamer_score_kernel(RotArgs<Real> A) {
 // ------------------------------------------------------------------ energies, culled
 
 // Energy forward with culling and compaction.  Per b1 rotamer r1 of a unit:
-//   cull      every atom of b2's rotamers (the candidates, taken 64 at a time
-//             in rotamer order) is tested against r1's sphere: an atom
+//   cull      every atom of b2's rotamers whose spheres r1's reaches (the
+//             candidates, taken 64 at a time in rotamer order) is tested against r1's sphere: an atom
 //             farther than R1 + max_dis from r1's centre reaches no atom of
 //             r1 (triangle inequality; 1e-3 A margin for rounding).
 //             Survivors are compacted, in order, into a 64-lane chunk.
@@ -765,8 +805,16 @@ rotamer_score_kernel(RotArgs<Real> A) {
 //             of the rotamers of the current window of 64 b2 rotamers.
 //   write     after the window, one store per rotamer pair and term (zero
 //             for pairs with no surviving atoms).
+//
+// Bound by VALU issue (75% busy): 8 x 200 residues take 2.3 M candidate
+// chunks, 18 M phase A steps, 4.1 M LJ and 1.5 M LK batches, about 1.3 G
+// wave instructions.  Dropping rotamers by sphere before their atoms, FIFO
+// rings in place of moving the rest to the front, scans by DPP and the heavy
+// atoms as lane masks took it from 2.47 to 2.32 ms (elec, the same changes:
+// forward 0.69 -> 0.63, backward 1.20 -> 1.16 ms for 5 x 151 residues).  Four
+// waves per SIMD: five cost more in registers than they hide (2.36 ms).
 
-constexpr int RFIFO = 2 * WAVE;  // FIFO capacity: < 64 left over + 64 appended
+constexpr int RFIFO = 2 * WAVE;  // FIFO ring: < 64 left over + 64 appended
 
 template <typename Real>
 struct RotLDS2 {
@@ -782,12 +830,12 @@ struct RotLDS2 {
 };
 
 template <typename Real>
-__device__ __forceinline__ void rot_fifo_lj(RotLDS2<Real>& L, int consume,
+__device__ __forceinline__ void rot_fifo_lj(RotLDS2<Real>& L, int head, int consume,
                                             const GlobalParams<Real>& gp, int lane) {
   using V = typename V4<Real>::T;
   using Acc = LdsAcc<Real>;
   if (lane < consume) {
-    const int e = L.lj[lane];
+    const int e = L.lj[(head + lane) & (RFIFO - 1)];
     const int a1 = e & 63, l2 = (e >> 6) & 63;
     const Real wcp = (e >> 12) & 1 ? Real(0.2) : Real(1);
     const V p1 = *(const V*)L.r1.pos[a1], p2 = *(const V*)L.pos2[l2];
@@ -805,12 +853,12 @@ __device__ __forceinline__ void rot_fifo_lj(RotLDS2<Real>& L, int consume,
 }
 
 template <typename Real>
-__device__ __forceinline__ void rot_fifo_lk(RotLDS2<Real>& L, int consume,
+__device__ __forceinline__ void rot_fifo_lk(RotLDS2<Real>& L, int head, int consume,
                                             const GlobalParams<Real>& gp, int lane) {
   using V = typename V4<Real>::T;
   using Acc = LdsAcc<Real>;
   if (lane < consume) {
-    const int e = L.lk[lane];
+    const int e = L.lk[(head + lane) & (RFIFO - 1)];
     const int a1 = e & 63, l2 = (e >> 6) & 63;
     const Real wcp = (e >> 12) & 1 ? Real(0.2) : Real(1);
     const V p1 = *(const V*)L.r1.pos[a1], p2 = *(const V*)L.pos2[l2];
@@ -831,23 +879,12 @@ __device__ __forceinline__ void rot_fifo_lk(RotLDS2<Real>& L, int consume,
   }
 }
 
-// consume the first `c` entries of a FIFO of n and move the rest to the front
-__device__ __forceinline__ void rot_fifo_shift(uint16_t* f, int c, int n, int lane) {
-  const int rem = n - c;
-  if (rem <= 0) return;
-  uint16_t v = 0;
-  if (lane < rem) v = f[c + lane];
-  wave_sync();
-  if (lane < rem) f[lane] = v;
-  wave_sync();
-}
-
 // phase A + B over the chunk's nb lanes against r1 (n1 atoms staged), then
 // fold the lanes' sums into the window's per-rotamer sums
 template <typename Real>
 __device__ void rot_chunk(RotLDS2<Real>& L, const GlobalParams<Real>& gp, int nb, int n1,
                           bool cp, int min_sep, int nc1, bool lig1, const AtomRegs<Real>& R1,
-                          int lane) {
+                          uint64_t heavy1, int lane) {
   using V = typename V4<Real>::T;
   using Acc = LdsAcc<Real>;
   wave_sync();
@@ -860,13 +897,13 @@ __device__ void rot_chunk(RotLDS2<Real>& L, const GlobalParams<Real>& gp, int nb
     meta = L.meta2[lane];
     pd2 = L.pd2[lane];
   }
-  const bool heavy2 = meta & F_HEAVY;
+  const uint64_t heavy2 = __ballot(meta & F_HEAVY);
   const int nc2 = (meta >> 8) & 7;
   const bool lig = lig1 && ((meta >> 11) & 1);
   L.lacc[0][lane] = 0;
   L.lacc[1][lane] = 0;
   L.lacc[2][lane] = 0;
-  int nlj = 0, nlk = 0;  // wave-uniform FIFO fill
+  int hlj = 0, tlj = 0, hlk = 0, tlk = 0;  // FIFO heads and tails (wave-uniform)
   // a1's data come from the registers of the lane that staged it
   // (wave-uniform readlane), so the test chain has no LDS latency
   for (int j = 0; j < n1; ++j) {
@@ -884,29 +921,27 @@ __device__ void rot_chunk(RotLDS2<Real>& L, const GlobalParams<Real>& gp, int nb
     const uint64_t m = __ballot(in);
     if (m == 0) continue;
     const uint16_t ent = (uint16_t)(j | (lane << 6) | (w02 ? (1 << 12) : 0));
-    if (in) L.lj[nlj + lanes_below(m)] = ent;
-    nlj += __popcll(m);
-    if (lane_val(R1.flags, j) & F_HEAVY) {
-      const uint64_t mh = __ballot(in && heavy2);
-      if (in && heavy2) L.lk[nlk + lanes_below(mh)] = ent;
-      nlk += __popcll(mh);
+    if (in) L.lj[(tlj + lanes_below(m)) & (RFIFO - 1)] = ent;
+    tlj += __popcll(m);
+    if ((heavy1 >> j) & 1) {
+      const uint64_t mh = m & heavy2;
+      if ((mh >> lane) & 1) L.lk[(tlk + lanes_below(mh)) & (RFIFO - 1)] = ent;
+      tlk += __popcll(mh);
     }
-    if (nlj >= WAVE) {
+    if (tlj - hlj >= WAVE) {
       wave_sync();
-      rot_fifo_lj(L, WAVE, gp, lane);
-      rot_fifo_shift(L.lj, WAVE, nlj, lane);
-      nlj -= WAVE;
+      rot_fifo_lj(L, hlj, WAVE, gp, lane);
+      hlj += WAVE;
     }
-    if (nlk >= WAVE) {
+    if (tlk - hlk >= WAVE) {
       wave_sync();
-      rot_fifo_lk(L, WAVE, gp, lane);
-      rot_fifo_shift(L.lk, WAVE, nlk, lane);
-      nlk -= WAVE;
+      rot_fifo_lk(L, hlk, WAVE, gp, lane);
+      hlk += WAVE;
     }
   }
   wave_sync();
-  if (nlj > 0) rot_fifo_lj(L, nlj, gp, lane);
-  if (nlk > 0) rot_fifo_lk(L, nlk, gp, lane);
+  if (tlj > hlj) rot_fifo_lj(L, hlj, tlj - hlj, gp, lane);
+  if (tlk > hlk) rot_fifo_lk(L, hlk, tlk - hlk, gp, lane);
   wave_sync();
   // fold: lanes of one rotamer (slot) are contiguous
   const int slot = meta >> 16;
@@ -927,6 +962,15 @@ __device__ void rot_chunk(RotLDS2<Real>& L, const GlobalParams<Real>& gp, int nb
     L.sum[2][slot] += e2;
   }
   wave_sync();
+}
+
+// rotamer spheres more than max_dis (with a margin for rounding) apart: reach
+// is the first's radius + max_dis + 1e-3
+template <typename V, typename Real>
+__device__ __forceinline__ bool rot_sphere_far(const V& s1, const V& s2, Real reach) {
+  const Real dx = s1.x - s2.x, dy = s1.y - s2.y, dz = s1.z - s2.z;
+  const Real r = reach + s2.w + Real(1e-3);
+  return dx * dx + dy * dy + dz * dz > r * r;
 }
 
 // inter-block unit, energies only
@@ -954,21 +998,15 @@ __device__ void rot_inter_energy(const RotArgs<Real>& A, RotLDS2<Real>& L,
   for (int w0 = 0; w0 < nr2; w0 += WAVE) {
     const int wn = min(WAVE, nr2 - w0);
     // the window's rotamers (lane = rotamer): type, first atom, atom count,
-    // first candidate; candidates fetch theirs by lane shuffle
-    int nat = 0, t2l = -1, o2l = 0;
+    // sphere; candidates fetch theirs by lane shuffle
+    int nat2 = 0, t2l = -1, o2l = 0;
+    V s2 = {};
     if (lane < wn) {
       t2l = v.block_type_for_rot[off2 + w0 + lane];
       o2l = v.rot_coord_offset[off2 + w0 + lane];
-      nat = t2l >= 0 ? A.bt.n_atoms[t2l] : 0;
+      nat2 = t2l >= 0 ? A.bt.n_atoms[t2l] : 0;
+      s2 = *(const V*)(A.rot_spheres + 4 * int64_t(off2 + w0 + lane));
     }
-    int incl = nat;
-#pragma unroll
-    for (int o = 1; o < WAVE; o <<= 1) {
-      const int t = __shfl_up(incl, o, WAVE);
-      if (lane >= o) incl += t;
-    }
-    const int excl = incl - nat;
-    const int total = lane_val(incl, wn - 1);
     for (int i = 0; i < r1_count; ++i) {
       const int r1 = r1_first + i;
       const int t1 = uni(v.block_type_for_rot[r1]);
@@ -980,10 +1018,15 @@ __device__ void rot_inter_energy(const RotArgs<Real>& A, RotLDS2<Real>& L,
       const int n1 = uni(A.bt.n_atoms[t1]);
       const int nc1 = uni(A.bt.n_conn[t1]);
       const bool lig1 = A.bt.is_ligand[t1];
-      const Real* sph = A.rot_spheres + int64_t(r1) * 4;
-      const Real cx = sph[0], cy = sph[1], cz = sph[2];
-      const Real reach = sph[3] + gp.max_dis + Real(1e-3);
+      const V sph = *(const V*)(A.rot_spheres + int64_t(r1) * 4);
+      const Real reach = sph.w + gp.max_dis + Real(1e-3);
       const Real reach2 = reach * reach;
+      // candidates: the atoms of the rotamers whose sphere r1's reaches (one
+      // that is not a number stays)
+      const int nat = rot_sphere_far(sph, s2, reach) ? 0 : nat2;
+      const int incl = wave_prefix(nat);
+      const int excl = incl - nat;
+      const int total = lane_val(incl, wn - 1);
       AtomRegs<Real> R1{};
       wave_sync();
       if (lane < n1) {
@@ -1001,6 +1044,7 @@ __device__ void rot_inter_energy(const RotArgs<Real>& A, RotLDS2<Real>& L,
         *(V*)L.r1.prm[lane] = q;
         L.r1.flg[lane] = R1.flags;
       }
+      const uint64_t heavy1 = __ballot(lane < n1 && (R1.flags & F_HEAVY));
       L.sum[0][lane] = 0;
       L.sum[1][lane] = 0;
       L.sum[2][lane] = 0;
@@ -1029,14 +1073,14 @@ __device__ void rot_inter_energy(const RotArgs<Real>& A, RotLDS2<Real>& L,
           x = xyz[0];
           y = xyz[1];
           z = xyz[2];
-          const Real ex = x - cx, ey = y - cy, ez = z - cz;
+          const Real ex = x - sph.x, ey = y - sph.y, ez = z - sph.z;
           keep = ex * ex + ey * ey + ez * ez < reach2;
         }
         const uint64_t mk = __ballot(keep);
         const int nk = __popcll(mk);
         if (nk == 0) continue;
         if (nb + nk > WAVE) {
-          rot_chunk(L, gp, nb, n1, cp, min_sep, nc1, lig1, R1, lane);
+          rot_chunk(L, gp, nb, n1, cp, min_sep, nc1, lig1, R1, heavy1, lane);
           nb = 0;
         }
         if (keep) {
@@ -1061,7 +1105,7 @@ __device__ void rot_inter_energy(const RotArgs<Real>& A, RotLDS2<Real>& L,
         }
         nb += nk;
       }
-      if (nb > 0) rot_chunk(L, gp, nb, n1, cp, min_sep, nc1, lig1, R1, lane);
+      if (nb > 0) rot_chunk(L, gp, nb, n1, cp, min_sep, nc1, lig1, R1, heavy1, lane);
       wave_sync();
       if (lane < wn) {
         const int64_t e = entry + int64_t(i) * nr2 + w0 + lane;
