@@ -1,7 +1,7 @@
 // Rotamer-pair LJ+LK scoring for packing (reference: LJLKRotamerScoreDispatch,
 // ljlk_pose_score.impl.hh:1479-2126; sphere_overlap.impl.hh:23-107, 455-610).
 //
-//   spheres   one bounding sphere per rotamer (spheres_kernel run over
+//   spheres   one bounding sphere per rotamer (setup_kernel run over
 //             rotamers), then one per block enclosing all of its rotamers
 //   rows      one wave per block b1 of a pose: the neighbor test against
 //             every b2 >= b1 (bit-identical to the reference), and the row's
