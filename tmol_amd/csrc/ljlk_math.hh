@@ -215,9 +215,10 @@ __device__ __forceinline__ void lk_sides(Real dist, Real d_min, Real cdmin, Real
     Real f0, df0;
     fdesolv<Real, SIDES>(d_min, side, f0, df0);
     const Real w = cdmax - cdmin;
-    const Real inv_w = fast_rcp(w);
-    Real tc = (dist - cdmin) * inv_w;
-    tc = tc > Real(0) ? tc : Real(0);
+    // below cdmin tc and the slope are 0 whatever w is: the knots' cap is on
+    // cdmax alone, so from a sigma of 5.234 on cdmin is not below it
+    const Real inv_w = dist < cdmin ? Real(0) : fast_rcp(w);
+    const Real tc = (dist - cdmin) * inv_w;
     const Real dp1 = df * w;
     const Real c2 = Real(3) * (f - f0) - dp1;
     const Real c3 = dp1 - Real(2) * (f - f0);
