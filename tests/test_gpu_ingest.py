@@ -248,3 +248,24 @@ def test_table_check_equals_the_tensor_checks(co, key, value, at):
     with pytest.raises(ingest.ops.LJLKLibraryError) as got:
         ingest.gen_pose_leaf_atoms(*[k[n].cuda() for n in keys])
     assert str(got.value) == str(want.value)
+
+
+@pytest.mark.parametrize("mask_dtype", [torch.bool, torch.uint8])
+def test_masks_cleared_between_forward_and_backward(co, mask_dtype):
+    """A program that marks the built atoms as present before it calls
+    backward gets the gradient of the atoms that the forward built."""
+    _, args = _random_missing(co, torch.float64)
+    grads = []
+    for clear in (False, True):
+        da = _dev(args)
+        da[1], da[2] = da[1].to(mask_dtype), da[2].to(mask_dtype)
+        X = da[0] = da[0].clone().requires_grad_(True)
+        out = ingest.gen_pose_leaf_atoms(*da)
+        if clear:
+            da[1].zero_()
+            da[2].zero_()
+        w = torch.randn(out.shape, dtype=out.dtype, generator=torch.Generator().manual_seed(4))
+        (out.nan_to_num(0) * w.cuda()).sum().backward()
+        grads.append(X.grad)
+    # the same kernels on the same inputs; atomic sums in another order
+    assert torch.allclose(grads[0], grads[1], rtol=1e-12, atol=1e-12)

@@ -299,10 +299,9 @@ class _LeafCall:
         P2, B, Amax = (int(x) for x in bmiss.shape)
         if P2 != P or tuple(pmiss.shape) != (P, NA) or tuple(btype.shape) != (P, B):
             raise ops.LJLKLibraryError("leaf-atom op: inconsistent pose shapes")
-        def u8(t):  # a bool is a byte of 0 or 1 already
-            t = t.to(device=dev).contiguous()
-            return t.view(torch.uint8) if t.dtype == torch.bool else t.to(torch.uint8)
-
+        # own copies: the backward reads the masks again, and a program that
+        # has its atoms built may mark them as present before it
+        u8 = lambda t: t.to(device=dev, dtype=torch.uint8, copy=True).contiguous()  # noqa: E731
         i32 = lambda t: ops._i32(torch.as_tensor(t), dev)  # noqa: E731
         f = lambda t: torch.as_tensor(t).to(device=dev, dtype=orig.dtype).contiguous()  # noqa
         self.keep = dict(bmiss=u8(bmiss), pmiss=u8(pmiss), boff=i32(boff), btype=i32(btype),
