@@ -269,3 +269,33 @@ def test_masks_cleared_between_forward_and_backward(co, mask_dtype):
         grads.append(X.grad)
     # the same kernels on the same inputs; atomic sums in another order
     assert torch.allclose(grads[0], grads[1], rtol=1e-12, atol=1e-12)
+
+
+def _reshaped(args, name):
+    a = list(args)
+    if name == "bt_n":  # [T, 2]
+        a[6] = torch.cat([a[6], a[6]]).view(-1, 2)
+    elif name == "boff":  # [B, P]
+        a[3] = a[3].t().contiguous()
+    else:  # irc [P, B * C, 1, 2]
+        a[5] = a[5].flatten(1, 2).unsqueeze(2)
+    return a
+
+
+@pytest.mark.parametrize("name", ["bt_n", "boff", "irc"])
+def test_table_shapes_refused(co, name):
+    """Tables of the right size in another shape are refused, not read in
+    the order of their words."""
+    _, args = _random_missing(co, torch.float32)
+    assert args[3].shape[0] != args[3].shape[1]
+    with pytest.raises((RuntimeError, IndexError)):
+        ingest.gen_pose_leaf_atoms(*_dev(_reshaped(args, name)))
+
+
+def test_block_offsets_with_a_leading_one(co):
+    """[1, P, B] block offsets are the [P, B] table."""
+    _, args = _random_missing(co, torch.float32)
+    want = ingest.gen_pose_leaf_atoms(*_dev(args))
+    args[3] = args[3].unsqueeze(0)
+    got = ingest.gen_pose_leaf_atoms(*_dev(args))
+    assert torch.equal(got.nan_to_num(0), want.nan_to_num(0))

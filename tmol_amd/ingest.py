@@ -260,7 +260,13 @@ def _validate_leaf_tables(k, P, NA, B, Amax, C):
             or tuple(k["anc_b"].shape) != (T, Amax, 3, 3) \
             or tuple(k["geom"].shape) != (T, Amax, 3) or tuple(k["geom_b"].shape) != (T, Amax, 3):
         raise ops.LJLKLibraryError("leaf-atom op: block-type table shapes")
-    if int(k["boff"].numel()) != P * B or (C > 0 and tuple(k["irc"].shape) != (P, B, C, 2)):
+    if int(k["bt_n"].numel()) != T:
+        raise ops.LJLKLibraryError("leaf-atom op: block-type table shapes")
+    # block offsets line up with the block types as tensors do: [P, B], or
+    # with ones in front of it (left out, for a single pose)
+    off = tuple(k["boff"].shape)
+    if (1,) * (2 - len(off)) + off != (1,) * (len(off) - 2) + (P, B) \
+            or (C > 0 and tuple(k["irc"].shape) != (P, B, C, 2)):
         raise ops.LJLKLibraryError("leaf-atom op: inconsistent pose shapes")
     if bt.is_cuda:
         return
