@@ -113,3 +113,30 @@ def test_eager_call_equals_the_registered_op(block_pair, dt):
         x = a[0].clone().requires_grad_(True)
         (g,) = torch.autograd.grad(ljlk_pose_scores(x, *a[1:])[0].sum(), x, create_graph=True)
         g.sum().backward()
+
+
+@pytest.mark.parametrize("call", ["total_lj", "total_lj_el", "op", "op_block_pair"])
+def test_second_order_raises(call):
+    """The gradient under create_graph is not a constant of the coordinates:
+    a penalty on it, or a Hessian-vector product, raises."""
+    from tmol_amd.ops import ljlk_pose_scores
+
+    ps = PoseStack(generate_poses(2, (9, 20), seed=5), device=DEV)
+    if call.startswith("total"):
+        types = LJ if call == "total_lj" else LJ + (S.fa_elec,)
+        x0, fn = ps.coords, _module(ps, types, (1.0, 0.55, 1.0, 1.0))
+        assert fn._total(x0) is not None
+    else:
+        a = pose_op_args(ps, LJLKEnergyTerm(device=DEV), block_pair=call == "op_block_pair")
+        x0, fn = a[0], lambda x: ljlk_pose_scores(x, *a[1:])[0]
+    x = x0.clone().requires_grad_(True)
+    total = fn(x).sum()
+    (g,) = torch.autograd.grad(total, x, create_graph=True)
+    (g0,) = torch.autograd.grad(fn(x).sum(), x)
+    assert not g0.requires_grad
+    # two passes over the same pairs: the order of the float sums
+    assert (g - g0).abs().max() <= 1e-5 * g0.abs().max()
+    with pytest.raises(RuntimeError):
+        (total + g.pow(2).sum()).backward()
+    with pytest.raises(RuntimeError):
+        torch.autograd.functional.hvp(lambda y: fn(y).sum(), x0, torch.ones_like(x0))

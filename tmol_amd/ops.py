@@ -25,7 +25,6 @@ import threading
 from typing import List, Optional
 
 import torch
-from torch.autograd.function import once_differentiable
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libtmol_ljlk_hip.so")
@@ -608,7 +607,7 @@ def ljlk_pose_scores(*args):
         raise TypeError("ljlk_pose_scores takes 27 arguments (%d given)" % len(args))
     if _plain_call(args) and args[0].is_cuda:
         require = args[0].requires_grad and torch.is_grad_enabled() and not args[-1]
-        return list(LJLKPoseScoreFunction.apply(require, *args))
+        return list(LJLKPoseScoreFunction.apply(require, *args)[:2])
     return torch.ops.tmol_ljlk.ljlk_pose_scores(*args)
 
 
@@ -633,10 +632,31 @@ def _plain_call(args) -> bool:
     return type(args[12]) is int and type(args[-2]) is not bool and type(args[-1]) is bool
 
 
+class _FirstOrder(torch.autograd.Function):
+    """A gradient computed from ``source``, whose derivative the kernels do
+    not give."""
+
+    @staticmethod
+    def forward(ctx, grad, source):
+        return grad.view_as(grad)
+
+    @staticmethod
+    def backward(ctx, grad_grad):
+        raise RuntimeError("the pose scores' gradient has no derivative (second order)")
+
+
+def _first_order(grad, source):
+    """``grad`` as a backward returns it.  Under ``create_graph`` it stays tied
+    to the coordinates through ``source`` (the coordinates, or an output saved
+    for the backward), so that a second differentiation raises instead of
+    taking it for a constant."""
+    return _FirstOrder.apply(grad, source) if torch.is_grad_enabled() else grad
+
+
 class LJLKPoseScoreFunction(torch.autograd.Function):
     """The eager form of the op and its registered autograd: whole-pose mode
-    saves dV/dx and pose_ind_for_atom, block-pair mode re-walks the neighbor
-    list (compiled.ops.cpp:29-279)."""
+    saves dV/dx (an output of its own) and pose_ind_for_atom, block-pair mode
+    re-walks the neighbor list (compiled.ops.cpp:29-279)."""
 
     @staticmethod
     def forward(ctx, require, *args):
@@ -650,22 +670,21 @@ class LJLKPoseScoreFunction(torch.autograd.Function):
             ctx.save_for_backward(args[0])
         else:
             ctx.save_for_backward(dvdx, args[2])
-        return score, nbr
+        return score, nbr, dvdx
 
     @staticmethod
-    @once_differentiable
-    def backward(ctx, grad_score, grad_nbr):
+    def backward(ctx, grad_score, grad_nbr, grad_dvdx):
         none = (None,) * ctx.n_args
         if grad_score is None:
             return none
         if ctx.block_pair:
             (coords,) = ctx.saved_tensors
-            grad = _block_pair_backward(grad_score, (coords,) + ctx.args)
+            grad = _first_order(_block_pair_backward(grad_score, (coords,) + ctx.args), coords)
         else:
             dvdx, atom_pose = ctx.saved_tensors
             if dvdx is None:
                 return none
-            grad = _backward_combine(dvdx, grad_score, atom_pose)
+            grad = _first_order(_backward_combine(dvdx, grad_score, atom_pose), dvdx)
         return (None, grad) + none[2:]
 
 
@@ -675,7 +694,7 @@ class WholePoseTotalFunction(torch.autograd.Function):
     takes the weighted gradient, which the backward scales by each pose's
     incoming gradient.  The weights are known at the forward pass, so per-term
     derivatives need not be kept.  elec_first: the weights' first row is
-    elec's."""
+    elec's.  Returns the totals and that gradient."""
 
     @staticmethod
     def forward(ctx, coords, weights, tail, elec_tail, elec_first, require):
@@ -709,11 +728,10 @@ class WholePoseTotalFunction(torch.autograd.Function):
             call.score(flags, weights=w, energies=energies, grad=grad)
         ctx.save_for_backward(grad, scale, call.keep["atom_pose"])
         order = weights.roll(-1, 0) if elec_first else weights
-        return (order * energies).sum(dim=0)
+        return (order * energies).sum(dim=0), grad
 
     @staticmethod
-    @once_differentiable
-    def backward(ctx, grad_total):
+    def backward(ctx, grad_total, grad_grad):
         grad, scale, atom_pose = ctx.saved_tensors
         if grad_total is None or grad is None:
             return (None,) * 6
@@ -723,7 +741,7 @@ class WholePoseTotalFunction(torch.autograd.Function):
                                          _p(atom_pose.contiguous()), grad.shape[0],
                                          _dtype_code(grad.dtype), _p(out), _stream(grad.device)),
                "total backward")
-        return (out,) + (None,) * 5
+        return (_first_order(out, grad),) + (None,) * 5
 
 
 def whole_pose_total(coords, weights, tail, elec_tail=None, elec_first=False):
@@ -752,7 +770,7 @@ def whole_pose_total(coords, weights, tail, elec_tail=None, elec_first=False):
     else:
         terms = None
     require = coords.requires_grad and torch.is_grad_enabled()
-    return WholePoseTotalFunction.apply(coords, weights, tail, terms, elec_first, require)
+    return WholePoseTotalFunction.apply(coords, weights, tail, terms, elec_first, require)[0]
 
 
 def debug_pair_separations(args, items: torch.Tensor) -> torch.Tensor:
