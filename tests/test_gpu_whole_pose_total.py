@@ -140,3 +140,14 @@ def test_second_order_raises(call):
         (total + g.pow(2).sum()).backward()
     with pytest.raises(RuntimeError):
         torch.autograd.functional.hvp(lambda y: fn(y).sum(), x0, torch.ones_like(x0))
+
+
+@pytest.mark.parametrize("types", [LJ, LJ + (S.fa_elec,)], ids=["lj", "lj_el"])
+def test_weights_changed_between_forward_and_backward_raise(types):
+    ps = PoseStack(generate_poses(2, (9, 20), seed=5), device=DEV)
+    m = _module(ps, types, (1.0, 0.55, 1.0, 1.0))
+    for sum_terms in (True, False):
+        total = m(ps.coords.clone().requires_grad_(True), sum_terms=sum_terms).sum()
+        m.weights.mul_(2)
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            total.backward()

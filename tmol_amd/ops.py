@@ -726,13 +726,15 @@ class WholePoseTotalFunction(torch.autograd.Function):
                                           _p(energies), _p(grad), 0, stream), "ljlk+elec score")
         else:
             call.score(flags, weights=w, energies=energies, grad=grad)
-        ctx.save_for_backward(grad, scale, call.keep["atom_pose"])
+        # the weights too: autograd refuses the backward once they changed, as
+        # where they multiply each term's scores
+        ctx.save_for_backward(grad, scale, call.keep["atom_pose"], weights)
         order = weights.roll(-1, 0) if elec_first else weights
         return (order * energies).sum(dim=0), grad
 
     @staticmethod
     def backward(ctx, grad_total, grad_grad):
-        grad, scale, atom_pose = ctx.saved_tensors
+        grad, scale, atom_pose, _ = ctx.saved_tensors
         if grad_total is None or grad is None:
             return (None,) * 6
         up = grad_total.to(grad.dtype).contiguous()
