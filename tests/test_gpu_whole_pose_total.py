@@ -151,3 +151,19 @@ def test_weights_changed_between_forward_and_backward_raise(types):
         m.weights.mul_(2)
         with pytest.raises(RuntimeError, match="modified by an inplace operation"):
             total.backward()
+
+
+@pytest.mark.parametrize("types", [LJ, LJ + (S.fa_elec,)], ids=["lj", "lj_el"])
+def test_saved_tensors_kept_on_the_host(types):
+    """Hooks that move saved tensors to the host and back give the same
+    gradient; left there, the backward raises before a kernel reads them."""
+    ps = PoseStack(generate_poses(2, (9, 20), seed=5), device=DEV)
+    m = _module(ps, types, (1.0, 0.55, 1.0, 1.0))
+    up = torch.tensor([0.5, 2.0], device=DEV)
+    _, want = _run(m, ps.coords, up)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.to(DEV)):
+        _, got = _run(m, ps.coords, up)
+    assert (got - want).abs().max() <= 1e-5 * want.abs().max()  # order of the float sums
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t):
+        with pytest.raises(RuntimeError):
+            _run(m, ps.coords, up)

@@ -737,11 +737,14 @@ class WholePoseTotalFunction(torch.autograd.Function):
         grad, scale, atom_pose, _ = ctx.saved_tensors
         if grad_total is None or grad is None:
             return (None,) * 6
-        up = grad_total.to(grad.dtype).contiguous()
-        out = torch.empty_like(grad)
-        _check(lib().tmol_total_backward(_p(grad.contiguous()), _p(up), _p(scale.contiguous()),
-                                         _p(atom_pose.contiguous()), grad.shape[0],
-                                         _dtype_code(grad.dtype), _p(out), _stream(grad.device)),
+        # saved tensors come back from a caller's hooks: on the device, or not
+        _require_device(grad)
+        dev = grad.device
+        up = grad_total.to(dev, grad.dtype).contiguous()
+        kept, scale, pose = grad.contiguous(), scale.to(dev).contiguous(), _i32(atom_pose, dev)
+        out = torch.empty_like(kept)
+        _check(lib().tmol_total_backward(_p(kept), _p(up), _p(scale), _p(pose), kept.shape[0],
+                                         _dtype_code(kept.dtype), _p(out), _stream(dev)),
                "total backward")
         return (_first_order(out, grad),) + (None,) * 5
 
