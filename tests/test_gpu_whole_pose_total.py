@@ -167,3 +167,36 @@ def test_saved_tensors_kept_on_the_host(types):
     with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t):
         with pytest.raises(RuntimeError):
             _run(m, ps.coords, up)
+
+
+@pytest.mark.parametrize("what", ["callable", "rendered_op", "class_forward", "class_call",
+                                  "class_unweighted"])
+def test_replaced_scoring_is_called(what, monkeypatch):
+    """A caller's own scoring callable, put in before or after the module is
+    rendered, on the module or its class, is what a weighted sum calls too."""
+    import tmol_amd.ops as ops
+    from tmol_amd.score.score_function import WholePoseScoringModule
+    from tmol_amd.score.scoring_module import TermPoseScoringModule as Term
+
+    ps = PoseStack(generate_poses(2, (9, 20), seed=5), device=DEV)
+    weights = (1.0, 0.55, 1.0, 1.0)
+    want = _module(ps, LJ + (S.fa_elec,), weights)(ps.coords)
+    seen = []
+
+    def seeing(fn):
+        return lambda *a, **k: (seen.append(1), fn(*a, **k))[1]
+
+    if what == "rendered_op":
+        monkeypatch.setattr(ops, "elec_pose_scores", seeing(ops.elec_pose_scores))
+    m = _module(ps, LJ + (S.fa_elec,), weights)
+    if what == "callable":
+        m.term_modules[0].term_score_poses = seeing(m.term_modules[0].term_score_poses)
+    elif what == "class_forward":
+        monkeypatch.setattr(Term, "forward", seeing(Term.forward))
+    elif what == "class_call":
+        monkeypatch.setattr(Term, "__call__", seeing(Term.__call__))
+    elif what == "class_unweighted":
+        monkeypatch.setattr(WholePoseScoringModule, "unweighted_scores",
+                            seeing(WholePoseScoringModule.unweighted_scores))
+    total = m(ps.coords)
+    assert seen and torch.allclose(total, want, rtol=1e-5)

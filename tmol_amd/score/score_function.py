@@ -7,7 +7,7 @@ their creation order, and each contributes its score types in its own order.
 import torch
 from torch.nn.modules.module import _has_any_global_hook as _any_global_hook
 
-from ..ops import whole_pose_total
+from ..ops import elec_pose_scores, ljlk_pose_scores, whole_pose_total
 from .elec_energy_term import ElecEnergyTerm
 from .ljlk_energy_term import LJLKEnergyTerm
 from .score_types import ScoreType
@@ -18,6 +18,9 @@ _TERM_FOR_SCORE_TYPE = {
     ScoreType.fa_lk: LJLKEnergyTerm,
     ScoreType.fa_elec: ElecEnergyTerm,
 }
+
+# the ops that one pass can take the place of
+_ONE_PASS_OPS = {LJLKEnergyTerm: ljlk_pose_scores, ElecEnergyTerm: elec_pose_scores}
 
 
 class ScoreFunction:
@@ -107,14 +110,18 @@ class WholePoseScoringModule:
         are known here."""
         mods = list(self.term_modules)
         if (type(self) is not WholePoseScoringModule or "unweighted_scores" in self.__dict__
+                or type(self).unweighted_scores is not _unweighted_scores
                 or len(mods) != len(self._one_pass) or _any_global_hook()
-                or any(m is not q or not m.is_plain()
-                       for m, q in zip(mods, self._one_pass.values()))):
+                or any(m is not q or not m.is_plain(_ONE_PASS_OPS[kind])
+                       for m, (kind, q) in zip(mods, self._one_pass.items()))):
             return None
         f64 = coords.dtype == torch.float64
         lj, elec = self._one_pass[LJLKEnergyTerm], self._one_pass.get(ElecEnergyTerm)
         return whole_pose_total(coords.flatten(start_dim=0, end_dim=-2), self.weights,
                                 lj.tail(f64), elec.tail(f64) if elec else None, mods[0] is elec)
+
+
+_unweighted_scores = WholePoseScoringModule.unweighted_scores
 
 
 class BlockPairScoringModule:

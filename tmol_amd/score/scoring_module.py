@@ -39,10 +39,14 @@ class TermPoseScoringModule(torch.nn.Module):
     def tail(self, f64):
         return self._tail_f64 if f64 else self._tail_f32
 
-    def is_plain(self):
-        """Called as it was rendered: no hook or replaced forward that a
+    def is_plain(self, score_poses):
+        """Called as it was rendered, on the op ``score_poses``: no hook, no
+        replaced callable or forward, of the module or its class, that a
         caller scoring the term by other means would pass by."""
-        return (type(self) is TermWholePoseScoringModule and "forward" not in self.__dict__
+        return (type(self) is TermWholePoseScoringModule
+                and self.term_score_poses is score_poses
+                and "forward" not in self.__dict__ and type(self).forward is _term_forward
+                and type(self).__call__ is torch.nn.Module.__call__
                 and not (self._forward_hooks or self._forward_pre_hooks or self._backward_hooks
                          or self._backward_pre_hooks))
 
@@ -50,6 +54,9 @@ class TermPoseScoringModule(torch.nn.Module):
         flat = coords.flatten(start_dim=0, end_dim=-2)
         scores, _ = self.term_score_poses(flat, *self.tail(coords.dtype == torch.float64))
         return scores
+
+
+_term_forward = TermPoseScoringModule.forward
 
 
 class TermWholePoseScoringModule(TermPoseScoringModule):
