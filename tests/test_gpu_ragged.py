@@ -195,3 +195,23 @@ def test_item_energies_sum_to_pose_energies(ubq_pdb, general):
         1, stack.block_pose.long(), per_block)
     e = sc.energies_only(x).cpu()
     torch.testing.assert_close(per_pose, e, rtol=1e-10, atol=1e-8)
+
+
+def test_f32_rounding_against_f64():
+    """Float32 energies and gradients against the same kernels in float64 on
+    the same inputs, as norms over 40 poses.  The gradients' 2.4e-7 is the
+    rounding of the distance and of a pair's few products; 4e-7 lies below
+    what sigma * rcp(x), off by 2-3 ulp, gives in the sixth power on the
+    linear piece (5.1e-7).  Energies: 4e-8, and 9e-8 with it."""
+    from tmol_amd.scorer import LJLKRaggedScorer
+
+    _say("f32 rounding")
+    poses = generate_poses(40, (50, 300), seed=19)
+    x = RaggedPoseStack(poses, dtype=torch.float32).coords.to(DEV)
+    out = {}
+    for dt in (torch.float32, torch.float64):
+        st = RaggedPoseStack(poses, dtype=dt)
+        sc = LJLKRaggedScorer(st, LJLKEnergyTerm(device=DEV), device=DEV, dtype=dt)
+        out[dt] = [t.double().clone() for t in sc.energy_and_grad(x.to(dt), torch.tensor(W))]
+    for got, want, bound in zip(out[torch.float32], out[torch.float64], (7e-8, 4e-7)):
+        assert (got - want).norm() <= bound * want.norm()

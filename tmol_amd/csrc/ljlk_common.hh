@@ -428,6 +428,8 @@ __device__ __forceinline__ GlobalParams<Real> load_global_params(const Real* g) 
   GlobalParams<Real> gp;
   gp.max_dis = g[0];
   gp.dlin_factor = g[1];
+  const double f2 = 1.0 / (double(g[1]) * double(g[1]));
+  gp.lin6 = Real(f2 * f2 * f2);
   gp.hbond_dis = g[2];
   gp.hbond_oh_dis = g[3];
   gp.hbond_hdis = g[4];

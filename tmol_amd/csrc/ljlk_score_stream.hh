@@ -303,7 +303,8 @@ __global__ __launch_bounds__(256, (stream_waves_per_simd<MODE, OCC>())) void sco
   const int shift = A.part_shift;
   RowQueue queue(A.row_cursor, int64_t(s.G) << shift, A.row_grab);
   const Real cull_pad = gp.max_dis + Real(1e-3);
-  const Real cut2 = C::ELEC && ek.cull2 > gp.max_dis2 ? ek.cull2 : gp.max_dis2;
+  // in a scalar register: the fused gradient mode is at its 128 VGPRs
+  const Real cut2 = wave_lane(C::ELEC && ek.cull2 > gp.max_dis2 ? ek.cull2 : gp.max_dis2, 0);
   const int u = lane & (SCH - 1), half = lane >> 5;
   const int odd = (lane & 1) ? SSLOTS : 0;
 
