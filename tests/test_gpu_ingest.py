@@ -221,6 +221,21 @@ def test_pose_stack_from_pdb(co):
 def test_table_check_equals_the_tensor_checks(co, key, value, at):
     """One table entry out of range, first or last of its table: the kernel's
     check raises what the tensor form of the checks raises on the host."""
+    _same_refusal(co, [(key, value)], at)
+
+
+@pytest.mark.parametrize("faults", [
+    [("boff", -1), ("anc0", -2)], [("pad", 0), ("bt_n", "A1")], [("boff", "NA"), ("pad", 0)],
+    [("btype", "T"), ("boff", -1)], [("down", "n"), ("irc0", "B")], [("anc2", "A"), ("anc_b0", -2)]],
+    ids=lambda f: "+".join(k for k, _ in f))
+@pytest.mark.parametrize("at", [0, -1])
+def test_several_tables_out_of_range(co, faults, at):
+    """Two tables at once: every range check that fails is named, in order,
+    and the checks that index with checked values only where none failed."""
+    _same_refusal(co, faults, at)
+
+
+def _same_refusal(co, faults, at):
     _, args = _random_missing(co, torch.float64)
     keys = ("orig", "bmiss", "pmiss", "boff", "btype", "irc", "bt_n", "down", "anc",
             "geom", "anc_b", "geom_b")
@@ -228,21 +243,22 @@ def test_table_check_equals_the_tensor_checks(co, key, value, at):
     P, NA = k["orig"].shape[:2]
     B, A = k["bmiss"].shape[1:]
     C, T = k["irc"].shape[2], k["bt_n"].shape[0]
-    name = key.rstrip("012")
-    v = {"T": T, "A1": A + 1, "n": A, "A": A, "C": C, "B": B, "NA": NA}.get(value, value)
-    if key == "pad":  # a connection to a block that does not exist
-        pose = int((k["btype"] < 0).any(dim=1).nonzero()[0, 0])
-        k["irc"][pose, 0, 0, 0] = int((k["btype"][pose] < 0).nonzero()[at, 0])
-        k["irc"][pose, 0, 0, 1] = 0
-    elif key == "boff":
-        b = (k["btype"].view(-1) >= 0).nonzero()[at, 0]
-        k["boff"].view(-1)[b] = v
-    elif key[-1] in "012":
-        row = k[name].view(-1, k[name].shape[-1])[at]
-        row[1 if key.startswith("anc") and key[-1] == "2" else 0] = 0
-        row[int(key[-1])] = v
-    else:
-        k[name].view(-1)[at] = v
+    for key, value in faults:
+        name = key.rstrip("012")
+        v = {"T": T, "A1": A + 1, "n": A, "A": A, "C": C, "B": B, "NA": NA}.get(value, value)
+        if key == "pad":  # a connection to a block that does not exist
+            pose = int((k["btype"] < 0).any(dim=1).nonzero()[0, 0])
+            k["irc"][pose, 0, 0, 0] = int((k["btype"][pose] < 0).nonzero()[at, 0])
+            k["irc"][pose, 0, 0, 1] = 0
+        elif key == "boff":
+            b = (k["btype"].view(-1) >= 0).nonzero()[at, 0]
+            k["boff"].view(-1)[b] = v
+        elif key[-1] in "012":
+            row = k[name].view(-1, k[name].shape[-1])[at]
+            row[1 if key.startswith("anc") and key[-1] == "2" else 0] = 0
+            row[int(key[-1])] = v
+        else:
+            k[name].view(-1)[at] = v
     with pytest.raises(ingest.ops.LJLKLibraryError) as want:
         ingest._validate_leaf_tables(k, P, NA, B, A, C)
     with pytest.raises(ingest.ops.LJLKLibraryError) as got:
