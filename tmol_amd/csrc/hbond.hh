@@ -446,10 +446,10 @@ __device__ __forceinline__ void hb_phase_b(HbLDS& L, const HbArgs<Real>& a, int 
 // cells; gradients through the derived atoms' indices with global atomics
 // (few pairs pass).
 // The kernel is bound by the latency of its dependent loads (row, item, type,
-// list entry, coordinates: 80% of the wave cycles waited), not by arithmetic
-// (VALU 25-28% busy), so a wave walks HB_ROWS rows at once, 16 lanes each: a
-// protein row has 10-20 items, which filled a quarter of the lanes of a wave
-// of its own.  The FIFO is carried from row to row: a row has about 2.5
+// list entry, coordinates: 70% of the wave cycles wait, 512 poses), not by
+// arithmetic (VALU issue 37%), so a wave walks HB_ROWS rows at once, 16 lanes
+// each: a protein row has 10-20 items, which filled a quarter of the lanes of
+// a wave of its own.  The FIFO is carried from row to row: a row has about 2.5
 // passing pairs, and draining them at its end ran the evaluation with 4% of
 // its lanes.  256 poses of 50-600 residues with gradients: one row per wave
 // 312 us, the carried FIFO alone 320 us, four rows 234 us, and 203 us with

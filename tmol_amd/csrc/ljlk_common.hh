@@ -447,8 +447,9 @@ __device__ __forceinline__ GlobalParams<Real> load_global_params(const Real* g) 
 // exhausted, rows of the other ranges: no wave idles while rows remain.  Rows
 // are handed out one at a time (a row is tens of microseconds of one wave's
 // work, so larger grabs lengthen the tail) and each cursor sits on its own
-// 256-byte line (same-line L2 atomics serialize).  The cursors are zeroed by
-// a fill kernel before every scoring launch.
+// 256-byte line (same-line L2 atomics serialize).  A launch neither clears
+// its cursors nor leaves them clear: whoever launches puts them in the
+// ClearList that runs before (the rotamer kernels: a fill).
 // The rows taken per cursor grab (`grab`, default 1) is a launch parameter the
 // autotuner may raise.
 constexpr int QROWS = 1;

@@ -41,7 +41,7 @@ constexpr int UNIT_R1 = 4;      // most b1 rotamers of a unit
 constexpr int UNIT_PAIRS = 32;  // rotamer pairs of a unit, where that is at least one b1 rotamer
 __device__ __forceinline__ int unit_r1(int nr2, bool diag) {
   return diag ? UNIT_R1 : max(1, min(UNIT_R1, UNIT_PAIRS / max(nr2, 1)));
-}  // b1 rotamers per work unit
+}
 
 struct RotView {
   int P, B, R, C;
@@ -806,7 +806,8 @@ rotamer_score_kernel(RotArgs<Real> A) {
 //   write     after the window, one store per rotamer pair and term (zero
 //             for pairs with no surviving atoms).
 //
-// Bound by VALU issue (75% busy): 8 x 200 residues take 2.3 M candidate
+// Bound by VALU issue (97% of the issue slots at four cycles an instruction,
+// 16 x 300 residues): 8 x 200 residues take 2.3 M candidate
 // chunks, 18 M phase A steps, 4.1 M LJ and 1.5 M LK batches, about 1.3 G
 // wave instructions.  Dropping rotamers by sphere before their atoms, FIFO
 // rings in place of moving the rest to the front, scans by DPP and the heavy

@@ -122,7 +122,7 @@ def run(device, poses=None, steps=20, warmup=3, kernel_reps=10, cpu=None, log=pr
             "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS,
             "traffic": fwd_prof.get("hbm_bytes_per_launch"),
-            "kernel": "leaf_atoms_kernel<float> (one-wave workgroups, 16 blocks each)",
+            "kernel": "leaf_atoms_kernel<float> (one-wave workgroups, 4 blocks each)",
             "algorithmic_bytes_per_launch": alg_bytes,
             "backward_traffic": {k: v.get("hbm_bytes_per_launch") for k, v in kern.items()
                                  if "backward" in k} or None,
