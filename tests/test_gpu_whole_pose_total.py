@@ -115,20 +115,50 @@ def test_eager_call_equals_the_registered_op(block_pair, dt):
         g.sum().backward()
 
 
-@pytest.mark.parametrize("call", ["total_lj", "total_lj_el", "op", "op_block_pair"])
-def test_second_order_raises(call):
-    """The gradient under create_graph is not a constant of the coordinates:
-    a penalty on it, or a Hessian-vector product, raises."""
+def _call(call):
+    """(coordinates, function of them): a total, or the eager op's scores."""
     from tmol_amd.ops import ljlk_pose_scores
 
     ps = PoseStack(generate_poses(2, (9, 20), seed=5), device=DEV)
     if call.startswith("total"):
-        types = LJ if call == "total_lj" else LJ + (S.fa_elec,)
-        x0, fn = ps.coords, _module(ps, types, (1.0, 0.55, 1.0, 1.0))
-        assert fn._total(x0) is not None
-    else:
-        a = pose_op_args(ps, LJLKEnergyTerm(device=DEV), block_pair=call == "op_block_pair")
-        x0, fn = a[0], lambda x: ljlk_pose_scores(x, *a[1:])[0]
+        fn = _module(ps, LJ if call == "total_lj" else LJ + (S.fa_elec,), (1.0, 0.55, 1.0, 1.0))
+        assert fn._total(ps.coords) is not None
+        return ps.coords, fn
+    a = pose_op_args(ps, LJLKEnergyTerm(device=DEV), block_pair=call == "op_block_pair")
+    return a[0], lambda x: ljlk_pose_scores(x, *a[1:])[0]
+
+
+CALLS = ["total_lj", "total_lj_el", "op", "op_block_pair"]
+
+
+@pytest.mark.parametrize("call", CALLS)
+def test_batched_gradients(call):
+    """Several incoming gradients at once (is_grads_batched, a vectorized
+    Jacobian) give what they give one by one; under create_graph a second
+    differentiation raises."""
+    x0, fn = _call(call)
+    x = x0.clone().requires_grad_(True)
+    y = fn(x).flatten()
+    pick = y.detach().abs().topk(min(4, y.numel())).indices
+    up = torch.zeros((len(pick), y.numel()), device=DEV)
+    up[torch.arange(len(pick)), pick] = torch.linspace(0.5, 2.0, len(pick), device=DEV)
+    (got,) = torch.autograd.grad(y, x, up, is_grads_batched=True, retain_graph=True)
+    want = torch.stack([torch.autograd.grad(y, x, u, retain_graph=True)[0] for u in up])
+    assert got.shape == want.shape and want.abs().max() > 0
+    assert (got - want).abs().max() <= 1e-5 * want.abs().max()  # order of the float sums
+    jac = torch.autograd.functional.jacobian(lambda z: fn(z).flatten()[pick], x0, vectorize=True)
+    one = torch.autograd.functional.jacobian(lambda z: fn(z).flatten()[pick], x0)
+    assert (jac - one).abs().max() <= 1e-5 * one.abs().max()
+    with pytest.raises(RuntimeError):
+        (g,) = torch.autograd.grad(y, x, up, is_grads_batched=True, create_graph=True)
+        (g.pow(2).sum() + y.sum()).backward()
+
+
+@pytest.mark.parametrize("call", CALLS)
+def test_second_order_raises(call):
+    """The gradient under create_graph is not a constant of the coordinates:
+    a penalty on it, or a Hessian-vector product, raises."""
+    x0, fn = _call(call)
     x = x0.clone().requires_grad_(True)
     total = fn(x).sum()
     (g,) = torch.autograd.grad(total, x, create_graph=True)

@@ -611,15 +611,29 @@ def ljlk_pose_scores(*args):
     return torch.ops.tmol_ljlk.ljlk_pose_scores(*args)
 
 
+def _only_autograd() -> bool:
+    """Nothing but autograd sees what runs here: no compilation, tracing,
+    function transform, dispatch or function mode."""
+    return not (torch.compiler.is_compiling() or torch.jit.is_tracing()
+                or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+                or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch.autograd.forward_ad._current_level >= 0)
+
+
+def _plain_gradient(grad) -> bool:
+    """A gradient that a backward may hand to the kernels itself (batched
+    gradients and the like take the registered ops, or tensor operations)."""
+    return (type(grad) is torch.Tensor and _only_autograd()
+            and not torch._C._functorch.is_functorch_wrapped_tensor(grad)
+            and not torch._C._functorch.is_legacy_batchedtensor(grad))
+
+
 def _plain_call(args) -> bool:
     """An eager call of plain tensors that only autograd has to see: nothing
     compiles, traces, transforms or intercepts it, so the registered op's
     dispatch (0.4 ms of host time per forward of a 27-argument op, the
     larger part of a small pose's call) would reach the same kernels."""
-    if (torch.compiler.is_compiling() or torch.jit.is_tracing()
-            or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-            or torch._C._functorch.peek_interpreter_stack() is not None
-            or torch.autograd.forward_ad._current_level >= 0):
+    if not _only_autograd():
         return False
     for a in args:
         t = type(a)
@@ -632,6 +646,9 @@ def _plain_call(args) -> bool:
     return type(args[12]) is int and type(args[-2]) is not bool and type(args[-1]) is bool
 
 
+_SECOND_ORDER = "the pose scores' gradient has no derivative (second order)"
+
+
 class _FirstOrder(torch.autograd.Function):
     """A gradient computed from ``source``, whose derivative the kernels do
     not give."""
@@ -642,7 +659,7 @@ class _FirstOrder(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_grad):
-        raise RuntimeError("the pose scores' gradient has no derivative (second order)")
+        raise RuntimeError(_SECOND_ORDER)
 
 
 def _first_order(grad, source):
@@ -675,16 +692,27 @@ class LJLKPoseScoreFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_score, grad_nbr, grad_dvdx):
         none = (None,) * ctx.n_args
+        if grad_dvdx is not None:
+            raise RuntimeError(_SECOND_ORDER)
         if grad_score is None:
             return none
+        plain = _plain_gradient(grad_score)
         if ctx.block_pair:
             (coords,) = ctx.saved_tensors
-            grad = _first_order(_block_pair_backward(grad_score, (coords,) + ctx.args), coords)
+            if plain:
+                grad = _first_order(_block_pair_backward(grad_score, (coords,) + ctx.args), coords)
+            else:
+                grad = torch.ops.tmol_amd.ljlk_block_pair_backward(
+                    grad_score.contiguous(), coords, *ctx.args[:-1])
         else:
             dvdx, atom_pose = ctx.saved_tensors
             if dvdx is None:
                 return none
-            grad = _first_order(_backward_combine(dvdx, grad_score, atom_pose), dvdx)
+            if plain:
+                grad = _first_order(_backward_combine(dvdx, grad_score, atom_pose), dvdx)
+            else:
+                grad = torch.ops.tmol_amd.ljlk_backward_combine(
+                    dvdx, grad_score.contiguous(), atom_pose)
         return (None, grad) + none[2:]
 
 
@@ -735,11 +763,16 @@ class WholePoseTotalFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_total, grad_grad):
         grad, scale, atom_pose, _ = ctx.saved_tensors
+        if grad_grad is not None:
+            raise RuntimeError(_SECOND_ORDER)
         if grad_total is None or grad is None:
             return (None,) * 6
         # saved tensors come back from a caller's hooks: on the device, or not
         _require_device(grad)
         dev = grad.device
+        if not _plain_gradient(grad_total):
+            up = grad_total.to(grad.dtype).index_select(0, atom_pose.to(dev).long())
+            return ((up * scale.to(dev)).unsqueeze(-1) * grad,) + (None,) * 5
         up = grad_total.to(dev, grad.dtype).contiguous()
         kept, scale, pose = grad.contiguous(), scale.to(dev).contiguous(), _i32(atom_pose, dev)
         out = torch.empty_like(kept)
